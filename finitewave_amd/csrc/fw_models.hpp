@@ -59,6 +59,8 @@ __device__ __forceinline__ double ftanh(double x) { return tanh(x); }
 __device__ __forceinline__ float ftanh(float x) { return tanhf(x); }
 __device__ __forceinline__ double fpow(double x, double y) { return pow(x, y); }
 __device__ __forceinline__ float fpow(float x, float y) { return powf(x, y); }
+__device__ __forceinline__ double fpow15(double x) { return pow15(x); }
+__device__ __forceinline__ float fpow15(float x) { return fpow(x, 1.5f); }
 
 // (e^y - 1)/y, continuous at y = 0.  The FP32 path evaluates the rate
 // expressions of the form x / (e^(k x) - 1) through it: in float e^(k x)
@@ -76,7 +78,7 @@ __device__ __forceinline__ float exprel(float y) {
 // a/b; the remainder a - b q1 is exact).  Holds while a/b is a normal number
 // or zero (a zero quotient comes out +0).  FP32 path: the plain division.
 template <typename R>
-__device__ __forceinline__ R div_rn(R a, R b, R y) {  // y = 1/b correctly rounded
+__host__ __device__ __forceinline__ R div_rn(R a, R b, R y) {  // y = 1/b correctly rounded
   const R q0 = a * y;
   const R q1 = fma(fma(-b, q0, a), y, q0);
   return fma(fma(-b, q1, a), y, q1);
@@ -110,6 +112,33 @@ __device__ __forceinline__ R dv(R a, R b) {
     return a / b;
   }
 }
+
+// FP64 path: quantities of the parameters alone, appended after a model's
+// parameters by complete_params on the host in the operation order of the
+// expressions they replace, so the values are those a node would compute (the
+// float update keeps forming its own per node).  1 / tau values serve div_rn.
+constexpr int kFkInv = 11;  // Fenton-Karma: 1 / parameters 0..7, then 1 / (2 tau_si)
+enum Lr91Derived { kLrENa = 15, kLrEK, kLrGK, kLrEK1, kLrGK1 };
+enum CrnDerived {
+  kCrnRTF = 39,   // R * T / F
+  kCrnRT2F,       // R * T / (2 * F)
+  kCrnRT,         // R * T
+  kCrnInvRT,
+  kCrnSig,        // (exp(nao / 67.3) - 1) / 7
+  kCrnKo,         // ko / (ko + kmko)
+  kCrnNao3,       // nao * (nao * nao)
+  kCrnT12,        // (kmnancx^3 + nao^3) * (kmcancx + cao)
+  kCrnFnF,        // 5e-13 / F
+  kCrnInvCaup,    // 1 / caupmax
+  kCrnVrelVup,    // Vrel / Vup
+  kCrnFVj,        // F * Vj
+  kCrnInvFVj,
+  kCrn2FVj,       // 2 * F * Vj
+  kCrnInv2FVj,
+  kCrnInvVj,
+  kCrnNDerivedEnd
+};
+static_assert(kCrnNDerivedEnd <= 64, "parameter block size");
 
 // TP06 quantities that are the same for every node (functions of the
 // parameters only), appended after its 49 parameters by complete_params on the
@@ -234,7 +263,7 @@ __device__ __forceinline__ R ionic_ap(R u, R un, SP& S, int64_t c,
   auto&& vref = ref<R>(S, 0, c);
   R v = vref;
   // calc_v: v += (-dt*(eap + (mu_1*v)/(mu_2 + u)) * (v + k*u*(u - a - 1.)))
-  v += (-dt * (eap + (mu_1 * v) / (mu_2 + u)) * (v + k * u * (u - a - R(1))));
+  v += (-dt * (eap + dv(mu_1 * v, mu_2 + u)) * (v + k * u * (u - a - R(1))));
   vref = v;
   // u_new += dt*(-k*u*(u - a)*(u - 1.) - u*v)
   return un + dt * (-k * u * (u - a) * (u - R(1)) - u * v);
@@ -284,19 +313,24 @@ __device__ __forceinline__ R ionic_fk(R u, R un, SP& S, int64_t c,
           tau_si = par<R>(P, 3), tau_v_m = par<R>(P, 4), tau_v_p = par<R>(P, 5),
           tau_w_m = par<R>(P, 6), tau_w_p = par<R>(P, 7), k = par<R>(P, 8),
           u_c = par<R>(P, 9), uc_si = par<R>(P, 10);
+  // x / tau, parameter q
+  auto over = [&](R x, R tau, int q) -> R {
+    if constexpr (sizeof(R) == 8) return div_rn(x, tau, P.v[kFkInv + q]);
+    else return x / tau;
+  };
   auto&& vref = ref<R>(S, 0, c);
   auto&& wref = ref<R>(S, 1, c);
   R v = vref, w = wref;
   const R H1 = (u_c - u) >= 0 ? R(1) : R(0);
   const R H2 = (u - u_c) >= 0 ? R(1) : R(0);
-  v += dt * (H1 * (R(1) - v) / tau_v_m - H2 * v / tau_v_p);
-  w += dt * (H1 * (R(1) - w) / tau_w_m - H2 * w / tau_w_p);
+  v += dt * (over(H1 * (R(1) - v), tau_v_m, 4) - over(H2 * v, tau_v_p, 5));
+  w += dt * (over(H1 * (R(1) - w), tau_w_m, 6) - over(H2 * w, tau_w_p, 7));
   vref = v;
   wref = w;
-  const R J_fi = -(v * H2 * (R(1) - u) * (u - u_c)) / tau_d;
-  const R J_so = u * H1 / tau_o + H2 / tau_r;
+  const R J_fi = over(-(v * H2 * (R(1) - u) * (u - u_c)), tau_d, 0);
+  const R J_so = over(u * H1, tau_o, 1) + over(H2, tau_r, 2);
   // calc_Jsi receives v (fenton_karma_2d.py:326)
-  const R J_si = -v * (R(1) + ftanh(k * (u - uc_si))) / (R(2) * tau_si);
+  const R J_si = over(-v * (R(1) + ftanh(k * (u - uc_si))), R(2) * tau_si, 8);
   return un + dt * (-J_fi - J_so - J_si);
 }
 
@@ -353,11 +387,15 @@ __device__ __forceinline__ R ionic_bo(R u, R un, SP& S, int64_t c,
 }
 
 // ---- Luo-Rudy 1991  luo_rudy91_2d.py:158-510 --------------------------------
+// FP64: bound by VALU issue and, on sheets of a wave or two per SIMD, by the
+// chain of dependent operations.  Divisions through dv / divc and the five
+// parameter-only logarithms and roots from the host: 291 x 259 iso 11.0 ->
+// 9.3 us per step, the same bits.
 template <typename R>
 __device__ __forceinline__ R lr91_gate(R var, R dt, R alpha, R beta) {
-  const R tau = R(1) / (alpha + beta);
-  const R inf = alpha / (alpha + beta);
-  var += dt * (inf - var) / tau;
+  const R tau = dv(R(1), alpha + beta);
+  const R inf = dv(alpha, alpha + beta);
+  var += dv(dt * (inf - var), tau);
   return var;
 }
 
@@ -369,8 +407,12 @@ __device__ __forceinline__ U ionic_lr91(U u_in, U un, SP& S, int64_t c, R dt,
           gkp = par<R>(P, 4), gb = par<R>(P, 5), ko = par<R>(P, 6), ki = par<R>(P, 7),
           nai = par<R>(P, 8), nao = par<R>(P, 9), R_ = par<R>(P, 11), T = par<R>(P, 12),
           F = par<R>(P, 13), PR_NaK = par<R>(P, 14);
-  // E_Na = R*T/F*np.log(nao/nai) (computed once per launch in the reference)
-  const R E_Na = R_ * T / F * flog(nao / nai);
+  // E_Na, E_K, E_K1, G_K, G_K1 depend on the parameters only (the reference
+  // computes them once per launch): the FP64 path takes the host's values
+  constexpr bool F64 = sizeof(R) == 8;
+  R E_Na;
+  if constexpr (F64) E_Na = P.v[kLrENa];
+  else E_Na = R_ * T / F * flog(nao / nai);
   auto&& mr = ref<R>(S, 0, c);
   auto&& hr = ref<R>(S, 1, c);
   auto&& jr = ref<R>(S, 2, c);
@@ -383,25 +425,25 @@ __device__ __forceinline__ U ionic_lr91(U u_in, U un, SP& S, int64_t c, R dt,
   {
     R alpha_h = 0, beta_h = 0, beta_J = 0, alpha_J = 0;
     if (u >= R(-40.0)) {
-      beta_h = R(1.0) / (R(0.13) * (R(1) + fexp((u + R(10.66)) / R(-11.1))));
-      beta_J = R(0.3) * fexp(R(-2.535 * 1e-07) * u) /
-               (R(1) + fexp(R(-0.1) * (u + R(32))));
+      beta_h = dv(R(1.0), R(0.13) * (R(1) + fexp(divc(u + R(10.66), R(-11.1)))));
+      beta_J = dv(R(0.3) * fexp(R(-2.535 * 1e-07) * u), R(1) + fexp(R(-0.1) * (u + R(32))));
     } else {
-      alpha_h = R(0.135) * fexp((R(80) + u) / R(-6.8));
+      alpha_h = R(0.135) * fexp(divc(R(80) + u, R(-6.8)));
       beta_h = R(3.56) * fexp(R(0.079) * u) +
                R(3.1 * 100000.0) * fexp(R(0.35) * u);
-      beta_J = R(0.1212) * fexp(R(-0.01052) * u) /
-               (R(1) + fexp(R(-0.1378) * (u + R(40.14))));
-      alpha_J = (R(-1.2714 * 100000.0) * fexp(R(0.2444) * u) -
-                 R(3.474 * 1e-05) * fexp(R(-0.04391) * u)) *
-                (u + R(37.78)) / (R(1) + fexp(R(0.311) * (u + R(79.23))));
+      beta_J = dv(R(0.1212) * fexp(R(-0.01052) * u),
+                  R(1) + fexp(R(-0.1378) * (u + R(40.14))));
+      alpha_J = dv((R(-1.2714 * 100000.0) * fexp(R(0.2444) * u) -
+                    R(3.474 * 1e-05) * fexp(R(-0.04391) * u)) *
+                       (u + R(37.78)),
+                   R(1) + fexp(R(0.311) * (u + R(79.23))));
     }
     R alpha_m;
     if constexpr (sizeof(R) == 4)
       alpha_m = R(3.2) / exprel(R(-0.1) * (u + R(47.13)));
     else
-      alpha_m = R(0.32) * (u + R(47.13)) / (R(1) - fexp(R(-0.1) * (u + R(47.13))));
-    const R beta_m = R(0.08) * fexp(-u / R(11));
+      alpha_m = dv(R(0.32) * (u + R(47.13)), R(1) - fexp(R(-0.1) * (u + R(47.13))));
+    const R beta_m = R(0.08) * fexp(divc(-u, R(11)));
     const R m = lr91_gate<R>(mr, dt, alpha_m, beta_m);
     const R h = lr91_gate<R>(hr, dt, alpha_h, beta_h);
     const R j = lr91_gate<R>(jr, dt, alpha_J, beta_J);
@@ -416,14 +458,14 @@ __device__ __forceinline__ U ionic_lr91(U u_in, U un, SP& S, int64_t c, R dt,
     R d = dr, f = fr, cai = cair;
     const R E_Si = R(7.7) - R(13.0287) * flog(cai);
     isi = gsi * d * f * (u - E_Si);
-    const R alpha_d = R(0.095) * fexp(R(-0.01) * (u - R(5))) /
-                      (R(1) + fexp(R(-0.072) * (u - R(5))));
-    const R beta_d = R(0.07) * fexp(R(-0.017) * (u + R(44))) /
-                     (R(1) + fexp(R(0.05) * (u + R(44))));
-    const R alpha_f = R(0.012) * fexp(R(-0.008) * (u + R(28))) /
-                      (R(1) + fexp(R(0.15) * (u + R(28))));
-    const R beta_f = R(0.0065) * fexp(R(-0.02) * (u + R(30))) /
-                     (R(1) + fexp(R(-0.2) * (u + R(30))));
+    const R alpha_d = dv(R(0.095) * fexp(R(-0.01) * (u - R(5))),
+                         R(1) + fexp(R(-0.072) * (u - R(5))));
+    const R beta_d = dv(R(0.07) * fexp(R(-0.017) * (u + R(44))),
+                        R(1) + fexp(R(0.05) * (u + R(44))));
+    const R alpha_f = dv(R(0.012) * fexp(R(-0.008) * (u + R(28))),
+                         R(1) + fexp(R(0.15) * (u + R(28))));
+    const R beta_f = dv(R(0.0065) * fexp(R(-0.02) * (u + R(30))),
+                        R(1) + fexp(R(-0.2) * (u + R(30))));
     d = lr91_gate<R>(d, dt, alpha_d, beta_d);
     f = lr91_gate<R>(f, dt, alpha_f, beta_f);
     cai += dt * (R(-0.0001) * isi + R(0.07) * (R(0.0001) - cai));
@@ -434,37 +476,49 @@ __device__ __forceinline__ U ionic_lr91(U u_in, U un, SP& S, int64_t c, R dt,
   // calc_ik: the current uses the old x
   R ik;
   {
-    const R E_K = R_ * T / F * flog((ko + PR_NaK * nao) / (ki + PR_NaK * nai));
-    const R G_K = gk * fsqrt(ko / R(5.4));
+    R E_K, G_K;
+    if constexpr (F64) {
+      E_K = P.v[kLrEK];
+      G_K = P.v[kLrGK];
+    } else {
+      E_K = R_ * T / F * flog((ko + PR_NaK * nao) / (ki + PR_NaK * nai));
+      G_K = gk * fsqrt(ko / R(5.4));
+    }
     R Xi;
     if (u > R(-100)) {
       if constexpr (sizeof(R) == 4)
         Xi = R(2.837 * 0.04) * exprel(R(0.04) * (u + R(77))) / fexp(R(0.04) * (u + R(35)));
       else
-        Xi = R(2.837) * (fexp(R(0.04) * (u + R(77))) - R(1)) /
-             ((u + R(77)) * fexp(R(0.04) * (u + R(35))));
+        Xi = dv(R(2.837) * (fexp(R(0.04) * (u + R(77))) - R(1)),
+                (u + R(77)) * fexp(R(0.04) * (u + R(35))));
     } else {
       Xi = R(1);
     }
     const R x = xr;
     ik = G_K * x * Xi * (u - E_K);
-    const R alpha_x = R(0.0005) * fexp(R(0.083) * (u + R(50))) /
-                      (R(1) + fexp(R(0.057) * (u + R(50))));
-    const R beta_x = R(0.0013) * fexp(R(-0.06) * (u + R(20))) /
-                     (R(1) + fexp(R(-0.04) * (u + R(20))));
+    const R alpha_x = dv(R(0.0005) * fexp(R(0.083) * (u + R(50))),
+                         R(1) + fexp(R(0.057) * (u + R(50))));
+    const R beta_x = dv(R(0.0013) * fexp(R(-0.06) * (u + R(20))),
+                        R(1) + fexp(R(-0.04) * (u + R(20))));
     xr = lr91_gate<R>(x, dt, alpha_x, beta_x);
   }
-  const R E_K1 = R_ * T / F * flog(ko / ki);
+  R E_K1, G_K1;
+  if constexpr (F64) {
+    E_K1 = P.v[kLrEK1];
+    G_K1 = P.v[kLrGK1];
+  } else {
+    E_K1 = R_ * T / F * flog(ko / ki);
+    G_K1 = gk1 * fsqrt(ko / R(5.4));
+  }
   // calc_ik1
-  const R alpha_K1 = R(1.02) / (R(1) + fexp(R(0.2385) * (u - E_K1 - R(59.215))));
-  const R beta_K1 = (R(0.49124) * fexp(R(0.08032) * (u - E_K1 + R(5.476))) +
-                     fexp(R(0.06175) * (u - E_K1 - R(594.31)))) /
-                    (R(1) + fexp(R(-0.5143) * (u - E_K1 + R(4.753))));
-  const R K_1x = alpha_K1 / (alpha_K1 + beta_K1);
-  const R G_K1 = gk1 * fsqrt(ko / R(5.4));
+  const R alpha_K1 = dv(R(1.02), R(1) + fexp(R(0.2385) * (u - E_K1 - R(59.215))));
+  const R beta_K1 = dv(R(0.49124) * fexp(R(0.08032) * (u - E_K1 + R(5.476))) +
+                           fexp(R(0.06175) * (u - E_K1 - R(594.31))),
+                       R(1) + fexp(R(-0.5143) * (u - E_K1 + R(4.753))));
+  const R K_1x = dv(alpha_K1, alpha_K1 + beta_K1);
   const R ik1 = G_K1 * K_1x * (u - E_K1);
   // calc_ikp, calc_ib
-  const R K_p = R(1.0) / (R(1) + fexp((R(7.488) - u) / R(5.98)));
+  const R K_p = dv(R(1.0), R(1) + fexp(divc(R(7.488) - u, R(5.98))));
   const R ikp = gkp * K_p * (u - E_K1);
   const R ib = gb * (u + R(59.87));
   const R ik1t = ik1 + ikp + ib;
@@ -743,9 +797,12 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
 // state order = the kernel's parameter order (courtemanche_2d.py:568-569):
 // nai ki cai caup carel m h j_ d f oa oi ua ui xs xr fca irel vrel urel wrel;
 // the model passes its xr array in the xs slot and vice versa.
+// FP64: bound by VALU issue.  Divisions through dv / divc / div_rn, the
+// parameter-only quantities from the host and pow15 for the device pow:
+// 514 x 387, 10 % fibrosis, per-node fibres, 49.8 -> 37.6 us per step.
 template <typename R>
 __device__ __forceinline__ R crn_gate(R x, R x_inf, R tau_x, R dt) {
-  return x_inf - (x_inf - x) * fexp(-dt / tau_x);
+  return x_inf - (x_inf - x) * fexp(dv(-dt, tau_x));
 }
 
 template <typename R, typename SP, typename U = R>
@@ -771,9 +828,18 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
   auto&& carelr = ref<R>(S, 4, c);
   const R nai = nair, ki = kir, cai = cair, caup = caupr, carel = carelr;
   // calc_equilibrum_potentials
-  const R ena = R_ * T / F * flog(nao / nai);
-  const R ek = R_ * T / F * flog(ko / ki);
-  const R eca = R_ * T / (R(2) * F) * flog(cao / cai);
+  constexpr bool F64 = sizeof(R) == 8;
+  const R rtf = F64 ? par<R>(P, kCrnRTF) : R_ * T / F;
+  const R rt2f = F64 ? par<R>(P, kCrnRT2F) : R_ * T / (R(2) * F);
+  const R ena = rtf * flog(dv(nao, nai));
+  const R ek = rtf * flog(dv(ko, ki));
+  const R eca = rt2f * flog(dv(cao, cai));
+  // x / b for a uniform b whose reciprocal is derived parameter iq
+  auto divu = [&](R x, R b, int iq) -> R {
+    if constexpr (F64) return div_rn(x, b, P.v[iq]);
+    else return x / b;
+  };
+  auto overRT = [&](R x) -> R { return divu(x, F64 ? par<R>(P, kCrnRT) : R_ * T, kCrnInvRT); };
   // calc_gating_m / h / j
   R m, h, j;
   {
@@ -785,12 +851,12 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
       if (u == R(-47.13)) {
         am = R(3.2);
       } else {
-        am = R(0.32) * (u + R(47.13)) / (R(1) - fexp(R(-0.1) * (u + R(47.13))));
+        am = dv(R(0.32) * (u + R(47.13)), R(1) - fexp(R(-0.1) * (u + R(47.13))));
       }
     }
-    const R bm = R(0.08) * fexp(-u / R(11));
-    const R m_inf = am / (am + bm);
-    const R tau_m = R(1) / (am + bm);
+    const R bm = R(0.08) * fexp(divc(-u, R(11)));
+    const R m_inf = dv(am, am + bm);
+    const R tau_m = dv(R(1), am + bm);
     m = crn_gate<R>(mr, m_inf, tau_m, dt);
     mr = m;
   }
@@ -799,13 +865,13 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
     R ah, bh;
     if (u >= R(-40)) {
       ah = R(0);
-      bh = R(1) / (R(0.13) * (R(1) + fexp(-(u + R(10.66)) / R(11.1))));
+      bh = dv(R(1), R(0.13) * (R(1) + fexp(divc(-(u + R(10.66)), R(11.1)))));
     } else {
-      ah = R(0.135) * fexp(-(R(80) + u) / R(6.8));
+      ah = R(0.135) * fexp(divc(-(R(80) + u), R(6.8)));
       bh = R(3.56) * fexp(R(0.079) * u) + R(310000) * fexp(R(0.35) * u);
     }
-    const R h_inf = ah / (ah + bh);
-    const R tau_h = R(1) / (ah + bh);
+    const R h_inf = dv(ah, ah + bh);
+    const R tau_h = dv(R(1), ah + bh);
     h = crn_gate<R>(hr, h_inf, tau_h, dt);
     hr = h;
   }
@@ -814,32 +880,33 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
     R aj, bj;
     if (u >= R(-40)) {
       aj = R(0);
-      bj = R(0.3) * fexp(R(-2.535e-07) * u) / (R(1) + fexp(R(-0.1) * (u + R(32))));
+      bj = dv(R(0.3) * fexp(R(-2.535e-07) * u), R(1) + fexp(R(-0.1) * (u + R(32))));
     } else {
-      aj = (R(-127140) * fexp(R(0.2444) * u) - R(3.474e-05) * fexp(R(-0.04391) * u)) *
-           (u + R(37.78)) / (R(1) + fexp(R(0.311) * (u + R(79.23))));
-      bj = R(0.1212) * fexp(R(-0.01052) * u) / (R(1) + fexp(R(-0.1378) * (u + R(40.14))));
+      aj = dv((R(-127140) * fexp(R(0.2444) * u) - R(3.474e-05) * fexp(R(-0.04391) * u)) *
+                  (u + R(37.78)),
+              R(1) + fexp(R(0.311) * (u + R(79.23))));
+      bj = dv(R(0.1212) * fexp(R(-0.01052) * u), R(1) + fexp(R(-0.1378) * (u + R(40.14))));
     }
-    const R j_inf = aj / (aj + bj);
-    const R tau_j = R(1) / (aj + bj);
-    j = j_inf - (j_inf - jr) * fexp(-dt / tau_j);
+    const R j_inf = dv(aj, aj + bj);
+    const R tau_j = dv(R(1), aj + bj);
+    j = j_inf - (j_inf - jr) * fexp(dv(-dt, tau_j));
     jr = j;
   }
   const R ina = gna * (m * (m * m)) * h * j * (u - ena);
-  const R ik1 = gk1 * (u - ek) / (R(1) + fexp(R(0.07) * (u + R(80))));
+  const R ik1 = dv(gk1 * (u - ek), R(1) + fexp(R(0.07) * (u + R(80))));
   // calc_ito
   R ito;
   {
     auto&& oar = ref<R>(S, 10, c);
     auto&& oir = ref<R>(S, 11, c);
-    const R ao = R(0.65) / (fexp(-(u + R(10)) / R(8.5)) + fexp(-(u - R(30)) / R(59.0)));
-    const R bo = R(0.65) / (R(2.5) + fexp((u + R(82)) / R(17.0)));
-    const R tau_o = R(1) / (kq10 * (ao + bo));
-    const R o_inf = R(1) / (R(1) + fexp(-(u + R(20.47)) / R(17.54)));
-    const R aoi = R(1) / (R(18.53) + fexp((u + R(113.7)) / R(10.95)));
-    const R boi = R(1) / (R(35.56) + fexp(-(u + R(1.26)) / R(7.44)));
-    const R tau_oi = R(1) / (kq10 * (aoi + boi));
-    const R oi_inf = R(1) / (R(1) + fexp((u + R(43.1)) / R(5.3)));
+    const R ao = dv(R(0.65), fexp(divc(-(u + R(10)), R(8.5))) + fexp(divc(-(u - R(30)), R(59.0))));
+    const R bo = dv(R(0.65), R(2.5) + fexp(divc(u + R(82), R(17.0))));
+    const R tau_o = dv(R(1), kq10 * (ao + bo));
+    const R o_inf = dv(R(1), R(1) + fexp(divc(-(u + R(20.47)), R(17.54))));
+    const R aoi = dv(R(1), R(18.53) + fexp(divc(u + R(113.7), R(10.95))));
+    const R boi = dv(R(1), R(35.56) + fexp(divc(-(u + R(1.26)), R(7.44))));
+    const R tau_oi = dv(R(1), kq10 * (aoi + boi));
+    const R oi_inf = dv(R(1), R(1) + fexp(divc(u + R(43.1), R(5.3))));
     const R oa = crn_gate<R>(oar, o_inf, tau_o, dt);
     const R oi = crn_gate<R>(oir, oi_inf, tau_oi, dt);
     oar = oa;
@@ -851,15 +918,15 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
   {
     auto&& uar = ref<R>(S, 12, c);
     auto&& uir = ref<R>(S, 13, c);
-    const R gkur = R(0.005) + R(0.05) / (R(1) + fexp(-(u - R(15)) / R(13.0)));
-    const R aua = R(0.65) / (fexp(-(u + R(10)) / R(8.5)) + fexp(-(u - R(30)) / R(59.0)));
-    const R bua = R(0.65) / (R(2.5) + fexp((u + R(82)) / R(17.0)));
-    const R tau_ua = R(1) / (kq10 * (aua + bua));
-    const R ua_inf = R(1) / (R(1) + fexp(-(u + R(30.3)) / R(9.6)));
-    const R aui = R(1) / (R(21) + fexp(-(u - R(185)) / R(28.0)));
-    const R bui = fexp((u - R(158)) / R(16.0));
-    const R tau_ui = R(1) / (kq10 * (aui + bui));
-    const R ui_inf = R(1) / (R(1) + fexp((u - R(99.45)) / R(27.48)));
+    const R gkur = R(0.005) + dv(R(0.05), R(1) + fexp(divc(-(u - R(15)), R(13.0))));
+    const R aua = dv(R(0.65), fexp(divc(-(u + R(10)), R(8.5))) + fexp(divc(-(u - R(30)), R(59.0))));
+    const R bua = dv(R(0.65), R(2.5) + fexp(divc(u + R(82), R(17.0))));
+    const R tau_ua = dv(R(1), kq10 * (aua + bua));
+    const R ua_inf = dv(R(1), R(1) + fexp(divc(-(u + R(30.3)), R(9.6))));
+    const R aui = dv(R(1), R(21) + fexp(divc(-(u - R(185)), R(28.0))));
+    const R bui = fexp(divc(u - R(158), R(16.0)));
+    const R tau_ui = dv(R(1), kq10 * (aui + bui));
+    const R ui_inf = dv(R(1), R(1) + fexp(divc(u - R(99.45), R(27.48))));
     const R ua = crn_gate<R>(uar, ua_inf, tau_ua, dt);
     const R ui = crn_gate<R>(uir, ui_inf, tau_ui, dt);
     uar = ua;
@@ -876,14 +943,14 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
       axr = R(0.0003 * 5) / exprel(-(u + R(14.1)) / R(5));
       bxr = R(7.3898e-05 * 5.1237) / exprel((u - R(3.3328)) / R(5.1237));
     } else {
-      axr = R(0.0003) * (u + R(14.1)) / (R(1) - fexp(-(u + R(14.1)) / R(5)));
-      bxr = R(7.3898e-05) * (u - R(3.3328)) / (fexp((u - R(3.3328)) / R(5.1237)) - R(1));
+      axr = dv(R(0.0003) * (u + R(14.1)), R(1) - fexp(divc(-(u + R(14.1)), R(5))));
+      bxr = dv(R(7.3898e-05) * (u - R(3.3328)), fexp(divc(u - R(3.3328), R(5.1237))) - R(1));
     }
-    const R tau_xr = R(1) / (axr + bxr);
-    const R xr_inf = R(1) / (R(1) + fexp(-(u + R(14.1)) / R(6.5)));
+    const R tau_xr = dv(R(1), axr + bxr);
+    const R xr_inf = dv(R(1), R(1) + fexp(divc(-(u + R(14.1)), R(6.5))));
     const R xr = crn_gate<R>(xrr, xr_inf, tau_xr, dt);
     xrr = xr;
-    ikr = gkr * xr * (u - ek) / (R(1) + fexp((u + R(15)) / R(22.4)));
+    ikr = dv(gkr * xr * (u - ek), R(1) + fexp(divc(u + R(15), R(22.4))));
   }
   // calc_iks on the kernel's xs slot (index 14)
   R iks;
@@ -894,11 +961,11 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
       axs = R(4e-05 * 17) / exprel(-(u - R(19.9)) / R(17));
       bxs = R(3.5e-05 * 9) / exprel((u - R(19.9)) / R(9));
     } else {
-      axs = R(4e-05) * (u - R(19.9)) / (R(1) - fexp(-(u - R(19.9)) / R(17)));
-      bxs = R(3.5e-05) * (u - R(19.9)) / (fexp((u - R(19.9)) / R(9)) - R(1));
+      axs = dv(R(4e-05) * (u - R(19.9)), R(1) - fexp(divc(-(u - R(19.9)), R(17))));
+      bxs = dv(R(3.5e-05) * (u - R(19.9)), fexp(divc(u - R(19.9), R(9))) - R(1));
     }
-    const R tau_xs = R(1) / (R(2) * (axs + bxs));
-    const R xs_inf = R(1) / fsqrt(R(1) + fexp(-(u - R(19.9)) / R(12.7)));
+    const R tau_xs = dv(R(1), R(2) * (axs + bxs));
+    const R xs_inf = dv(R(1), fsqrt(R(1) + fexp(divc(-(u - R(19.9)), R(12.7)))));
     const R xs = crn_gate<R>(xsr, xs_inf, tau_xs, dt);
     xsr = xs;
     iks = gks * (xs * xs) * (u - ek);
@@ -914,15 +981,15 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
       const R y = -(u + R(10)) / R(6.24);
       tau_d = exprel(y) / (R(6.24 * 0.035) * (R(1) + fexp(y)));
     } else {
-      tau_d = (R(1) - fexp(-(u + R(10)) / R(6.24))) /
-              (R(0.035) * (u + R(10)) * (R(1) + fexp(-(u + R(10)) / R(6.24))));
+      const R e = fexp(divc(-(u + R(10)), R(6.24)));
+      tau_d = dv(R(1) - e, R(0.035) * (u + R(10)) * (R(1) + e));
     }
-    const R d_inf = R(1) / (R(1) + fexp(-(u + R(10)) / R(8.0)));
-    const R tau_f = R(9) / (R(0.0197) * fexp(-R(0.0337 * 0.0337) * ((u + R(10)) * (u + R(10)))) +
-                            R(0.02));
-    const R f_inf = R(1) / (R(1) + fexp((u + R(28)) / R(6.9)));
+    const R d_inf = dv(R(1), R(1) + fexp(divc(-(u + R(10)), R(8.0))));
+    const R tau_f = dv(R(9), R(0.0197) * fexp(-R(0.0337 * 0.0337) * ((u + R(10)) * (u + R(10)))) +
+                                 R(0.02));
+    const R f_inf = dv(R(1), R(1) + fexp(divc(u + R(28), R(6.9))));
     const R tau_fca = R(2);
-    const R fca_inf = R(1) / (R(1) + cai / R(0.00035));
+    const R fca_inf = dv(R(1), R(1) + divc(cai, R(0.00035)));
     const R d = crn_gate<R>(dr, d_inf, tau_d, dt);
     const R f = crn_gate<R>(fr, f_inf, tau_f, dt);
     const R fca = crn_gate<R>(fcar, fca_inf, tau_fca, dt);
@@ -932,25 +999,26 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
     ical = gcal * d * f * fca * (u - R(65));
   }
   // calc_inak
-  const R sig = R(1 / 7.0) * (fexp(nao / R(67.3)) - R(1));
-  const R fnak = R(1) / (R(1) + R(0.1245) * fexp(R(-0.1) * (F * u) / (R_ * T)) +
-                         R(0.0365) * sig * fexp(-(F * u) / (R_ * T)));
-  const R inak = inakmax * fnak * (R(1) / (R(1) + fpow(kmnai / nai, R(1.5)))) *
-                 (ko / (ko + kmko));
+  const R sig = F64 ? par<R>(P, kCrnSig) : R(1 / 7.0) * (fexp(nao / R(67.3)) - R(1));
+  const R ko_km = F64 ? par<R>(P, kCrnKo) : ko / (ko + kmko);
+  const R fnak = dv(R(1), R(1) + R(0.1245) * fexp(overRT(R(-0.1) * (F * u))) +
+                              R(0.0365) * sig * fexp(overRT(-(F * u))));
+  const R inak = inakmax * fnak * dv(R(1), R(1) + fpow15(dv(kmnai, nai))) * ko_km;
   // calc_inaca
   const R gamma = R(0.35);
-  const R exp_term = fexp(gamma * (F * u) / (R_ * T));
-  const R exp_rev_term = fexp((gamma - R(1)) * (F * u) / (R_ * T));
-  const R nao3 = nao * (nao * nao);
+  const R exp_term = fexp(overRT(gamma * (F * u)));
+  const R exp_rev_term = fexp(overRT((gamma - R(1)) * (F * u)));
+  const R nao3 = F64 ? par<R>(P, kCrnNao3) : nao * (nao * nao);
   const R numerator =
       inacamax * (exp_term * (nai * (nai * nai)) * cao - exp_rev_term * nao3 * cai);
   const R term1 = kmnancx * (kmnancx * kmnancx) + nao3;
   const R term2 = kmcancx + cao;
+  const R term12 = F64 ? par<R>(P, kCrnT12) : term1 * term2;
   const R term3 = R(1) + ksatncx * exp_rev_term;
-  const R inaca = numerator / (term1 * term2 * term3);
+  const R inaca = dv(numerator, term12 * term3);
   const R ibca = gcab * (u - eca);
   const R ibna = gnab * (u - ena);
-  const R ipca = ipcamax * cai / (cai + R(0.0005));
+  const R ipca = dv(ipcamax * cai, cai + R(0.0005));
   // calc_irel (uses the irel stored by the previous step)
   R irel;
   {
@@ -959,7 +1027,11 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
     auto&& urr = ref<R>(S, 19, c);
     auto&& wrr = ref<R>(S, 20, c);
     const R tau_u = R(8);
-    const R Fn = R(1e-12) * Vrel * irr - R(5 * 1e-13) / F * (R(0.5) * ical - R(0.2) * inaca);
+    // Fn spans decades around thresholds 1e-15 wide: the exponentials below
+    // overflow in ordinary use, so their divisions keep the full sequence
+    // (1 / inf = 0)
+    const R fnf = F64 ? par<R>(P, kCrnFnF) : R(5 * 1e-13) / F;
+    const R Fn = R(1e-12) * Vrel * irr - fnf * (R(0.5) * ical - R(0.2) * inaca);
     const R u_inf = R(1) / (R(1) + fexp(-(Fn - R(3.4175e-13)) / R(1.367e-15)));
     const R tau_v = R(1.91) + R(2.09) / (R(1) + fexp(-(Fn - R(3.4175e-13)) / R(1.367e-15)));
     const R v_inf = R(1) - R(1) / (R(1) + fexp(-(Fn - R(6.835e-14)) / R(1.367e-15)));
@@ -968,10 +1040,10 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
       const R y = -(u - R(7.9)) / R(5.0);
       tau_w = R(6.0 / 5.0) * exprel(y) / (R(1) + R(0.3) * fexp(y));
     } else {
-      tau_w = R(6) * (R(1) - fexp(-(u - R(7.9)) / R(5.0))) /
-              ((R(1) + R(0.3) * fexp(-(u - R(7.9)) / R(5.0))) * (u - R(7.9)));
+      const R e = fexp(divc(-(u - R(7.9)), R(5.0)));
+      tau_w = dv(R(6) * (R(1) - e), (R(1) + R(0.3) * e) * (u - R(7.9)));
     }
-    const R w_inf = R(1) - R(1) / (R(1) + fexp(-(u - R(40)) / R(17.0)));
+    const R w_inf = R(1) - dv(R(1), R(1) + fexp(divc(-(u - R(40)), R(17.0))));
     const R urel = crn_gate<R>(urr, u_inf, tau_u, dt);
     const R vrel = crn_gate<R>(vrr, v_inf, tau_v, dt);
     const R wrel = crn_gate<R>(wrr, w_inf, tau_w, dt);
@@ -981,21 +1053,26 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
     irel = krel * (urel * urel) * vrel * wrel * (carel - cai);
     irr = irel;
   }
-  const R itr = (caup - carel) / R(180);
-  const R iup = iupmax / (R(1) + kup / cai);
-  const R iupleak = caup / caupmax * iupmax;
-  caupr = caup + dt * (iup - iupleak - itr * (Vrel / Vup));
-  nair = nai + dt * ((R(-3) * inak - R(3) * inaca - ibna - ina) / (F * Vj));
-  kir = ki + dt * ((R(2) * inak - ik1 - ito - ikur - ikr - iks - ibk) / (F * Vj));
+  auto overFVj = [&](R x) -> R {
+    return divu(x, F64 ? par<R>(P, kCrnFVj) : F * Vj, kCrnInvFVj);
+  };
+  const R vrel_vup = F64 ? par<R>(P, kCrnVrelVup) : Vrel / Vup;
+  const R itr = divc(caup - carel, R(180));
+  const R iup = dv(iupmax, R(1) + dv(kup, cai));
+  const R iupleak = divu(caup, caupmax, kCrnInvCaup) * iupmax;
+  caupr = caup + dt * (iup - iupleak - itr * vrel_vup);
+  nair = nai + dt * overFVj(R(-3) * inak - R(3) * inaca - ibna - ina);
+  kir = ki + dt * overFVj(R(2) * inak - ik1 - ito - ikur - ikr - iks - ibk);
   {
-    const R B1 = (R(2) * inaca - ipca - ical - ibca) / (R(2) * F * Vj) +
-                 (Vup * (iupleak - iup) + irel * Vrel) / Vj;
-    const R B2 = R(1) + trpnmax * kmtrpn / ((cai + kmtrpn) * (cai + kmtrpn)) +
-                 cmdnmax * kmcmdn / ((cai + kmcmdn) * (cai + kmcmdn));
-    cair = cai + dt * (B1 / B2);
+    const R B1 = divu(R(2) * inaca - ipca - ical - ibca,
+                      F64 ? par<R>(P, kCrn2FVj) : R(2) * F * Vj, kCrnInv2FVj) +
+                 divu(Vup * (iupleak - iup) + irel * Vrel, Vj, kCrnInvVj);
+    const R B2 = R(1) + dv(trpnmax * kmtrpn, (cai + kmtrpn) * (cai + kmtrpn)) +
+                 dv(cmdnmax * kmcmdn, (cai + kmcmdn) * (cai + kmcmdn));
+    cair = cai + dt * dv(B1, B2);
   }
-  carelr = carel + dt * ((itr - irel) /
-                         (R(1) + csqnmax * kmcsqn / ((carel + kmcsqn) * (carel + kmcsqn))));
+  carelr = carel + dt * dv(itr - irel, R(1) + dv(csqnmax * kmcsqn,
+                                                 (carel + kmcsqn) * (carel + kmcsqn)));
   return un - dt * (ina + ik1 + ito + ikur + ikr + iks + ical + ipca + inak +
                     inaca + ibna + ibca);
 }
