@@ -224,6 +224,7 @@ __global__ __launch_bounds__(kBlock, (batch_min_waves<MODEL, R>())) void k_batch
   const uint32_t b = blockIdx.x;
   const uint32_t lb = XCD ? (b % kXcds) * a.per_xcd + b / kXcds : b;
   if (lb >= a.nblocks) return;
+  if constexpr (uses_exp64<MODEL, R>()) exp_table_to_lds();
   // the record, read uniformly before any store
   const int32_t t = __builtin_amdgcn_readfirstlane(a.btis[lb]);
   const int32_t start = __builtin_amdgcn_readfirstlane(a.bstart[lb]);

@@ -1050,6 +1050,7 @@ __global__ __launch_bounds__(kBlock, (step_min_waves<NDIM, MODEL, PREC>())) void
     const KArgs<R, UType<MODEL, R>> a) {
   const int64_t lb = logical_block(a.per_xcd);
   if (lb >= a.nblocks) return;
+  if constexpr (uses_exp64<MODEL, R>()) exp_table_to_lds();
   const int64_t c = lb * kBlock + threadIdx.x;
   if (c >= a.N) return;
   const int32_t step = a.step_in ? *a.step_in : a.step;
@@ -1250,6 +1251,7 @@ __global__ __launch_bounds__(kBlock) void k_ionic(UType<MODEL, R>* __restrict__ 
                                                   const StatePtrs st,
                                                   const int64_t* __restrict__ idx,
                                                   int64_t n, R dt, const Params P) {
+  if constexpr (uses_exp64<MODEL, R>()) exp_table_to_lds();
   const int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (q >= n) return;
   const int64_t c = idx[q];

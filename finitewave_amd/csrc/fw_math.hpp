@@ -84,14 +84,16 @@ FW_HD inline double t128_exp_special(double x, double tmp, uint64_t sbits, uint6
   return 0x1p-1022 * y;
 }
 
-FW_HD inline double t128_exp(double x) {
+// tab: kExpTab, or a kernel's copy of it
+template <typename Tab>
+FW_HD inline double t128_exp_tab(double x, const Tab* tab) {
   double kd = fma(mt::kInvLn2N, x, mt::kShift);
   const uint64_t ki = f64_bits(kd);
   kd -= mt::kShift;
   const double r = fma(kd, mt::kNegLn2loN, fma(kd, mt::kNegLn2hiN, x));
   const uint32_t j = (uint32_t)ki & 127u;
-  const double tail = f64_from(mt::kExpTab[2 * j]);
-  const uint64_t sbits = mt::kExpTab[2 * j + 1] + (ki << 45);
+  const double tail = f64_from(tab[2 * j]);
+  const uint64_t sbits = tab[2 * j + 1] + (ki << 45);
   const double r2 = r * r;
   const double tmp =
       fma(r2 * r2, fma(r, mt::kC5, mt::kC4), fma(r2, fma(r, mt::kC3, mt::kC2), tail + r));
@@ -100,6 +102,8 @@ FW_HD inline double t128_exp(double x) {
   const double scale = f64_from(sbits);
   return fma(scale, tmp, scale);
 }
+
+FW_HD inline double t128_exp(double x) { return t128_exp_tab(x, mt::kExpTab); }
 
 FW_HD inline void two_sum(double a, double b, double& s, double& e) {
   s = a + b;

@@ -49,7 +49,25 @@ struct StreamStatePtrs {
 // ---- math dispatch --------------------------------------------------------
 // FP64: the exp/log of fw_math.hpp, whose last bits follow the host libm the
 // reference's numba kernels call (exp bit for bit); FP32: the device library.
-__device__ __forceinline__ double fexp(double x) { return t128_exp(x); }
+// exp's table in LDS, one copy per block: an update calls exp some 40 to 75
+// times, each waiting for its table entry, and an LDS read answers in a
+// fraction of a vector cache hit's time.  The FP64 TP06 step spent half its
+// wave cycles on those waits (1026^2, 9-point: 125 -> 102 us per step, VALU
+// busy 76 % -> 96 %; Courtemanche 514 x 387: 35.8 -> 32.1 us).  Every kernel that
+// calls fexp(double) fills the table first (exp_table_to_lds).
+__device__ __forceinline__ uint64_t* exp_lds() {
+  __shared__ __align__(16) uint64_t tab[256];
+  return tab;
+}
+
+// Called by all work-items of a block, before any of them returns.
+__device__ __forceinline__ void exp_table_to_lds() {
+  uint64_t* const t = exp_lds();
+  for (int q = threadIdx.x; q < 256; q += blockDim.x) t[q] = mt::kExpTab[q];
+  __syncthreads();
+}
+
+__device__ __forceinline__ double fexp(double x) { return t128_exp_tab(x, exp_lds()); }
 __device__ __forceinline__ float fexp(float x) { return __expf(x); }
 __device__ __forceinline__ double flog(double x) { return dd_log(x); }
 __device__ __forceinline__ float flog(float x) { return __logf(x); }
@@ -1131,6 +1149,12 @@ __device__ __forceinline__ U node_update(U uc, SP& S, int64_t c, R dt, const Par
   } else {
     return ionic_update<MODEL, R>(uc, diffusion(), S, c, dt, P);
   }
+}
+
+// models whose FP64 update calls exp (exp_table_to_lds)
+template <int MODEL, typename R>
+constexpr bool uses_exp64() {
+  return MODEL >= 5 && sizeof(R) == 8;
 }
 
 __host__ __device__ constexpr int model_n_params(int model) {
