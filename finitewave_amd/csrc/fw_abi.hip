@@ -4,11 +4,13 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <functional>
 #include <mutex>
 #include <vector>
 
 #include "fw_batch.hpp"
 #include "fw_internal.hpp"
+#include "fw_multi2d.hpp"
 
 namespace fw {
 
@@ -36,6 +38,23 @@ StepLauncher step_launcher(int precision, int model) {
       {fw_step_launch_p1_m0, fw_step_launch_p1_m1, fw_step_launch_p1_m2, fw_step_launch_p1_m3,
        fw_step_launch_p1_m4, fw_step_launch_p1_m5, fw_step_launch_p1_m6, fw_step_launch_p1_m7}};
   if (precision < 0 || precision > 1 || model < 0 || model > 7) return nullptr;
+  return table[precision][model];
+}
+
+#define FW_DECL_MULTI(p, m)                                                     \
+  int fw_multi_launch_p##p##_m##m(const fw_plan*, void*, void*, const StatePtrs&, \
+                                  const TrackArgs&, int32_t, int32_t, int32_t, hipStream_t);
+FW_DECL_MULTI(0, 0) FW_DECL_MULTI(0, 1) FW_DECL_MULTI(0, 2) FW_DECL_MULTI(0, 3)
+FW_DECL_MULTI(0, 4) FW_DECL_MULTI(1, 0) FW_DECL_MULTI(1, 1) FW_DECL_MULTI(1, 2)
+FW_DECL_MULTI(1, 3) FW_DECL_MULTI(1, 4)
+
+MultiLauncher multi_launcher(int precision, int model) {
+  static const MultiLauncher table[2][5] = {
+      {fw_multi_launch_p0_m0, fw_multi_launch_p0_m1, fw_multi_launch_p0_m2,
+       fw_multi_launch_p0_m3, fw_multi_launch_p0_m4},
+      {fw_multi_launch_p1_m0, fw_multi_launch_p1_m1, fw_multi_launch_p1_m2,
+       fw_multi_launch_p1_m3, fw_multi_launch_p1_m4}};
+  if (precision < 0 || precision > 1 || model < 0 || model > 4) return nullptr;
   return table[precision][model];
 }
 
@@ -445,6 +464,28 @@ static int plan_host_init(const fw_plan_desc* desc, fw_plan* p, const char* who)
   return FW_OK;
 }
 
+// The step words' share of their allocation: what follows is aligned for any load.
+constexpr size_t kStepWordBytes = 256;
+
+// The largest sheet stepped by multi-step launches (2000^2 still gains 2 % to
+// 17 %, past it both are bound by HBM), the largest of the models with tanh
+// where multi_shape says so, and the single steps in a row (a long stimulus)
+// that are worth capturing a graph for beside them.
+constexpr int64_t kMultiMaxNodes = (int64_t)1 << 22;
+constexpr int64_t kMultiMaxTanh = (int64_t)1 << 18;
+constexpr int32_t kMultiGraphSteps = 64;
+
+// Bytes of a plan's second state set, 0 for plans without multi-step launches
+// (fw_multi2d.hpp): 2D, light models, uniform half-step fields.
+static size_t multi_alt_bytes(const fw_plan* p) {
+  const fw_plan_desc& d = p->desc;
+  if (d.ndim != 2 || d.model > 4 || d.stencil == FW_STENCIL_WEIGHTS ||
+      p->field_layout != fw::kFieldsUniform || p->N > kMultiMaxNodes)
+    return 0;
+  return (size_t)p->N * model_n_state(d.model) *
+         (d.precision == FW_PREC_FP64 ? sizeof(double) : sizeof(float));
+}
+
 // Whether a plan's step kernel reads float copies of its tabulated fields
 // (FP32 plans whose potential is float)
 static bool wants_float_tables(const fw_plan_desc& d) {
@@ -470,7 +511,9 @@ int fw_plan_create(const fw_plan_desc* desc, fw_plan** out) {
   }
   const int need_fields = needed_fields(d);
   const int64_t N = p->N;
-  hipError_t e = hipMalloc(&p->step_words, 4 * sizeof(int32_t));
+  const size_t alt = multi_alt_bytes(p);
+  hipError_t e = hipMalloc(&p->step_words, kStepWordBytes + alt);
+  if (e == hipSuccess && alt) p->alt = reinterpret_cast<char*>(p->step_words) + kStepWordBytes;
   if (e != hipSuccess) {
     set_error("fw_plan_create: hipMalloc failed: %s", hipGetErrorString(e));
     delete p;
@@ -630,10 +673,192 @@ static int run_plain(const fw_plan* plan, void* u, void* u_new, void* const* sta
   return FW_OK;
 }
 
+// Whether the multi-step launches may use the plan's second state set on
+// `stream`.  One set cannot serve two runs in flight: it goes to the first
+// stream that asks, whose calls are ordered, and runs of the plan on any other
+// stream keep to single steps, as does a stream being captured (its graph may
+// be replayed on any stream) and the per-thread stream (one handle, a stream
+// per thread).
+static bool multi_stream_ok(fw_plan* plan, hipStream_t s) {
+  if (s == hipStreamPerThread) return false;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return false;
+  }
+  uintptr_t none = 0;
+  const uintptr_t me = reinterpret_cast<uintptr_t>(s) + 1;
+  return plan->alt_stream.compare_exchange_strong(none, me) || none == me;
+}
+
+// Steps per launch (K) and region rows of a sheet's multi-step launches; K = 0
+// where single steps are the faster.  A launch costs about 5 us before its
+// first step, then each step the issue of its region's wavefronts: while every
+// block has a CU of its own (256) the most steps and the fewest rows win, as
+// the halo is computed by CUs that would idle.  Past that the halo's work
+// counts and K = 4 takes over (Aliev-Panfilov iso, us per step, K = 8 / 4 /
+// single: 102^2 FP64 0.93 / 1.36 / 3.32, 400^2 2.33 / 2.38 / 3.88, 900^2 7.7 /
+// 6.1 / 9.2; FP32 0.81 / 1.22 / 2.64, 1.73 / 1.86 / 2.94, 5.7 / 4.6 / 6.0).
+// The FP64 Fenton-Karma and Bueno-Orovio updates cost 4 and 10 times as much,
+// so redundant nodes stop paying once CUs are shared (400^2 iso: 5.2 and 10.9
+// at K = 4 against 5.3 and 7.8); in FP32 with the 9-point stencil they do
+// between 400^2 (3.1 and 4.1 against 3.6 and 4.3) and 900^2 (9.2 and 11.3
+// against 8.3 and 10.4), Bueno-Orovio with the 5-point one at 560^2 (4.8
+// against 4.7).
+static int32_t multi_blocks(const fw_plan* plan, int32_t K, int32_t rows) {
+  const int64_t w = kMultiW - 2 * K, h = rows - 2 * K;
+  return (int32_t)(((plan->desc.shape[0] + h - 1) / h) * ((plan->desc.shape[1] + w - 1) / w));
+}
+
+static void multi_shape(const fw_plan* plan, int32_t* K, int32_t* rows) {
+  constexpr int32_t kCus = 256;
+  const fw_plan_desc& d = plan->desc;
+  const bool f64 = d.precision == FW_PREC_FP64, aniso = d.stencil == FW_STENCIL_ANISO;
+  const bool tanh_model = d.model >= 3;  // Fenton-Karma, Bueno-Orovio
+  const bool heavy = f64 && tanh_model;
+  *K = 8;
+  for (int32_t r : {20, 24, 32}) {
+    *rows = r;
+    if (multi_blocks(plan, 8, r) <= kCus) return;
+    if (heavy) break;
+  }
+  *K = 4;
+  *rows = 16;
+  if (heavy) {
+    if (multi_blocks(plan, 4, 16) > kCus) *K = 0;
+  } else if (tanh_model && (aniso || d.model == 4)) {
+    if (plan->N > kMultiMaxTanh) *K = 0;
+  } else if (!(aniso && f64)) {
+    *rows = 32;
+  }
+}
+
+// Steps a run can take in multi-step pairs before a scheduled stimulus
+// applies: the step kernels hand stimulus s + 1 on from step s, so steps
+// [step, step + n) are free of it when no window meets (step, step + n].
+static int64_t stim_free(const fw_plan* plan, int64_t step, int64_t n, int64_t stim_end) {
+  int64_t free_steps = n;
+  for (int32_t q = 0; q < plan->n_stims; ++q) {
+    const int64_t lo = plan->stims[q].step_lo;
+    const int64_t hi = plan->stims[q].step_hi < stim_end ? plan->stims[q].step_hi : stim_end - 1;
+    if (hi < lo || hi <= step) continue;
+    const int64_t until = lo > step + 1 ? lo - step - 1 : 0;
+    if (until < free_steps) free_steps = until;
+  }
+  return free_steps;
+}
+
+// The first step after `step` whose hand-over applies no stimulus, at most
+// `last`.
+static int64_t stim_until(const fw_plan* plan, int64_t step, int64_t last, int64_t stim_end) {
+  while (step < last && stim_free(plan, step, 1, stim_end) == 0) ++step;
+  return step;
+}
+
+// n_steps with multi-step launches wherever they apply, single steps
+// elsewhere (among them the last: u_new then holds the step before).
+// `singles` runs the single steps.  *done = false: nothing launched, the run
+// has no multi-step form.
+typedef std::function<int(void*, void*, int64_t, int32_t, const fw_track_desc*)> Singles;
+static int run_multi(fw_plan* plan, void* u, void* u_new, void* const* state, int64_t step0,
+                     int32_t n_steps, const fw_track_desc* track, hipStream_t s,
+                     const Singles& singles, bool* done) {
+  *done = false;
+  if (!plan->alt) return FW_OK;
+  int32_t shape_k, rows;
+  multi_shape(plan, &shape_k, &rows);
+  // K of a stretch of `room` steps: pairs of the shape's, or of 4 or 2 steps
+  // (a region of 2 K + 4 rows or more owns some)
+  auto fit = [&](int64_t room) {
+    int32_t k = shape_k;
+    while (k > 2 && 2 * k > room) k /= 2;
+    return 2 * k <= room ? k : 0;
+  };
+  int32_t K = fit(n_steps - 1);
+  if (K == 0 || step0 < 0 || step0 + n_steps > INT32_MAX) return FW_OK;
+  int32_t act_on = 0;
+  bool probes = false;
+  if (track && track->act) {
+    act_on = track->act_flags ? track->act_flags[0] != 0 : 1;
+    if (track->act_flags)
+      for (int32_t q = 1; q < n_steps; ++q)
+        if ((track->act_flags[q] != 0) != (act_on != 0)) return FW_OK;
+  }
+  if (track && track->n_probe > 0 && track->probe_rows) {
+    // rows that follow each other, or no row at all
+    const int32_t r0 = track->probe_rows[0];
+    for (int32_t q = 1; q < n_steps; ++q)
+      if (r0 >= 0 ? track->probe_rows[q] != r0 + q : track->probe_rows[q] >= 0) return FW_OK;
+    probes = r0 >= 0;
+  }
+  if (!multi_stream_ok(plan, s)) return FW_OK;
+  *done = true;
+  const int64_t stim_end = track ? track->stim_end : 0;
+  const MultiLauncher L = multi_launcher(plan->desc.precision, plan->desc.model);
+  const StatePtrs st = make_state(state, model_n_state(plan->desc.model));
+  void* a = u;
+  void* b = u_new;
+  int32_t pos = 0;
+  while (pos < n_steps) {
+    const int64_t step = step0 + pos;
+    const int32_t room = (int32_t)stim_free(plan, step, n_steps - 1 - pos, stim_end);
+    K = fit(room);
+    if (K > 0) {
+      TrackArgs tr{};
+      tr.step = (int32_t)step;
+      tr.act_on = act_on;
+      tr.probe_row = -1;
+      if (track) {
+        tr.act = track->act;
+        tr.act_thr = track->act_thr;
+        if (probes) {
+          tr.n_probe = track->n_probe;
+          tr.probe_idx = track->probe_idx;
+          tr.probe_var = track->probe_var;
+          tr.probe_buf = track->probe_buf;
+          tr.probe_row = track->probe_rows[pos];
+        }
+      }
+      const int32_t pairs = room / (2 * K);
+      const int rc = L(plan, a, b, st, tr, K, rows, pairs, s);
+      if (rc) return rc;
+      pos += 2 * K * pairs;
+      continue;
+    }
+    // to the end of the stimulus, or of the run when that is near
+    const int64_t to = stim_until(plan, step + 1, step0 + n_steps, stim_end);
+    int32_t n = (int32_t)(to - step);
+    if (room > 0 && n < room + 1) n = room + 1;
+    if (n > n_steps - pos) n = n_steps - pos;
+    fw_track_desc sub{};
+    if (track) {
+      sub = *track;
+      if (track->act_flags) sub.act_flags = track->act_flags + pos;
+      if (track->probe_rows) sub.probe_rows = track->probe_rows + pos;
+    }
+    const int rc = singles(a, b, step, n, track ? &sub : nullptr);
+    if (rc) return rc;
+    pos += n;
+    if (n % 2) {
+      void* t = a;
+      a = b;
+      b = t;
+    }
+  }
+  return FW_OK;
+}
+
 int fw_run(fw_plan* plan, void* u, void* u_new, void* const* state, int64_t step0,
            int32_t n_steps, const fw_track_desc* track, void* stream) {
   int rc = check_run_args(plan, u, u_new, state, n_steps, track);
   if (rc) return rc;
+  bool done = false;
+  rc = run_multi(plan, u, u_new, state, step0, n_steps, track, as_stream(stream),
+                 [&](void* a, void* b, int64_t step, int32_t n, const fw_track_desc* t) {
+                   return run_plain(plan, a, b, state, step, n, t, stream);
+                 },
+                 &done);
+  if (rc || done) return rc;
   return run_plain(plan, u, u_new, state, step0, n_steps, track, stream);
 }
 
@@ -804,12 +1029,9 @@ static int capture_pairs(fw_plan* plan, void* u, void* u_new, const StatePtrs& s
   return FW_OK;
 }
 
-// The graph set fw_run_graph replays for these buffers, tracker and schedule
-// (the plan's schedule is in every captured kernel's arguments; changing it
-// drops the graphs), with the graphs an n_steps run needs captured.
-static int ensure_graphs(fw_plan* plan, void* u, void* u_new, void* const* state,
-                         int32_t n_steps, const fw_track_desc* track, int32_t* act_on_out,
-                         fw_plan::GraphSet** set_out) {
+// fw_run_graph's arguments, and whether the run records activation times
+static int check_graph_args(fw_plan* plan, void* u, void* u_new, void* const* state,
+                            int32_t n_steps, const fw_track_desc* track, int32_t* act_on_out) {
   int rc = check_run_args(plan, u, u_new, state, n_steps, track);
   if (rc) return rc;
   if (track && track->n_probe > 0) {
@@ -817,9 +1039,7 @@ static int ensure_graphs(fw_plan* plan, void* u, void* u_new, void* const* state
     return FW_E_UNSUPPORTED;
   }
   int32_t act_on = 0;
-  int32_t* act = nullptr;
   if (track && track->act) {
-    act = track->act;
     act_on = track->act_flags ? track->act_flags[0] : 1;
     if (track->act_flags)
       for (int32_t s = 1; s < n_steps; ++s)
@@ -828,6 +1048,20 @@ static int ensure_graphs(fw_plan* plan, void* u, void* u_new, void* const* state
           return FW_E_UNSUPPORTED;
         }
   }
+  *act_on_out = act_on;
+  return FW_OK;
+}
+
+// The graph set fw_run_graph replays for these buffers, tracker and schedule
+// (the plan's schedule is in every captured kernel's arguments; changing it
+// drops the graphs), with the graphs an n_steps run needs captured.
+static int ensure_graphs(fw_plan* plan, void* u, void* u_new, void* const* state,
+                         int32_t n_steps, const fw_track_desc* track, int32_t* act_on_out,
+                         fw_plan::GraphSet** set_out) {
+  int32_t act_on = 0;
+  int rc = check_graph_args(plan, u, u_new, state, n_steps, track, &act_on);
+  if (rc) return rc;
+  int32_t* act = track ? track->act : nullptr;
   *act_on_out = act_on;
   const double act_thr = track ? track->act_thr : 0.0;
   const int ns = model_n_state(plan->desc.model);
@@ -876,11 +1110,16 @@ int fw_run_graph_prepare(fw_plan* plan, void* u, void* u_new, void* const* state
                          int32_t n_steps, const fw_track_desc* track) {
   int32_t act_on = 0;
   fw_plan::GraphSet* gs = nullptr;
+  // multi-step plans replay graphs only across long stimuli
+  if (plan && plan->alt && plan->n_stims == 0)
+    return check_graph_args(plan, u, u_new, state, n_steps, track, &act_on);
   return ensure_graphs(plan, u, u_new, state, n_steps, track, &act_on, &gs);
 }
 
-int fw_run_graph(fw_plan* plan, void* u, void* u_new, void* const* state, int64_t step0,
-                 int32_t n_steps, const fw_track_desc* track, void* stream) {
+// n_steps single steps: pairs of steps replayed from graphs, an odd last one
+// as a plain launch
+static int run_graphs(fw_plan* plan, void* u, void* u_new, void* const* state, int64_t step0,
+                      int32_t n_steps, const fw_track_desc* track, void* stream) {
   int32_t act_on = 0;
   fw_plan::GraphSet* gs = nullptr;
   int rc = ensure_graphs(plan, u, u_new, state, n_steps, track, &act_on, &gs);
@@ -913,9 +1152,26 @@ int fw_run_graph(fw_plan* plan, void* u, void* u_new, void* const* state, int64_
       one = *track;
       one.act_flags = &flag;
     }
-    return fw_run(plan, u, u_new, state, step0 + 2 * pairs, 1, track ? &one : nullptr, stream);
+    return run_plain(plan, u, u_new, state, step0 + 2 * pairs, 1, track ? &one : nullptr, stream);
   }
   return FW_OK;
+}
+
+int fw_run_graph(fw_plan* plan, void* u, void* u_new, void* const* state, int64_t step0,
+                 int32_t n_steps, const fw_track_desc* track, void* stream) {
+  int32_t act_on = 0;
+  int rc = check_graph_args(plan, u, u_new, state, n_steps, track, &act_on);
+  if (rc) return rc;
+  bool done = false;
+  rc = run_multi(plan, u, u_new, state, step0, n_steps, track, as_stream(stream),
+                 [&](void* a, void* b, int64_t step, int32_t n, const fw_track_desc* t) {
+                   return n >= kMultiGraphSteps
+                              ? run_graphs(plan, a, b, state, step, n, t, stream)
+                              : run_plain(plan, a, b, state, step, n, t, stream);
+                 },
+                 &done);
+  if (rc || done) return rc;
+  return run_graphs(plan, u, u_new, state, step0, n_steps, track, stream);
 }
 
 int fw_stim_apply(fw_plan* plan, void* u, const fw_stim_desc* stim, void* stream) {

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "../../include/finitewave_amd.h"
 #include "fw_models.hpp"
 
@@ -43,6 +45,11 @@ struct fw_plan {
   int32_t field_layout;
   double* ktab[FW_MAX_FIELDS];
   float* fktab[FW_MAX_FIELDS];
+  // the second state set of the multi-step launches (fw_multi2d.hpp), in the
+  // allocation of step_words; null for plans without them.  It belongs to the
+  // first stream that uses it (fw_abi.hip, multi_stream_ok)
+  void* alt;
+  std::atomic<uintptr_t> alt_stream;  // that stream's handle + 1; 0 while none
 };
 
 namespace fw {
@@ -76,6 +83,12 @@ typedef int (*StepLauncher)(const fw_plan* plan, const void* u, void* u_new,
 
 // one launcher per (precision, model), defined in fw_step_inst.hip builds
 StepLauncher step_launcher(int precision, int model);
+
+// multi-step launches of the light 2D models (fw_multi2d.hpp)
+typedef int (*MultiLauncher)(const fw_plan* plan, void* u, void* u_new, const StatePtrs& st,
+                             const TrackArgs& tr, int32_t K, int32_t rows, int32_t pairs,
+                             hipStream_t stream);
+MultiLauncher multi_launcher(int precision, int model);
 
 typedef int (*EcgLauncher)(const fw_plan* plan, const void* u, const double* coords,
                            int32_t n_points, double dr, double* out, hipStream_t stream);

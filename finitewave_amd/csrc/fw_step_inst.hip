@@ -7,6 +7,9 @@
 #include "fw_internal.hpp"
 #include "fw_kernels.hpp"
 #include "fw_march3d.hpp"
+#if FW_MODEL <= 4
+#include "fw_multi2d.hpp"
+#endif
 
 #ifndef FW_PREC
 #error "FW_PREC must be defined"
@@ -202,6 +205,64 @@ int FW_LAUNCHER(const fw_plan* plan, const void* u, void* u_new,
     return FW_E_HIP;
   }
   return FW_OK;
+}
+
+#define FW_MULTI_LAUNCHER FW_CAT4(fw_multi_launch_p, FW_PREC, _m, FW_MODEL)
+
+// `pairs` pairs of K-step launches (fw_multi2d.hpp) from step tr.step on; the
+// current potential is in u before and after, u_new then holds that of K
+// steps earlier
+int FW_MULTI_LAUNCHER(const fw_plan* plan, void* u, void* u_new, const StatePtrs& st,
+                      const TrackArgs& tr, int32_t K, int32_t rows, int32_t pairs,
+                      hipStream_t s) {
+#if FW_MODEL <= 4
+  constexpr int NS = model_n_state(FW_MODEL);
+  const fw_plan_desc& d = plan->desc;
+  KArgs<Real, UReal> a;
+  fill_args(plan, u, u_new, st, tr, a);
+  MultiArgs<Real> g;
+  g.K = K;
+  g.rows = rows;
+  g.own_w = kMultiW - 2 * K;
+  g.own_h = rows - 2 * K;
+  g.ni = (int32_t)a.ni;
+  g.nj = (int32_t)a.nj;
+  g.tiles_j = (g.nj + g.own_w - 1) / g.own_w;
+  g.step = tr.step;
+  g.probe_row = a.probe_row;
+  Real* const buf[2] = {static_cast<Real*>(u), static_cast<Real*>(u_new)};
+  Real* alt[3] = {};
+  for (int k = 0; k < NS; ++k) alt[k] = static_cast<Real*>(plan->alt) + k * plan->N;
+  g.even = buf[0];  // K is even: every launch starts at the parity of u
+  g.odd = buf[1];
+  const dim3 grid((unsigned)(g.tiles_j * ((g.ni + g.own_h - 1) / g.own_h))), blk(kMultiW * rows);
+  for (int32_t p = 0; p < 2 * pairs; ++p) {
+    const int ph = p & 1;
+    g.cur = buf[ph];
+    g.out = buf[1 - ph];
+    for (int k = 0; k < NS; ++k) {
+      Real* const own = static_cast<Real*>(st.p[k]);
+      g.sin[k] = ph ? alt[k] : own;
+      g.sout[k] = ph ? own : alt[k];
+    }
+    if (d.stencil == FW_STENCIL_ISO)
+      hipLaunchKernelGGL((k_multi2d<0, FW_MODEL, Real>), grid, blk, 0, s, a, g);
+    else
+      hipLaunchKernelGGL((k_multi2d<1, FW_MODEL, Real>), grid, blk, 0, s, a, g);
+    g.step += K;
+    if (g.probe_row >= 0) g.probe_row += K;
+  }
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    set_error("multi-step launch failed: %s", hipGetErrorString(e));
+    return FW_E_HIP;
+  }
+  return FW_OK;
+#else
+  (void)plan, (void)u, (void)u_new, (void)st, (void)tr, (void)K, (void)rows, (void)pairs, (void)s;
+  set_error("multi-step launch: model %d has none", FW_MODEL);
+  return FW_E_UNSUPPORTED;
+#endif
 }
 
 #define FW_ECG_LAUNCHER FW_CAT4(fw_ecg_launch_p, FW_PREC, _m, FW_MODEL)

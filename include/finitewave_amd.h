@@ -7,7 +7,8 @@
  * parameter block; for an FP32 plan whose potential is float, float copies
  * of its tabulated half-step fields; for a 3D plan whose fields are uniform
  * or tables along the last axis, each field as such a table in double and
- * float -- all read once at creation),
+ * float -- all read once at creation; for a 2D plan of a light model with
+ * uniform fields, a second set of state arrays),
  * fw_batch_create (the tissue descriptor table) and fw_batch_set_active (the
  * block table, when it grows).  `stream` is a
  * hipStream_t passed as void* (NULL = the default stream).  All launches are
@@ -227,7 +228,10 @@ int fw_plan_set_weights_k(fw_plan* plan, int32_t K);
 
 /* n_steps fused steps starting at global step `step0`: step s reads `u`,
  * writes `u_new`, then the two swap; after an odd n_steps the result is in
- * the buffer passed as u_new.  state: host array of device pointers. */
+ * the buffer passed as u_new.  state: host array of device pointers.
+ * Plans with a second state set take several steps per launch where that is
+ * faster (the same bits); the set serves the first stream that uses it, runs
+ * of the plan on other streams keep to one step per launch. */
 int fw_run(fw_plan* plan, void* u, void* u_new, void* const* state,
            int64_t step0, int32_t n_steps, const fw_track_desc* track,
            void* stream);
