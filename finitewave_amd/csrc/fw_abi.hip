@@ -76,6 +76,12 @@ EcgLauncher ecg_launcher(int precision, int model) {
   return table[precision][model];
 }
 
+static void put_recip(double* to, double b) {
+  const Recip y = recip(b);
+  to[0] = y.hi;
+  to[1] = y.lo;
+}
+
 static void derive_tp06(Params& P) {
   // TP06 parameter order (tp06_2d.py:1073 call)
   const double ko = P.v[0], cao = P.v[1], nao = P.v[2], Vc = P.v[3], Vsr = P.v[4],
@@ -85,8 +91,7 @@ static void derive_tp06(Params& P) {
   d[kInvVcF] = 1.0 / (Vc * F);
   d[kInvVssF2] = 1.0 / (2 * Vss * F);
   d[kFFoverRT] = F * F / (R * T);
-  d[kRT] = R * T;
-  d[kInvRT] = 1.0 / (R * T);
+  put_recip(d + kInvRT, R * T);
   d[kInvNaCaK] = 1.0 / (KmNai * KmNai * KmNai + nao * nao * nao);
   d[kInvKmCaCao] = 1.0 / (KmCa + cao);
   d[kKoOverKoKmK] = ko / (ko + KmK);
@@ -111,20 +116,17 @@ static void derive_crn(Params& P) {
                kmnancx = P.v[24], kmcancx = P.v[25];
   P.v[kCrnRTF] = R * T / F;
   P.v[kCrnRT2F] = R * T / (2.0 * F);
-  P.v[kCrnRT] = R * T;
-  P.v[kCrnInvRT] = 1.0 / (R * T);
+  put_recip(P.v + kCrnInvRT, R * T);
   P.v[kCrnSig] = 1 / 7.0 * (t128_exp(nao / 67.3) - 1.0);
   P.v[kCrnKo] = ko / (ko + kmko);
   P.v[kCrnNao3] = nao * (nao * nao);
   P.v[kCrnT12] = (kmnancx * (kmnancx * kmnancx) + P.v[kCrnNao3]) * (kmcancx + cao);
   P.v[kCrnFnF] = 5 * 1e-13 / F;
-  P.v[kCrnInvCaup] = 1.0 / caupmax;
   P.v[kCrnVrelVup] = Vrel / Vup;
-  P.v[kCrnFVj] = F * Vj;
-  P.v[kCrnInvFVj] = 1.0 / (F * Vj);
-  P.v[kCrn2FVj] = 2.0 * F * Vj;
-  P.v[kCrnInv2FVj] = 1.0 / (2.0 * F * Vj);
-  P.v[kCrnInvVj] = 1.0 / Vj;
+  put_recip(P.v + kCrnInvCaup, caupmax);
+  put_recip(P.v + kCrnInvFVj, F * Vj);
+  put_recip(P.v + kCrnInv2FVj, 2.0 * F * Vj);
+  put_recip(P.v + kCrnInvVj, Vj);
 }
 
 void complete_params(int model, Params& P) {
@@ -134,8 +136,8 @@ void complete_params(int model, Params& P) {
     P.v[6] = 1.0 / P.v[0];
   }
   if (model == 3) {
-    for (int q = 0; q < 8; ++q) P.v[kFkInv + q] = 1.0 / P.v[q];
-    P.v[kFkInv + 8] = 1.0 / (2.0 * P.v[3]);
+    for (int q = 0; q < 8; ++q) put_recip(P.v + kFkInv + 2 * q, P.v[q]);
+    put_recip(P.v + kFkInv + 16, 2.0 * P.v[3]);
   }
   if (model == 5) derive_lr91(P);
   if (model == 6) derive_tp06(P);

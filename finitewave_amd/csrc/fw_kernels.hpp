@@ -288,12 +288,12 @@ __host__ __device__ __forceinline__ void minor_exact(double d, const MinorQ* T, 
     return;
   }
   // mh and ml are 3 or 4: d / 4 is exact as d * 0.25 and d / 3 the correctly
-  // rounded quotient from RN(1/3), once for both sides (a negative d only
+  // rounded quotient (div_recip), once for both sides (a negative d only
   // changes its sign); m2 = m3 = 1 makes the middle pair's factor one of
   // three constants.  The same bits as dividing (the reference's four
   // quotients) in a quarter of the operations: Aliev-Panfilov 131 x 115 x 147
   // FP64 with per-node fibres 127 -> 106 us per step.
-  const double d4 = d * 0.25, d3 = div_rn(d, 3.0, 1.0 / 3.0);
+  const double d4 = d * 0.25, d3 = div_recip(d, recip(3.0));
   const double nq = -(ml == 4 ? d4 : d3), pq = mh == 4 ? d4 : d3;
   const double dc = d * (mh == ml ? 0.0 : (mh == 4 ? 0.25 - 1.0 / 3.0 : 1.0 / 3.0 - 0.25));
   q[0] = m0 ? nq : 0.0;

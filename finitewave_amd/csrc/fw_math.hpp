@@ -152,6 +152,26 @@ FW_HD inline double dd_log(double x) {
   return s2 + tail;
 }
 
+// 1/b as an unevaluated sum: hi = RN(1/b) and lo = RN(1/b - hi), from the exact
+// remainder 1 - b hi.
+struct Recip {
+  double hi, lo;
+};
+
+FW_HD inline Recip recip(double b) {
+  const double hi = 1.0 / b;
+  return Recip{hi, __builtin_fma(-b, hi, 1.0) / b};
+}
+
+// a / b from b's reciprocal pair, in two operations: a lo is rounded at 2^-53 of
+// a term 2^-53 of the quotient, so the fused sum is within 2^-105 of a/b before
+// its one rounding (Brisebarre and Muller, IEEE Trans. Computers 53(8), 2004).
+// The result is RN(a/b) unless a/b lies that close to a rounding boundary,
+// which no quotient by a divisor of up to 50 significant bits does: a boundary
+// is then at least 2^-104 away.  Holds while a lo does not underflow; a zero
+// quotient may come out with the other sign.
+FW_HD inline double div_recip(double a, Recip y) { return fma(a, y.hi, a * y.lo); }
+
 // x^1.5 as x sqrt(x), with the root's remainder r = x - s s (sqrt(x) = s +
 // r / 2s, so x sqrt(x) = x s + s r / 2 to second order) and the product's
 // rounding error folded back in: within 0.5001 ulp of the exact value, for a

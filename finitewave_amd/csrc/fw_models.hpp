@@ -88,41 +88,32 @@ __device__ __forceinline__ float exprel(float y) {
   return fabsf(y) < 1e-4f ? 1.0f + 0.5f * y : expm1f(y) / y;
 }
 
-// a / b for a literal b.  FP64 path: the correctly rounded quotient in five
-// operations instead of a full division, from y = 1/b correctly rounded
-// (folded at compile time): q0 = a y is within 1.5 ulp of a/b, one
-// correction q1 = q0 + (a - b q0) y is faithful, and a second gives RN(a/b)
-// by Markstein's theorem (y within half an ulp of 1/b, q1 within one ulp of
-// a/b; the remainder a - b q1 is exact).  Holds while a/b is a normal number
-// or zero (a zero quotient comes out +0).  FP32 path: the plain division.
-template <typename R>
-__host__ __device__ __forceinline__ R div_rn(R a, R b, R y) {  // y = 1/b correctly rounded
-  const R q0 = a * y;
-  const R q1 = fma(fma(-b, q0, a), y, q0);
-  return fma(fma(-b, q1, a), y, q1);
-}
-
+// a / b for a literal b.  FP64: div_recip with the pair folded at compile
+// time, two operations instead of a division's eleven.  FP32: the plain
+// division.
 template <typename R>
 __device__ __forceinline__ R divc(R a, R b) {
-  if constexpr (sizeof(R) == 8) return div_rn(a, b, R(1) / b);
+  if constexpr (sizeof(R) == 8) return div_recip(a, recip(b));
   else return a / b;
 }
 
-// a / b for a node-dependent b.  FP64: the core of the IEEE division
-// sequence, without its operand scaling (two v_div_scale), its scaled
-// correction and its special-case fix-up: r = 1/b from the hardware estimate
-// refined by two Newton steps, q = a r, then q + (a - b q) r.  These are the
-// operations and roundings of the full sequence, so the quotient is the same
-// bits wherever the full sequence would not rescale: a, b, 1/b and a/b normal
-// and their exponents less than 768 apart (the models' rates, gates,
+// a / b for a node-dependent b.  FP64: r = 1/b from the hardware estimate and
+// one Newton step, q = a r, then q + (a - b q) r: six operations, without the
+// compiler's second Newton step, operand scaling (two v_div_scale), scaled
+// correction and special-case fix-up.  The estimate is within 2^-24.3
+// (measured), so r is within 2^-48.6 and the value before the last rounding
+// within 2^-97 of a/b: the quotient is RN(a/b) unless a/b lies that close to a
+// rounding boundary (no difference from the full sequence in 8.4e10 random
+// quotients), wherever the full sequence would not rescale: a, b, 1/b and a/b
+// normal and their exponents less than 768 apart (the models' rates, gates,
 // concentrations and time constants stay far inside that while the state is
 // finite).  It differs for b infinite (NaN instead of 0) and for a = -0
-// (+0).  FP32: the plain division.
+// (+0).  The TP06 update divides 76 times: with this and div_recip 1026^2 went
+// from 101.8 to 94.6 us per step.  FP32: the plain division.
 template <typename R>
 __device__ __forceinline__ R dv(R a, R b) {
   if constexpr (sizeof(R) == 8) {
     double r = __builtin_amdgcn_rcp(b);
-    r = fma(fma(-b, r, 1.0), r, r);
     r = fma(fma(-b, r, 1.0), r, r);
     const double q = a * r;
     return fma(fma(-b, q, a), r, q);
@@ -134,29 +125,37 @@ __device__ __forceinline__ R dv(R a, R b) {
 // FP64 path: quantities of the parameters alone, appended after a model's
 // parameters by complete_params on the host in the operation order of the
 // expressions they replace, so the values are those a node would compute (the
-// float update keeps forming its own per node).  1 / tau values serve div_rn.
-constexpr int kFkInv = 11;  // Fenton-Karma: 1 / parameters 0..7, then 1 / (2 tau_si)
+// float update keeps forming its own per node).  A divisor's reciprocal pair
+// (div_recip) takes two entries, hi then lo.
+constexpr int kFkInv = 11;  // Fenton-Karma: the pairs of parameters 0..7, then of 2 tau_si
 enum Lr91Derived { kLrENa = 15, kLrEK, kLrGK, kLrEK1, kLrGK1 };
 enum CrnDerived {
   kCrnRTF = 39,   // R * T / F
   kCrnRT2F,       // R * T / (2 * F)
-  kCrnRT,         // R * T
-  kCrnInvRT,
+  kCrnInvRT,      // pair of R * T
+  kCrnInvRTLo,
   kCrnSig,        // (exp(nao / 67.3) - 1) / 7
   kCrnKo,         // ko / (ko + kmko)
   kCrnNao3,       // nao * (nao * nao)
   kCrnT12,        // (kmnancx^3 + nao^3) * (kmcancx + cao)
   kCrnFnF,        // 5e-13 / F
-  kCrnInvCaup,    // 1 / caupmax
   kCrnVrelVup,    // Vrel / Vup
-  kCrnFVj,        // F * Vj
+  kCrnInvCaup,    // pairs of caupmax, F * Vj, 2 * F * Vj, Vj
+  kCrnInvCaupLo,
   kCrnInvFVj,
-  kCrn2FVj,       // 2 * F * Vj
+  kCrnInvFVjLo,
   kCrnInv2FVj,
+  kCrnInv2FVjLo,
   kCrnInvVj,
+  kCrnInvVjLo,
   kCrnNDerivedEnd
 };
 static_assert(kCrnNDerivedEnd <= 64, "parameter block size");
+
+// the reciprocal pair at derived parameter q
+__device__ __forceinline__ Recip par_recip(const Params& P, int q) {
+  return Recip{P.v[q], P.v[q + 1]};
+}
 
 // TP06 quantities that are the same for every node (functions of the
 // parameters only), appended after its 49 parameters by complete_params on the
@@ -169,8 +168,8 @@ enum Tp06Derived {
   kInvVcF,      // 1.0 / (Vc * F)
   kInvVssF2,    // 1.0 / (2 * Vss * F)
   kFFoverRT,    // F * F / (R * T)
-  kRT,          // R * T
-  kInvRT,       // 1.0 / (R * T)
+  kInvRT,       // reciprocal pair of R * T
+  kInvRTLo,
   kInvNaCaK,    // 1.0 / (KmNai * KmNai * KmNai + nao * nao * nao)
   kInvKmCaCao,  // 1.0 / (KmCa + cao)
   kKoOverKoKmK, // ko / (ko + KmK)
@@ -333,7 +332,7 @@ __device__ __forceinline__ R ionic_fk(R u, R un, SP& S, int64_t c,
           u_c = par<R>(P, 9), uc_si = par<R>(P, 10);
   // x / tau, parameter q
   auto over = [&](R x, R tau, int q) -> R {
-    if constexpr (sizeof(R) == 8) return div_rn(x, tau, P.v[kFkInv + q]);
+    if constexpr (sizeof(R) == 8) return div_recip(x, par_recip(P, kFkInv + 2 * q));
     else return x / tau;
   };
   auto&& vref = ref<R>(S, 0, c);
@@ -406,7 +405,7 @@ __device__ __forceinline__ R ionic_bo(R u, R un, SP& S, int64_t c,
 
 // ---- Luo-Rudy 1991  luo_rudy91_2d.py:158-510 --------------------------------
 // FP64: bound by VALU issue and, on sheets of a wave or two per SIMD, by the
-// chain of dependent operations.  Divisions through dv / divc and the five
+// chain of dependent operations.  Divisions through dv and divc and the five
 // parameter-only logarithms and roots from the host: 291 x 259 iso 11.0 ->
 // 9.3 us per step, the same bits.
 template <typename R>
@@ -572,7 +571,7 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
   const D inversevssF2 = Dv[kInvVssF2];
   // x / (R T) for a node-dependent x
   auto overRT = [&](R x) -> R {
-    if constexpr (F64) return div_rn(x, par<R>(P, kTp06Derived + kRT), par<R>(P, kTp06Derived + kInvRT));
+    if constexpr (F64) return div_recip(x, par_recip(P, kTp06Derived + kInvRT));
     else return x / (R_ * T);
   };
 
@@ -815,7 +814,7 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
 // state order = the kernel's parameter order (courtemanche_2d.py:568-569):
 // nai ki cai caup carel m h j_ d f oa oi ua ui xs xr fca irel vrel urel wrel;
 // the model passes its xr array in the xs slot and vice versa.
-// FP64: bound by VALU issue.  Divisions through dv / divc / div_rn, the
+// FP64: bound by VALU issue.  Divisions through dv and div_recip, the
 // parameter-only quantities from the host and pow15 for the device pow:
 // 514 x 387, 10 % fibrosis, per-node fibres, 49.8 -> 37.6 us per step.
 template <typename R>
@@ -852,12 +851,12 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
   const R ena = rtf * flog(dv(nao, nai));
   const R ek = rtf * flog(dv(ko, ki));
   const R eca = rt2f * flog(dv(cao, cai));
-  // x / b for a uniform b whose reciprocal is derived parameter iq
+  // x / b for a uniform b whose reciprocal pair is derived parameter iq
   auto divu = [&](R x, R b, int iq) -> R {
-    if constexpr (F64) return div_rn(x, b, P.v[iq]);
+    if constexpr (F64) return div_recip(x, par_recip(P, iq));
     else return x / b;
   };
-  auto overRT = [&](R x) -> R { return divu(x, F64 ? par<R>(P, kCrnRT) : R_ * T, kCrnInvRT); };
+  auto overRT = [&](R x) -> R { return divu(x, R_ * T, kCrnInvRT); };
   // calc_gating_m / h / j
   R m, h, j;
   {
@@ -1071,9 +1070,7 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
     irel = krel * (urel * urel) * vrel * wrel * (carel - cai);
     irr = irel;
   }
-  auto overFVj = [&](R x) -> R {
-    return divu(x, F64 ? par<R>(P, kCrnFVj) : F * Vj, kCrnInvFVj);
-  };
+  auto overFVj = [&](R x) -> R { return divu(x, F * Vj, kCrnInvFVj); };
   const R vrel_vup = F64 ? par<R>(P, kCrnVrelVup) : Vrel / Vup;
   const R itr = divc(caup - carel, R(180));
   const R iup = dv(iupmax, R(1) + dv(kup, cai));
@@ -1083,7 +1080,7 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
   kir = ki + dt * overFVj(R(2) * inak - ik1 - ito - ikur - ikr - iks - ibk);
   {
     const R B1 = divu(R(2) * inaca - ipca - ical - ibca,
-                      F64 ? par<R>(P, kCrn2FVj) : R(2) * F * Vj, kCrnInv2FVj) +
+                      R(2) * F * Vj, kCrnInv2FVj) +
                  divu(Vup * (iupleak - iup) + irel * Vrel, Vj, kCrnInvVj);
     const R B2 = R(1) + dv(trpnmax * kmtrpn, (cai + kmtrpn) * (cai + kmtrpn)) +
                  dv(cmdnmax * kmcmdn, (cai + kmcmdn) * (cai + kmcmdn));
