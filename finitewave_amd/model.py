@@ -20,6 +20,12 @@ import numpy as np
 from . import _native
 
 _CHUNK = 4096  # steps per library call between host synchronisations
+# event-free steps in a row before the loop looks ahead for more of them, and
+# the steps it then looks at: a look costs some 60 us, a step taken by itself
+# 2.5 us, so runs with an event every few steps never pay for one (model.run()
+# of 1,000 event-free steps on 102 x 102 nodes: 3.04 -> 1.46 ms)
+_LOOK_AFTER = 32
+_LOOK_AHEAD = 1024
 
 
 def _gate_open(tracker, t, step) -> bool:
@@ -27,6 +33,11 @@ def _gate_open(tracker, t, step) -> bool:
     if tracker.start_time > t or t > tracker.end_time:
         return False
     return step % tracker.step == 0
+
+
+def _gates(tracker, t, steps):
+    """_gate_open at times t and step numbers steps (arrays)."""
+    return ~((tracker.start_time > t) | (t > tracker.end_time)) & (steps % tracker.step == 0)
 
 
 def _saver_due(saver, model) -> bool:
@@ -240,7 +251,10 @@ class CardiacModel:
             except Exception:  # pragma: no cover
                 bar = None
 
-        chunk_flags, chunk_rows, chunk_row_owners = [], [], []
+        # per step of the pending chunk: activation flag and probe row; per
+        # probe tracker: the rows its gate was open at
+        chunk_flags, chunk_rows = [], []
+        chunk_open = [[] for _ in probe_trackers]
         chunk_start = [self.step]
 
         def flush():
@@ -251,25 +265,58 @@ class CardiacModel:
             flags = np.array(chunk_flags, dtype=np.uint8) if fused_act is not None else None
             rows = np.array(chunk_rows, dtype=np.int32) if probes is not None else None
             eng.run_steps(s0, n, fused_act, flags, probes, rows, use_graph=self.use_graphs)
-            if probes is not None and any(r >= 0 for r in chunk_rows):
-                self._collect_probes(probes, probe_trackers, slices, chunk_row_owners)
+            if probes is not None:
+                self._collect_probes(probes, probe_trackers, slices, chunk_open)
             if bar is not None:
                 bar.update(n)
             chunk_flags.clear()
             chunk_rows.clear()
-            chunk_row_owners.clear()
 
         dt = self.dt
         # stimuli on the device schedule: their steps need no host event
         sched = self._schedule_stims(eng, stims, iters)
-        for _ in range(iters):
+        look = self._can_look_ahead(trackers)
+        done, calm = 0, 0
+        while done < iters:
+            if look and calm >= _LOOK_AFTER:
+                calm = 0
+                if len(chunk_flags) == 0:
+                    chunk_start[0] = self.step
+                ask = min(iters - done, _CHUNK - len(chunk_flags),
+                          _LOOK_AHEAD if len(chunk_flags) < _LOOK_AHEAD else _CHUNK)
+                ahead = self._look_ahead(ask, stims, commands, fused_act, probe_trackers,
+                                         extra_act + host_trackers + dev_trackers)
+                n = len(ahead[0])
+                if n:
+                    flags, gates, times, t_next = ahead
+                    base = len(chunk_flags)
+                    rows = np.full(n, -1)
+                    for k, g in enumerate(gates):
+                        at = np.flatnonzero(g)
+                        rows[at] = base + at
+                        chunk_open[k].extend((base + at).tolist())
+                    chunk_flags.extend(flags.tolist())
+                    chunk_rows.extend(rows.tolist())
+                    self._t_hist.extend(times)
+                    self.t = t_next
+                    self.step += n
+                    done += n
+                    if len(chunk_flags) >= _CHUNK:
+                        flush()
+                    if n == ask:
+                        calm = _LOOK_AFTER
+                    if self.check_termination():
+                        break
+                    continue
             t, step = self.t, self.step
+            done += 1
+            calm += 1
             if len(chunk_flags) == 0:
                 chunk_start[0] = step
             due_stims = [s for s in stims if t >= s.t and not s.passed]
             act_open = fused_act is not None and _gate_open(fused_act, t, step)
             extra_open = [tr for tr in extra_act if _gate_open(tr, t, step)]
-            probe_open = [tr for tr in probe_trackers if _gate_open(tr, t, step)]
+            probe_open = [k for k, tr in enumerate(probe_trackers) if _gate_open(tr, t, step)]
             host_open = [tr for tr in host_trackers if _gate_open(tr, t, step)]
             dev_open = [tr for tr in dev_trackers if _gate_open(tr, t, step)]
             t_next = t + dt
@@ -291,7 +338,8 @@ class CardiacModel:
                     s._host_advance(self)
                 chunk_flags.append(1 if act_open else 0)
                 chunk_rows.append(row)
-                chunk_row_owners.append(probe_open)
+                for k in probe_open:
+                    chunk_open[k].append(row)
                 self.t = t_next
                 self.step = step + 1
                 if len(chunk_flags) >= _CHUNK:
@@ -300,6 +348,7 @@ class CardiacModel:
                     break
                 continue
             # a step with host-side work
+            calm = 0
             flush()
             chunk_start[0] = step
             if sched:
@@ -315,21 +364,17 @@ class CardiacModel:
                 tr._device_track(self, eng)
             chunk_flags.append(1 if act_open else 0)
             chunk_rows.append(0 if probe_open else -1)
-            chunk_row_owners.append(probe_open)
+            for k in probe_open:
+                chunk_open[k].append(0)
+            # host trackers see the pre-step u and the post-ionic state
+            self._run_single(eng, chunk_flags, chunk_rows, chunk_open, fused_act, probes,
+                             probe_trackers, slices)
+            for tr in extra_open:
+                eng.act_update(tr, step)
             if host_open:
-                # host trackers see the pre-step u and the post-ionic state
-                self._run_single(eng, chunk_flags, chunk_rows, chunk_row_owners, fused_act,
-                                 probes, probe_trackers, slices, pre_swap_hook=True)
-                for tr in extra_open:
-                    eng.act_update(tr, step)
                 self._sync_pre_swap(eng)
                 for tr in host_open:
                     tr._track()
-            else:
-                self._run_single(eng, chunk_flags, chunk_rows, chunk_row_owners, fused_act,
-                                 probes, probe_trackers, slices)
-                for tr in extra_open:
-                    eng.act_update(tr, step)
             if bar is not None:
                 bar.update(1)
             self.t = t_next
@@ -355,6 +400,45 @@ class CardiacModel:
         if bar is not None:
             bar.close()
 
+    def _can_look_ahead(self, trackers) -> bool:
+        """Whether the loop may resolve event-free steps in bulk: the time
+        fold, gates and termination rule are the package's own."""
+        return (isinstance(self.dt, float) and not self.state_saver and
+                type(self).check_termination is CardiacModel.check_termination and
+                "check_termination" not in self.__dict__ and
+                all(type(tr.step) is int and tr.step > 0 for tr in trackers))
+
+    def _look_ahead(self, n, stims, commands, fused_act, probe_trackers, event_trackers):
+        """The event-free steps among the next n: (activation flags, a gate
+        per probe tracker, their times, the time after them).  They end
+        before the first step with a due stimulus, an open event tracker or a
+        due command, and with the step that terminates the run."""
+        if not isinstance(self.t, (int, float)):
+            return np.zeros(0), [], [], self.t
+        # the left fold t += dt (accumulate adds in order)
+        t = np.add.accumulate(np.concatenate(([self.t], np.full(n, self.dt))))
+        steps = np.arange(self.step, self.step + n)
+
+        def first(mask):
+            k = int(np.argmax(mask)) if len(mask) else 0
+            return k if len(mask) and mask[k] else len(mask)
+
+        stop = first((t[1:] > self.t_max) | (steps + 1 > int(np.ceil(self.t_max / self.dt)))) + 1
+        for s in stims:
+            if not s.passed:
+                stop = min(stop, first(t[:n] >= s.t))
+        for c in commands:
+            if not c.passed:
+                stop = min(stop, first(t[1:] >= c.t))
+        for tr in event_trackers:
+            stop = min(stop, first(_gates(tr, t[:n], steps)))
+        n = min(n, stop)
+        t, steps = t[:n + 1], steps[:n]
+        flags = (_gates(fused_act, t[:n], steps) if fused_act is not None
+                 else np.zeros(n)).astype(np.uint8)
+        times = t.tolist()
+        return flags, [_gates(tr, t[:n], steps) for tr in probe_trackers], times[:n], times[n]
+
     def _schedule_stims(self, eng, stims, iters) -> bool:
         """Puts the run's stimuli on the device schedule (fw_plan_set_stims):
         the steps each applies on, from the time fold, and its descriptor.
@@ -375,8 +459,7 @@ class CardiacModel:
         eng.set_stim_schedule(entries)
         return True
 
-    def _run_single(self, eng, flags, rows, owners, fused_act, probes, probe_trackers, slices,
-                    pre_swap_hook=False):
+    def _run_single(self, eng, flags, rows, opened, fused_act, probes, probe_trackers, slices):
         """One fused step from the current orientation without the swap
         bookkeeping (the caller swaps)."""
         s0 = self.step
@@ -384,11 +467,10 @@ class CardiacModel:
         r = np.array(rows, dtype=np.int32) if probes is not None else None
         eng.run_steps(s0, 1, fused_act, f, probes, r, use_graph=False, stim_first=False)
         eng.swapped = not eng.swapped  # run_steps swapped; undo, caller owns it
-        if probes is not None and rows[0] >= 0:
-            self._collect_probes(probes, probe_trackers, slices, owners)
+        if probes is not None:
+            self._collect_probes(probes, probe_trackers, slices, opened)
         flags.clear()
         rows.clear()
-        owners.clear()
 
     def _sync_pre_swap(self, eng) -> None:
         """Host view during a step: u = pre-step potential, state after the
@@ -408,13 +490,17 @@ class CardiacModel:
         eng.upload()
         self._engine = eng
 
-    def _collect_probes(self, probes, probe_trackers, slices, owners) -> None:
-        data = probes.buf[: len(owners)].cpu().numpy()
-        for r, open_trackers in enumerate(owners):
-            for tr in open_trackers:
-                k = probe_trackers.index(tr)
-                a, n = slices[k]
-                tr._append(data[r, a:a + n])
+    def _collect_probes(self, probes, probe_trackers, slices, opened) -> None:
+        """Hands each probe tracker the rows its gate was open at (opened[k],
+        cleared) of the chunk that has run."""
+        n = max((rows[-1] + 1 for rows in opened if rows), default=0)
+        if n == 0:
+            return
+        data = probes.buf[:n].cpu().numpy()
+        for tr, (a, m), rows in zip(probe_trackers, slices, opened):
+            if rows:
+                tr._extend(data[rows, a:a + m])
+                rows.clear()
 
     def _finish_trackers(self, eng) -> None:
         from .tracker import _DeviceTracker

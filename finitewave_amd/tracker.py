@@ -138,6 +138,11 @@ class _ProbeTracker(Tracker):
     def _append(self, values: np.ndarray) -> None:
         raise NotImplementedError
 
+    def _extend(self, rows: np.ndarray) -> None:
+        """_append of each row, one per tracked step."""
+        for values in rows:
+            self._append(values)
+
     @staticmethod
     def _flat_cells(model, cell_ind) -> np.ndarray:
         cells = np.atleast_2d(np.asarray(cell_ind))
@@ -169,6 +174,12 @@ class ActionPotential2DTracker(_ProbeTracker):
 
     def _append(self, values):
         self.act_pot.append(np.array(values))
+
+    def _extend(self, rows):
+        if type(self)._append is ActionPotential2DTracker._append:
+            self.act_pot.extend(np.array(rows))
+        else:
+            super()._extend(rows)
 
     def _track(self):
         cell_ind = tuple(np.atleast_2d(self.cell_ind).T)
