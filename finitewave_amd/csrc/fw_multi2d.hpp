@@ -122,7 +122,7 @@ __global__ __launch_bounds__(kMultiThreads) void k_multi2d(const KArgs<R, R> a,
 #pragma unroll
         for (int k = 0; k < 9; ++k) M.m[3 * k + 1] = q.m[k];
         const double xx = a.f[0].value, xy = a.f[1].value, yx = a.f[2].value, yy = a.f[3].value;
-        wts_aniso2d(W, M, xx, xx, xy, xy, yx, yx, yy, yy, &a.mq[1], &a.mq[2]);
+        wts_aniso2d(W, M, xx, xx, xy, xy, yx, yx, yy, yy);
         scale_exact<9>(W, 4, a.D, a.dtd, a.dr2, a.inv_dr2);
       }
     }
