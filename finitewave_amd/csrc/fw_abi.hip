@@ -1363,7 +1363,6 @@ static BatchLaunch batch_args(const fw_batch* b, int32_t step, const int32_t* in
   L.D = b->D;
   L.dt = b->dt;
   L.dr2 = b->dr2;
-  L.inv_dr2 = b->inv_dr2;
   L.P = b->P;
   return L;
 }
@@ -1491,9 +1490,6 @@ int fw_batch_create(int32_t model, int32_t precision, double D_model, double dt,
   b->D = D_model;
   b->dt = dt;
   b->dr2 = dr2;
-  int e2;
-  const double mant = frexp(dr2, &e2);
-  b->inv_dr2 = (mant == 0.5 && e2 > -1000 && e2 < 1000) ? ldexp(1.0, 1 - e2) : 0.0;
   for (int q = 0; q < FW_MAX_PARAMS; ++q) b->P.v[q] = q < n_params ? params[q] : 0.0;
   complete_params(model, b->P);
   b->host = new (std::nothrow) fw_tissue_desc[max_tissues]();

@@ -84,7 +84,8 @@ struct BatchArgs {
   const int32_t* step_in;
   int32_t* step_out;
   int32_t step;
-  double D, dtd, dr2, inv_dr2;
+  double D, dtd;
+  Recip rdr2;  // 1 / dr**2
   R dt;
   U s;  // D * dt / dr**2 in the potential's type
   Params P;
@@ -102,8 +103,8 @@ using Nb9 = Hood2<R>;
 // kernel's operands)
 template <typename R, bool EXACT>
 __device__ __forceinline__ R diffuse9(int stencil, const double* dd, const float* df,
-                                      const Nb9<R>& q, double D, double dtd, double dr2,
-                                      double inv_dr2, R s) {
+                                      const Nb9<R>& q, double D, double dtd, Recip rdr2,
+                                      R s) {
   const R uc = q.v[4];
   if (stencil == FW_STENCIL_ISO) {
     const int mN = q.m[1], mS = q.m[7], mW = q.m[3], mE = q.m[5];
@@ -114,7 +115,7 @@ __device__ __forceinline__ R diffuse9(int stencil, const double* dd, const float
       W[3] = iso_comp(dd[1], mE, mW);
       W[4] = iso_comp(dd[0], mS, mN);
       W[2] = -(W[0] + W[1] + W[3] + W[4]);
-      scale_exact<5>(W, 2, D, dtd, dr2, inv_dr2);
+      scale_exact<5>(W, 2, D, dtd, rdr2);
       return q.v[1] * W[0] + q.v[3] * W[1] + uc * W[2] + q.v[5] * W[3] + q.v[7] * W[4];
     } else {
       const R dx = sizeof(R) == 8 ? (R)dd[0] : (R)df[0];
@@ -133,7 +134,7 @@ __device__ __forceinline__ R diffuse9(int stencil, const double* dd, const float
     const double dxx = dd[0], dxy = dd[1], dyx = dd[2], dyy = dd[3];
     double W[9];
     wts_aniso2d(W, M, dxx, dxx, dxy, dxy, dyx, dyx, dyy, dyy);
-    scale_exact<9>(W, 4, D, dtd, dr2, inv_dr2);
+    scale_exact<9>(W, 4, D, dtd, rdr2);
     return q.v[0] * W[0] + q.v[1] * W[1] + q.v[2] * W[2] + q.v[3] * W[3] + uc * W[4] +
            q.v[5] * W[5] + q.v[6] * W[6] + q.v[7] * W[7] + q.v[8] * W[8];
   } else {
@@ -290,7 +291,7 @@ __global__ __launch_bounds__(kBlock, (batch_min_waves<MODEL, R>())) void k_batch
         q.m[k] = need ? (code[c + di * nj + dj] & 1) : 0;
       }
     const U val = node_update<MODEL, R>(uc, S, (int64_t)c, a.dt, a.P, [&] {
-      return diffuse9<U, EXACT>(stencil, dd, df, q, a.D, a.dtd, a.dr2, a.inv_dr2, a.s);
+      return diffuse9<U, EXACT>(stencil, dd, df, q, a.D, a.dtd, a.rdr2, a.s);
     });
     st_state<NT>(un + c, val);
   } else {
@@ -355,7 +356,7 @@ __global__ __launch_bounds__(kBlock, (batch_min_waves<MODEL, R>())) void k_batch
 #pragma unroll
         for (int s = 0; s < NS; ++s) rs.v[s] = st[s][k];
         const R val = node_update<MODEL, R>(uc, rs, 0, a.dt, a.P, [&] {
-          return diffuse9<R, EXACT>(stencil, dd, df, q, a.D, a.dtd, a.dr2, a.inv_dr2, a.s);
+          return diffuse9<R, EXACT>(stencil, dd, df, q, a.D, a.dtd, a.rdr2, a.s);
         });
         out[k] = upd ? val : uc;
 #pragma unroll
@@ -390,7 +391,7 @@ __global__ __launch_bounds__(kBlock, (batch_min_waves<MODEL, R>())) void k_batch
 #pragma unroll
       for (int s = 0; s < NS; ++s) rs.v[s] = ld_state<NT>((const global_t<R>*)S.p[s] + cc);
       const R val = node_update<MODEL, R>(uc, rs, 0, a.dt, a.P, [&] {
-        return diffuse9<R, EXACT>(stencil, dd, df, q, a.D, a.dtd, a.dr2, a.inv_dr2, a.s);
+        return diffuse9<R, EXACT>(stencil, dd, df, q, a.D, a.dtd, a.rdr2, a.s);
       });
       st_state<NT>(un + cc, val);
 #pragma unroll

@@ -37,8 +37,7 @@ static BatchArgs<BReal, UReal> kernel_args(const BatchLaunch& L) {
   a.step = L.step;
   a.D = L.D;
   a.dtd = L.dt;
-  a.dr2 = L.dr2;
-  a.inv_dr2 = L.inv_dr2;
+  a.rdr2 = recip(L.dr2);
   a.dt = (BReal)L.dt;
   a.s = (UReal)(L.D * L.dt / L.dr2);
   a.P = L.P;

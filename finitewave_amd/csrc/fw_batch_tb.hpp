@@ -242,7 +242,7 @@ __device__ __forceinline__ void tb_march(const BatchArgs<R, R>& a, const BatchTi
         q.m[7] = pS & 1;
         q.m[8] = (pS >> 16) & 1;
         val = node_update<MODEL, R>(uc, s1, 0, a.dt, a.P, [&] {
-          return diffuse9<R, EXACT>(stencil, dd, df, q, a.D, a.dtd, a.dr2, a.inv_dr2, a.s);
+          return diffuse9<R, EXACT>(stencil, dd, df, q, a.D, a.dtd, a.rdr2, a.s);
         });
       }
       const bool upd = (pC & 3) == 1;

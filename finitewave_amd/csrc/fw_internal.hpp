@@ -134,7 +134,7 @@ struct BatchLaunch {
   int32_t* step_out;
   int32_t step;
   int32_t variant;  // launch shape (fw_batch.hpp: kBatchVec | kBatchXcd | kBatchNT | kBatchList)
-  double D, dt, dr2, inv_dr2;
+  double D, dt, dr2;
   Params P;
 };
 
@@ -151,7 +151,7 @@ BatchTbLauncher batch_tb_launcher(int precision, int model);
 
 struct fw_batch {
   int32_t model, precision, max_tissues;
-  double D, dt, dr2, inv_dr2;
+  double D, dt, dr2;
   fw::Params P;
   void* table;            // device fw::BatchTissue[max_tissues]
   int32_t* btis;          // device block table

@@ -20,6 +20,7 @@
 // hit that XCD's own L2).
 #pragma once
 
+#include <type_traits>
 #include <utility>
 
 #include <hip/hip_runtime.h>
@@ -143,7 +144,8 @@ struct KArgs {
   uint32_t per_xcd;  // logical blocks per XCD
   Field f[9];
   const double* __restrict__ w;  // precomputed weights (stencil 2)
-  double D, dtd, dr2, inv_dr2;  // inv_dr2: exact 1/dr2 when dr2 = 2^k, else 0
+  double D, dtd;
+  Recip rdr2;  // 1 / dr**2
   R dt;
   U s;  // D * dt / dr**2 in the potential's type
   Params P;
@@ -250,50 +252,47 @@ __host__ __device__ __forceinline__ double iso_comp(double d, int m0, int m1) {
   return d * (double)m0 * (double)(m0 + (m1 == 0));
 }
 
-// asymmetric_stencil_2d.py:204-259 for 0/1 mesh values: zeros unless the two
-// face nodes conduct and both 4-node sides hold at least 3 conducting nodes.
-// Zeros are returned as +0.0; adding or subtracting a signed zero leaves
-// the accumulated weights unchanged, so this matches the reference bits.
-__host__ __device__ __forceinline__ void minor_exact(double d, int m0, int m1,
-                                                     int m2, int m3, int m4, int m5,
-                                                     double q[6]) {
-  const int mh = m2 + m3 + m4 + m5;
-  const int ml = m0 + m1 + m2 + m3;
-  if (m2 == 0 || m3 == 0 || mh < 3 || ml < 3) {
-    q[0] = q[1] = q[2] = q[3] = q[4] = q[5] = 0.0;
-    return;
-  }
-  // mh and ml are 3 or 4: d / 4 is exact as d * 0.25 and d / 3 the correctly
-  // rounded quotient (div_recip), once for both sides (a negative d only
-  // changes its sign); m2 = m3 = 1 makes the middle pair's factor one of
-  // three constants.  The same bits as dividing (the reference's four
-  // quotients) in a quarter of the operations: Aliev-Panfilov 131 x 115 x 147
-  // FP64 with per-node fibres 127 -> 106 us per step.  With uniform fields it
-  // also beats selecting among quotients made once per launch (80 -> 61 us).
+// asymmetric_stencil_2d.py:204-259 for 0/1 mesh values m0..m5, added to
+// (S = 1) or taken from (S = -1) the weights w0..w5: nothing unless the two face
+// nodes m2, m3 conduct and both 4-node sides (m0..m3, m2..m5) hold at least 3
+// conducting nodes.
+template <int S>
+__host__ __device__ __forceinline__ void minor_exact(double d, int m0, int m1, int m2, int m3,
+                                                     int m4, int m5, double& w0, double& w1,
+                                                     double& w2, double& w3, double& w4,
+                                                     double& w5) {
+  const bool fl = m0 && m1, fh = m4 && m5;  // a side of 4, else 3
+  const bool on = m2 && m3 && (m0 || m1) && (m4 || m5);
+  d = on ? d : 0.0;
+  // d / 4 is exact as d * 0.25 and d / 3 the correctly rounded quotient
+  // (div_recip), once for both sides (a negative d only changes its sign);
+  // m2 = m3 = 1 makes the middle pair's factor 0 or the difference of 1/3 and
+  // 1/4.  A product by a 0/1 mask is exact, so a fused multiply-add is the
+  // masked sum in one operation.  The same bits as the reference's four
+  // quotients, without a branch: with one per minor and a register per conduct
+  // bit the 3D step took 153 registers and 3 waves, now 120 and 4, and a wave's
+  // loads overlap its minors (Aliev-Panfilov 131 x 115 x 147: uniform fields 61
+  // -> 44, layered 64 -> 49, per node 102 -> 78 us per step).
   const double d4 = d * 0.25, d3 = div_recip(d, recip(3.0));
-  const double nq = -(ml == 4 ? d4 : d3), pq = mh == 4 ? d4 : d3;
-  const double dc = d * (mh == ml ? 0.0 : (mh == 4 ? 0.25 - 1.0 / 3.0 : 1.0 / 3.0 - 0.25));
-  q[0] = m0 ? nq : 0.0;
-  q[1] = m1 ? nq : 0.0;
-  q[2] = dc;
-  q[3] = dc;
-  q[4] = m4 ? pq : 0.0;
-  q[5] = m5 ? pq : 0.0;
+  const double nq = fl ? d4 : d3, pq = fh ? d4 : d3;
+  constexpr double kThird = 1.0 / 3.0 - 0.25;
+  const double dc = d * (fl == fh ? 0.0 : (fl ? kThird : -kThird));
+  w0 = fma(S > 0 ? -nq : nq, (double)m0, w0);
+  w1 = fma(S > 0 ? -nq : nq, (double)m1, w1);
+  w2 = S > 0 ? w2 + dc : w2 - dc;
+  w3 = S > 0 ? w3 + dc : w3 - dc;
+  w4 = fma(S > 0 ? pq : -pq, (double)m4, w4);
+  w5 = fma(S > 0 ? pq : -pq, (double)m5, w5);
 }
 
-// numpy epilogue: w = w * D * dt / dr**2 ; w[..., centre] += 1.  When dr**2
-// is a power of two, inv_dr2 != 0 holds its exact reciprocal and the division
-// is the same multiplication (barring subnormal results).
+// numpy epilogue: w = w * D * dt / dr**2 ; w[..., centre] += 1.  The division
+// is div_recip's two operations by the launch's reciprocal pair: of a power of
+// two its second half is zero and the product exact.
 template <int K>
 __host__ __device__ __forceinline__ void scale_exact(double W[K], int centre, double D,
-                                            double dt, double dr2, double inv_dr2) {
-  if (inv_dr2 != 0.0) {
+                                            double dt, Recip rdr2) {
 #pragma unroll
-    for (int q = 0; q < K; ++q) W[q] = W[q] * D * dt * inv_dr2;
-  } else {
-#pragma unroll
-    for (int q = 0; q < K; ++q) W[q] = W[q] * D * dt / dr2;
-  }
+  for (int q = 0; q < K; ++q) W[q] = div_recip(W[q] * D * dt, rdr2);
   W[centre] += 1.0;
 }
 
@@ -305,6 +304,38 @@ struct Nbr {
   }
 };
 
+typedef uint32_t __attribute__((aligned(1))) u32_unaligned;
+
+// The same bits of the 19-point stencil (no corners) in one register instead of
+// 19: bytes 0..2 hold the planes dk = -1, 0, 1 of the rows (di, dj) = (-1, 0),
+// (0, -1), (0, 0), (0, 1), (1, 0), byte 3 the middles of the other four rows.
+// A minor's tests are masks of it.  (The 9-point steps gained nothing from it.)
+struct NbrBits {
+  uint32_t m;
+  static constexpr __device__ int bit(int di, int dj, int dk) {
+    return di && dj ? 24 + (di + 1) + (dj + 1) / 2 : 8 * (dk + 1) + 2 + 2 * di + dj;
+  }
+  __device__ __forceinline__ int operator()(int di, int dj, int dk) const {
+    return (m >> bit(di, dj, dk)) & 1;
+  }
+};
+
+// of interior node c: a row's three codes by one 4-byte load (its fourth byte is
+// at most code[N - 1])
+__device__ __forceinline__ NbrBits load_bits(const uint8_t* __restrict__ code, int64_t c,
+                                             int64_t si, int64_t sj) {
+  NbrBits M{0};
+#pragma unroll
+  for (int di = -1; di <= 1; ++di)
+#pragma unroll
+    for (int dj = -1; dj <= 1; ++dj) {
+      const uint8_t* row = code + (c + di * si + dj * sj);
+      if (di && dj) M.m |= (uint32_t)(row[0] & 1) << NbrBits::bit(di, dj, 0);
+      else M.m |= (*(const u32_unaligned*)(row - 1) & 0x00010101u) << NbrBits::bit(di, dj, -1);
+    }
+  return M;
+}
+
 // asymmetric_stencil_2d.py:291-433 (2D: dk = 0 everywhere)
 __host__ __device__ __forceinline__ void wts_aniso2d(double W[9], const Nbr& M,
                                             double dxx0, double dxx1,
@@ -313,102 +344,90 @@ __host__ __device__ __forceinline__ void wts_aniso2d(double W[9], const Nbr& M,
                                             double dyy0, double dyy1) {
 #pragma unroll
   for (int q = 0; q < 9; ++q) W[q] = 0.0;
-  double q[6], qm;
+  double qm;
   qm = dxx0 * (double)M(-1, 0, 0);
   W[1] += qm; W[4] -= qm;
-  minor_exact(dxy0, M(-1, -1, 0), M(0, -1, 0), M(-1, 0, 0), M(0, 0, 0),
-              M(-1, 1, 0), M(0, 1, 0), q);
-  W[0] -= q[0]; W[3] -= q[1]; W[1] -= q[2]; W[4] -= q[3]; W[2] -= q[4]; W[5] -= q[5];
+  minor_exact<-1>(dxy0, M(-1, -1, 0), M(0, -1, 0), M(-1, 0, 0),
+                  M(0, 0, 0), M(-1, 1, 0), M(0, 1, 0),
+                  W[0], W[3], W[1], W[4], W[2], W[5]);
   qm = dyy0 * (double)M(0, -1, 0);
   W[3] += qm; W[4] -= qm;
-  minor_exact(dyx0, M(-1, -1, 0), M(-1, 0, 0), M(0, -1, 0), M(0, 0, 0),
-              M(1, -1, 0), M(1, 0, 0), q);
-  W[0] -= q[0]; W[1] -= q[1]; W[3] -= q[2]; W[4] -= q[3]; W[6] -= q[4]; W[7] -= q[5];
+  minor_exact<-1>(dyx0, M(-1, -1, 0), M(-1, 0, 0), M(0, -1, 0),
+                  M(0, 0, 0), M(1, -1, 0), M(1, 0, 0),
+                  W[0], W[1], W[3], W[4], W[6], W[7]);
   qm = dyy1 * (double)M(0, 1, 0);
   W[5] += qm; W[4] -= qm;
-  minor_exact(dyx1, M(-1, 1, 0), M(-1, 0, 0), M(0, 1, 0), M(0, 0, 0),
-              M(1, 1, 0), M(1, 0, 0), q);
-  W[2] += q[0]; W[1] += q[1]; W[5] += q[2]; W[4] += q[3]; W[8] += q[4]; W[7] += q[5];
+  minor_exact<1>(dyx1, M(-1, 1, 0), M(-1, 0, 0), M(0, 1, 0),
+                  M(0, 0, 0), M(1, 1, 0), M(1, 0, 0),
+                  W[2], W[1], W[5], W[4], W[8], W[7]);
   qm = dxx1 * (double)M(1, 0, 0);
   W[7] += qm; W[4] -= qm;
-  minor_exact(dxy1, M(1, -1, 0), M(0, -1, 0), M(1, 0, 0), M(0, 0, 0),
-              M(1, 1, 0), M(0, 1, 0), q);
-  W[6] += q[0]; W[3] += q[1]; W[7] += q[2]; W[4] += q[3]; W[8] += q[4]; W[5] += q[5];
+  minor_exact<1>(dxy1, M(1, -1, 0), M(0, -1, 0), M(1, 0, 0),
+                  M(0, 0, 0), M(1, 1, 0), M(0, 1, 0),
+                  W[6], W[3], W[7], W[4], W[8], W[5]);
 }
 
 // asymmetric_stencil_3d.py:163-458; d[face][comp]: faces x0 x1 y0 y1 z0 z1,
 // comps: x faces (xx, xy, xz), y faces (yy, yx, yz), z faces (zz, zx, zy)
-__device__ __forceinline__ void wts_aniso3d(double W[19], const Nbr& M,
-                                            const double d[6][3]) {
+template <typename NB>
+__device__ __forceinline__ void wts_aniso3d(double W[19], const NB& M, const double d[6][3]) {
 #pragma unroll
   for (int q = 0; q < 19; ++q) W[q] = 0.0;
-  double q[6], qm;
+  double qm;
   // q (i-1/2, j, k)
   qm = d[0][0] * (double)M(-1, 0, 0);
   W[1] += qm; W[4] -= qm;
-  minor_exact(d[0][1],
-              M(-1, -1, 0), M(0, -1, 0), M(-1, 0, 0), M(0, 0, 0),
-              M(-1, 1, 0), M(0, 1, 0), q);
-  W[0] -= q[0]; W[3] -= q[1]; W[1] -= q[2]; W[4] -= q[3]; W[2] -= q[4]; W[5] -= q[5];
-  minor_exact(d[0][2],
-              M(-1, 0, -1), M(0, 0, -1), M(-1, 0, 0), M(0, 0, 0),
-              M(-1, 0, 1), M(0, 0, 1), q);
-  W[15] -= q[0]; W[11] -= q[1]; W[1] -= q[2]; W[4] -= q[3]; W[17] -= q[4]; W[12] -= q[5];
+  minor_exact<-1>(d[0][1], M(-1, -1, 0), M(0, -1, 0), M(-1, 0, 0),
+                  M(0, 0, 0), M(-1, 1, 0), M(0, 1, 0),
+                  W[0], W[3], W[1], W[4], W[2], W[5]);
+  minor_exact<-1>(d[0][2], M(-1, 0, -1), M(0, 0, -1), M(-1, 0, 0),
+                  M(0, 0, 0), M(-1, 0, 1), M(0, 0, 1),
+                  W[15], W[11], W[1], W[4], W[17], W[12]);
   // q (i+1/2, j, k)
   qm = d[1][0] * (double)M(1, 0, 0);
   W[7] += qm; W[4] -= qm;
-  minor_exact(d[1][1],
-              M(1, -1, 0), M(0, -1, 0), M(1, 0, 0), M(0, 0, 0),
-              M(1, 1, 0), M(0, 1, 0), q);
-  W[6] += q[0]; W[3] += q[1]; W[7] += q[2]; W[4] += q[3]; W[8] += q[4]; W[5] += q[5];
-  minor_exact(d[1][2],
-              M(1, 0, -1), M(0, 0, -1), M(1, 0, 0), M(0, 0, 0),
-              M(1, 0, 1), M(0, 0, 1), q);
-  W[16] += q[0]; W[11] += q[1]; W[7] += q[2]; W[4] += q[3]; W[18] += q[4]; W[12] += q[5];
+  minor_exact<1>(d[1][1], M(1, -1, 0), M(0, -1, 0), M(1, 0, 0),
+                  M(0, 0, 0), M(1, 1, 0), M(0, 1, 0),
+                  W[6], W[3], W[7], W[4], W[8], W[5]);
+  minor_exact<1>(d[1][2], M(1, 0, -1), M(0, 0, -1), M(1, 0, 0),
+                  M(0, 0, 0), M(1, 0, 1), M(0, 0, 1),
+                  W[16], W[11], W[7], W[4], W[18], W[12]);
   // q (i, j-1/2, k)
   qm = d[2][0] * (double)M(0, -1, 0);
   W[3] += qm; W[4] -= qm;
-  minor_exact(d[2][1],
-              M(-1, -1, 0), M(-1, 0, 0), M(0, -1, 0), M(0, 0, 0),
-              M(1, -1, 0), M(1, 0, 0), q);
-  W[0] -= q[0]; W[1] -= q[1]; W[3] -= q[2]; W[4] -= q[3]; W[6] -= q[4]; W[7] -= q[5];
-  minor_exact(d[2][2],
-              M(0, -1, -1), M(0, 0, -1), M(0, -1, 0), M(0, 0, 0),
-              M(0, -1, 1), M(0, 0, 1), q);
-  W[9] -= q[0]; W[11] -= q[1]; W[3] -= q[2]; W[4] -= q[3]; W[10] -= q[4]; W[12] -= q[5];
+  minor_exact<-1>(d[2][1], M(-1, -1, 0), M(-1, 0, 0), M(0, -1, 0),
+                  M(0, 0, 0), M(1, -1, 0), M(1, 0, 0),
+                  W[0], W[1], W[3], W[4], W[6], W[7]);
+  minor_exact<-1>(d[2][2], M(0, -1, -1), M(0, 0, -1), M(0, -1, 0),
+                  M(0, 0, 0), M(0, -1, 1), M(0, 0, 1),
+                  W[9], W[11], W[3], W[4], W[10], W[12]);
   // q (i, j+1/2, k)
   qm = d[3][0] * (double)M(0, 1, 0);
   W[5] += qm; W[4] -= qm;
-  minor_exact(d[3][1],
-              M(-1, 1, 0), M(-1, 0, 0), M(0, 1, 0), M(0, 0, 0),
-              M(1, 1, 0), M(1, 0, 0), q);
-  W[2] += q[0]; W[1] += q[1]; W[5] += q[2]; W[4] += q[3]; W[8] += q[4]; W[7] += q[5];
-  minor_exact(d[3][2],
-              M(0, 1, -1), M(0, 0, -1), M(0, 1, 0), M(0, 0, 0),
-              M(0, 1, 1), M(0, 0, 1), q);
-  W[13] += q[0]; W[11] += q[1]; W[5] += q[2]; W[4] += q[3]; W[14] += q[4]; W[12] += q[5];
+  minor_exact<1>(d[3][1], M(-1, 1, 0), M(-1, 0, 0), M(0, 1, 0),
+                  M(0, 0, 0), M(1, 1, 0), M(1, 0, 0),
+                  W[2], W[1], W[5], W[4], W[8], W[7]);
+  minor_exact<1>(d[3][2], M(0, 1, -1), M(0, 0, -1), M(0, 1, 0),
+                  M(0, 0, 0), M(0, 1, 1), M(0, 0, 1),
+                  W[13], W[11], W[5], W[4], W[14], W[12]);
   // q (i, j, k-1/2)
   qm = d[4][0] * (double)M(0, 0, -1);
   W[11] += qm; W[4] -= qm;
-  minor_exact(d[4][1],
-              M(-1, 0, -1), M(-1, 0, 0), M(0, 0, -1), M(0, 0, 0),
-              M(1, 0, -1), M(1, 0, 0), q);
-  W[15] -= q[0]; W[1] -= q[1]; W[11] -= q[2]; W[4] -= q[3]; W[16] -= q[4]; W[7] -= q[5];
-  minor_exact(d[4][2],
-              M(0, -1, -1), M(0, -1, 0), M(0, 0, -1), M(0, 0, 0),
-              M(0, 1, -1), M(0, 1, 0), q);
-  W[9] -= q[0]; W[3] -= q[1]; W[11] -= q[2]; W[4] -= q[3]; W[13] -= q[4]; W[5] -= q[5];
+  minor_exact<-1>(d[4][1], M(-1, 0, -1), M(-1, 0, 0), M(0, 0, -1),
+                  M(0, 0, 0), M(1, 0, -1), M(1, 0, 0),
+                  W[15], W[1], W[11], W[4], W[16], W[7]);
+  minor_exact<-1>(d[4][2], M(0, -1, -1), M(0, -1, 0), M(0, 0, -1),
+                  M(0, 0, 0), M(0, 1, -1), M(0, 1, 0),
+                  W[9], W[3], W[11], W[4], W[13], W[5]);
   // q (i, j, k+1/2)
   qm = d[5][0] * (double)M(0, 0, 1);
   W[12] += qm; W[4] -= qm;
-  minor_exact(d[5][1],
-              M(-1, 0, 1), M(-1, 0, 0), M(0, 0, 1), M(0, 0, 0),
-              M(1, 0, 1), M(1, 0, 0), q);
-  W[17] += q[0]; W[1] += q[1]; W[12] += q[2]; W[4] += q[3]; W[18] += q[4]; W[7] += q[5];
-  minor_exact(d[5][2],
-              M(0, -1, 1), M(0, -1, 0), M(0, 0, 1), M(0, 0, 0),
-              M(0, 1, 1), M(0, 1, 0), q);
-  W[10] += q[0]; W[3] += q[1]; W[12] += q[2]; W[4] += q[3]; W[14] += q[4]; W[5] += q[5];
+  minor_exact<1>(d[5][1], M(-1, 0, 1), M(-1, 0, 0), M(0, 0, 1),
+                  M(0, 0, 0), M(1, 0, 1), M(1, 0, 0),
+                  W[17], W[1], W[12], W[4], W[18], W[7]);
+  minor_exact<1>(d[5][2], M(0, -1, 1), M(0, -1, 0), M(0, 0, 1),
+                  M(0, 0, 0), M(0, 1, 1), M(0, 1, 0),
+                  W[10], W[3], W[12], W[4], W[14], W[5]);
 }
 
 // symmetric_stencil_2d.py:120-150 (weights builder only)
@@ -724,7 +743,7 @@ __device__ __forceinline__ R diffuse(const KArgs<RA, R>& a, int64_t i, int64_t j
         W[3] = iso_comp(dE, mE, mW);
         W[4] = iso_comp(dS, mS, mN);
         W[2] = -(W[0] + W[1] + W[3] + W[4]);
-        scale_exact<5>(W, 2, a.D, a.dtd, a.dr2, a.inv_dr2);
+        scale_exact<5>(W, 2, a.D, a.dtd, a.rdr2);
       }
       return u[c - sN] * W[0] + u[c - 1] * W[1] + uc * W[2] + u[c + 1] * W[3] +
              u[c + sN] * W[4];
@@ -761,11 +780,8 @@ __device__ __forceinline__ R diffuse(const KArgs<RA, R>& a, int64_t i, int64_t j
 #pragma unroll
         for (int q = 0; q < 9; ++q) W[q] = a.wfull[q];
       } else {
-        if constexpr (FL == kFieldsUniform)
-          wts_aniso2d(W, M, dxx0, dxx1, dxy0, dxy1, dyx0, dyx1, dyy0, dyy1);
-        else
-          wts_aniso2d(W, M, dxx0, dxx1, dxy0, dxy1, dyx0, dyx1, dyy0, dyy1);
-        scale_exact<9>(W, 4, a.D, a.dtd, a.dr2, a.inv_dr2);
+        wts_aniso2d(W, M, dxx0, dxx1, dxy0, dxy1, dyx0, dyx1, dyy0, dyy1);
+        scale_exact<9>(W, 4, a.D, a.dtd, a.rdr2);
       }
       return u[c - sN - 1] * W[0] + u[c - sN] * W[1] + u[c - sN + 1] * W[2] +
              u[c - 1] * W[3] + uc * W[4] + u[c + 1] * W[5] +
@@ -807,7 +823,7 @@ __device__ __forceinline__ R diffuse(const KArgs<RA, R>& a, int64_t i, int64_t j
         W[5] = iso_comp(dYp, mYp, mYm);
         W[6] = iso_comp(dXp, mXp, mXm);
         W[3] = -(W[0] + W[1] + W[2] + W[4] + W[5] + W[6]);
-        scale_exact<7>(W, 3, a.D, a.dtd, a.dr2, a.inv_dr2);
+        scale_exact<7>(W, 3, a.D, a.dtd, a.rdr2);
         return u[c - si] * W[0] + u[c - sj] * W[1] + u[c - 1] * W[2] + uc * W[3] +
                u[c + 1] * W[4] + u[c + sj] * W[5] + u[c + si] * W[6];
       } else {
@@ -823,17 +839,21 @@ __device__ __forceinline__ R diffuse(const KArgs<RA, R>& a, int64_t i, int64_t j
         return uc + a.s * fl;
       }
     } else {  // anisotropic 19-point
-      Nbr M;
+      std::conditional_t<EXACT, NbrBits, Nbr> M;
+      if constexpr (EXACT) {
+        M = load_bits(a.code, c, si, sj);
+      } else {
 #pragma unroll
-      for (int di = -1; di <= 1; ++di)
+        for (int di = -1; di <= 1; ++di)
 #pragma unroll
-        for (int dj = -1; dj <= 1; ++dj)
+          for (int dj = -1; dj <= 1; ++dj)
 #pragma unroll
-          for (int dk = -1; dk <= 1; ++dk) {
-            const int corner = (di != 0) && (dj != 0) && (dk != 0);
-            M.m[(di + 1) * 9 + (dj + 1) * 3 + dk + 1] =
-                corner ? 0 : (a.code[c + di * si + dj * sj + dk] & 1);
-          }
+            for (int dk = -1; dk <= 1; ++dk) {
+              const int corner = (di != 0) && (dj != 0) && (dk != 0);
+              M.m[(di + 1) * 9 + (dj + 1) * 3 + dk + 1] =
+                  corner ? 0 : (a.code[c + di * si + dj * sj + dk] & 1);
+            }
+      }
       // fields: 0 xx 1 xy 2 xz 3 yx 4 yy 5 yz 6 zx 7 zy 8 zz
       R d[6][3];
       fval_pair_l<R, 0, FL>(a.f[0], i, j, k, c, si, d[1][0], d[0][0]);
@@ -848,7 +868,7 @@ __device__ __forceinline__ R diffuse(const KArgs<RA, R>& a, int64_t i, int64_t j
       if constexpr (EXACT) {
         double W[19];
         wts_aniso3d(W, M, d);
-        scale_exact<19>(W, 4, a.D, a.dtd, a.dr2, a.inv_dr2);
+        scale_exact<19>(W, 4, a.D, a.dtd, a.rdr2);
         return u[c - si - sj] * W[0] + u[c - si] * W[1] + u[c - si + sj] * W[2] +
                u[c - sj] * W[3] + uc * W[4] + u[c + sj] * W[5] +
                u[c + si - sj] * W[6] + u[c + si] * W[7] + u[c + si + sj] * W[8] +
@@ -904,7 +924,6 @@ struct Vec4T<int32_t> {
 };
 template <typename T>
 using Vec4 = typename Vec4T<T>::type;
-typedef uint32_t __attribute__((aligned(1))) u32_unaligned;
 
 // A point probe's value at node c (pre-step potential uc, post-update state)
 template <typename R, int MODEL, int PREC, typename A>

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(kMultiThreads) void k_multi2d(const KArgs<R, R> a,
         W[3] = iso_comp(d1, q.m[5], q.m[3]);
         W[4] = iso_comp(d0, q.m[7], q.m[1]);
         W[2] = -(W[0] + W[1] + W[3] + W[4]);
-        scale_exact<5>(W, 2, a.D, a.dtd, a.dr2, a.inv_dr2);
+        scale_exact<5>(W, 2, a.D, a.dtd, a.rdr2);
       } else {
         Nbr M;
 #pragma unroll
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(kMultiThreads) void k_multi2d(const KArgs<R, R> a,
         for (int k = 0; k < 9; ++k) M.m[3 * k + 1] = q.m[k];
         const double xx = a.f[0].value, xy = a.f[1].value, yx = a.f[2].value, yy = a.f[3].value;
         wts_aniso2d(W, M, xx, xx, xy, xy, yx, yx, yy, yy);
-        scale_exact<9>(W, 4, a.D, a.dtd, a.dr2, a.inv_dr2);
+        scale_exact<9>(W, 4, a.D, a.dtd, a.rdr2);
       }
     }
   }

@@ -107,12 +107,7 @@ static void fill_args(const fw_plan* plan, const void* u, void* u_new, const Sta
   a.w = d.weights;
   a.D = d.D_model;
   a.dtd = d.dt;
-  a.dr2 = d.dr2;
-  {
-    int e2;
-    const double mant = frexp(d.dr2, &e2);
-    a.inv_dr2 = (mant == 0.5 && e2 > -1000 && e2 < 1000) ? ldexp(1.0, 1 - e2) : 0.0;
-  }
+  a.rdr2 = recip(d.dr2);
   if (FW_PREC == 0 && plan->field_layout == kFieldsUniform && d.ndim == 2) {
     // the exact weights of a node whose 3x3 neighbourhood all conducts, by
     // the kernel's own functions (this FP64 unit is built without
@@ -124,14 +119,14 @@ static void fill_args(const fw_plan* plan, const void* u, void* u_new, const Sta
     if (d.stencil == FW_STENCIL_ANISO) {
       const double f2 = d.fields[2].value, f3 = d.fields[3].value;
       wts_aniso2d(W, M, f0, f0, f1, f1, f2, f2, f3, f3);
-      scale_exact<9>(W, 4, a.D, a.dtd, a.dr2, a.inv_dr2);
+      scale_exact<9>(W, 4, a.D, a.dtd, a.rdr2);
     } else {
       W[0] = iso_comp(f0, 1, 1);
       W[1] = iso_comp(f1, 1, 1);
       W[3] = iso_comp(f1, 1, 1);
       W[4] = iso_comp(f0, 1, 1);
       W[2] = -(W[0] + W[1] + W[3] + W[4]);
-      scale_exact<5>(W, 2, a.D, a.dtd, a.dr2, a.inv_dr2);
+      scale_exact<5>(W, 2, a.D, a.dtd, a.rdr2);
     }
   }
   a.dt = (Real)d.dt;
