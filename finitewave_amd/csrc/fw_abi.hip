@@ -431,27 +431,31 @@ static int plan_host_init(const fw_plan_desc* desc, fw_plan* p, const char* who)
   p->per_xcd = (p->nblocks + kXcds - 1) / kXcds;
   p->grid = p->per_xcd * kXcds;
   p->K = d.ndim == 2 ? 9 : 19;
-  // the field layout: every field uniform (kFieldsUniform), or in 3D every
-  // field uniform or tabulated along the last axis (kFieldsK, layered
-  // fibres); such plans get their step kernel without the per-field mode
-  // dispatch
+  // the field layout: every field uniform (kFieldsUniform), in 3D every field
+  // uniform or tabulated along the last axis (kFieldsK, layered fibres), or
+  // every field uniform or a full array (kFieldsFull); such plans get their
+  // step kernel without the per-field mode dispatch
   p->field_layout = fw::kFieldsGeneral;
   if (d.stencil != FW_STENCIL_WEIGHTS) {
-    bool uni = true, along_k = d.ndim == 3;
+    bool uni = true, along_k = d.ndim == 3, full = true;
     for (int q = 0; q < need_fields; ++q) {
       const fw_field& f = d.fields[q];
       if (f.mode != FW_FIELD_UNIFORM) uni = false;
+      if (f.mode == FW_FIELD_AXIS) full = false;
       if (!(f.mode == FW_FIELD_UNIFORM || (f.mode == FW_FIELD_AXIS && f.axis == 2)))
         along_k = false;
     }
     if (uni) p->field_layout = fw::kFieldsUniform;
     else if (along_k) p->field_layout = fw::kFieldsK;
+    else if (full) p->field_layout = fw::kFieldsFull;
   }
   return FW_OK;
 }
 
-// The step words' share of their allocation: what follows is aligned for any load.
+// The step words' and uniform field values' share of their allocation: what
+// follows is aligned for any load.
 constexpr size_t kStepWordBytes = 256;
+static_assert(16 + FW_MAX_FIELDS * (sizeof(double) + sizeof(float)) <= kStepWordBytes);
 
 // The largest sheet stepped by multi-step launches (2000^2 still gains 2 % to
 // 17 %, past it both are bound by HBM), the largest of the models with tanh
@@ -556,6 +560,20 @@ int fw_plan_create(const fw_plan_desc* desc, fw_plan** out) {
       set_error("fw_plan_create: field tables along k: %s", hipGetErrorString(e));
       fw_plan_destroy(p);
       return FW_E_NOMEM;
+    }
+  }
+  if (p->field_layout == fw::kFieldsFull) {
+    for (int q = 0; q < need_fields; ++q)
+      if (d.fields[q].mode == FW_FIELD_UNIFORM)
+        hipLaunchKernelGGL(k_fill_ktab, dim3(1), dim3(64), 0, 0, nullptr, d.fields[q].value,
+                           uniform_values(p->step_words) + q, uniform_fvalues(p->step_words) + q,
+                           (int64_t)1);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (e != hipSuccess) {
+      set_error("fw_plan_create: uniform field values: %s", hipGetErrorString(e));
+      fw_plan_destroy(p);
+      return FW_E_HIP;
     }
   }
   *out = p;
@@ -902,6 +920,10 @@ int fw_run_noalloc(const fw_plan_desc* desc, void* u, void* u_new, void* const* 
   if (rc) return rc;
   const fw_plan_desc& d = p.desc;
   const int need = needed_fields(d);
+  // no device words to hold uniform fields' values
+  for (int q = 0; q < need; ++q)
+    if (p.field_layout == kFieldsFull && d.fields[q].mode == FW_FIELD_UNIFORM)
+      p.field_layout = kFieldsGeneral;
   // offsets of the tables in the scratch array, then its size
   size_t off_f[FW_MAX_FIELDS] = {}, off_kd[FW_MAX_FIELDS] = {}, off_kf[FW_MAX_FIELDS] = {};
   int64_t len_f[FW_MAX_FIELDS] = {};

@@ -16,7 +16,8 @@ struct fw_plan {
   uint32_t per_xcd;  // logical blocks per XCD
   uint32_t grid;     // launched blocks = per_xcd * 8
   int32_t K;         // weights per node for FW_STENCIL_WEIGHTS
-  int32_t* step_words;  // device int32[4]: graph step words [0..1], stim_end [2]
+  // device int32[4]: graph step words [0..1], stim_end [2]; then uniform_values
+  int32_t* step_words;
   // captured step graphs for two buffer orientations (u, u_new) and (u_new,
   // u): per orientation, graphs of 2^b pairs of steps (b = 0..kGraphBits-1),
   // captured when first needed; all keyed on the same tracker and state
@@ -53,6 +54,15 @@ struct fw_plan {
 };
 
 namespace fw {
+
+// The values of a kFieldsFull plan's uniform fields, in double and in float, in
+// device memory behind the step words.
+inline double* uniform_values(int32_t* step_words) {
+  return reinterpret_cast<double*>(step_words + 4);
+}
+inline float* uniform_fvalues(int32_t* step_words) {
+  return reinterpret_cast<float*>(uniform_values(step_words) + FW_MAX_FIELDS);
+}
 
 struct TrackArgs {
   int32_t* act;

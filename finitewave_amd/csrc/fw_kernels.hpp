@@ -32,7 +32,7 @@ namespace fw {
 
 struct Field {
   int32_t mode;  // 0 uniform, 1 per-axis table, 2 full
-  int32_t axis;
+  int32_t axis;  // of mode 1; kFieldsFull: the index mask, -1 or 0 (uniform)
   double value;
   const double* data;
   float fvalue;        // the same in float, for kernels computing in float:
@@ -42,8 +42,15 @@ struct Field {
 // How a plan's half-step fields are stored, as far as the step kernel is
 // specialised for it: kFieldsUniform, every field uniform; kFieldsK (3D),
 // every field a table along the last axis (the plan tabulates uniform ones
-// too: layered fibres); kFieldsGeneral, a mode per field, read by dispatch.
-enum FieldLayout : int32_t { kFieldsGeneral = 0, kFieldsUniform = 1, kFieldsK = 2 };
+// too: layered fibres); kFieldsFull, every field a full array or uniform
+// (per-node fibres or conductivity); kFieldsGeneral, a mode per field, read by
+// dispatch.
+enum FieldLayout : int32_t {
+  kFieldsGeneral = 0,
+  kFieldsUniform = 1,
+  kFieldsK = 2,
+  kFieldsFull = 3
+};
 
 // a half-step field at node (i, j, k) = flat index c, in the type F the
 // diffusion is computed in; the mode is uniform across a launch
@@ -77,9 +84,21 @@ __device__ __forceinline__ void fval_pair(const Field& f, int64_t i, int64_t j, 
     below = fval<F>(f, i - (DIR == 0), j - (DIR == 1), k - (DIR == 2), c - step);
 }
 
+// a field of a kFieldsFull plan at node c: its axis is -1, or 0 for a uniform
+// field, whose data is the one value.  No branch, so a node's loads are in flight
+// together; behind the dispatch each waited for the one before (131 x 115 x 147,
+// per-node fibres, FP64: 78 -> 54 us per step, FP32: 40 -> 26; a 514 x 387 sheet
+// of Courtemanche FP64 29.5 -> 28.4, of TP06 FP32 14.0 -> 12.4).
+template <typename F>
+__device__ __forceinline__ F ffull(const Field& f, int64_t c) {
+  const int64_t q = c & f.axis;
+  if constexpr (sizeof(F) == 4) return ((const global_t<float>*)f.fdata)[q];
+  else return ((const global_t<double>*)f.data)[q];
+}
+
 // fval_pair for a kernel specialised to a field layout FL: uniform values
-// straight from the arguments, tables along the last axis indexed by k, or
-// the general per-field dispatch
+// straight from the arguments, tables along the last axis indexed by k, full
+// arrays indexed by the node, or the general per-field dispatch
 template <typename F, int DIR, int FL>
 __device__ __forceinline__ void fval_pair_l(const Field& f, int64_t i, int64_t j, int64_t k,
                                             int64_t c, int64_t step, F& at_c, F& below) {
@@ -91,6 +110,9 @@ __device__ __forceinline__ void fval_pair_l(const Field& f, int64_t i, int64_t j
     else t = (const global_t<F>*)f.data;
     at_c = t[k];
     below = DIR == 2 ? t[k - 1] : at_c;
+  } else if constexpr (FL == kFieldsFull) {
+    at_c = ffull<F>(f, c);
+    below = ffull<F>(f, c - step);
   } else {
     fval_pair<F, DIR>(f, i, j, k, c, step, at_c, below);
   }
@@ -594,35 +616,22 @@ __device__ __forceinline__ R flux_aniso(const Hood2<R>& q, R dxx0, R dxx1, R dxy
 }
 
 // FP32 flux form of the 2D isotropic (ST 0) and anisotropic (ST 1) stencils
-// on a loaded neighbourhood; R is the potential's storage type.  UNI: every
-// field is uniform and its value comes straight from the arguments
-template <int ST, bool UNI, typename RA, typename R>
+// on a loaded neighbourhood; R is the potential's storage type
+template <int ST, int FL, typename RA, typename R>
 __device__ __forceinline__ R flux2d(const KArgs<RA, R>& a, int64_t i, int64_t j, int64_t c,
                                     R uc, const Hood2<R>& q) {
   const int64_t sN = a.nj;
   if constexpr (ST == 0) {
     R dN, dS, dW, dE;
-    if constexpr (UNI) {
-      dN = dS = funi<R>(a.f[0]);
-      dW = dE = funi<R>(a.f[1]);
-    } else {
-      fval_pair<R, 0>(a.f[0], i, j, 0, c, sN, dS, dN);
-      fval_pair<R, 1>(a.f[1], i, j, 0, c, 1, dE, dW);
-    }
+    fval_pair_l<R, 0, FL>(a.f[0], i, j, 0, c, sN, dS, dN);
+    fval_pair_l<R, 1, FL>(a.f[1], i, j, 0, c, 1, dE, dW);
     return flux_iso<R>(q, dN, dW, dE, dS, a.s);
   } else {
     R dxx0, dxx1, dxy0, dxy1, dyx0, dyx1, dyy0, dyy1;
-    if constexpr (UNI) {
-      dxx0 = dxx1 = funi<R>(a.f[0]);
-      dxy0 = dxy1 = funi<R>(a.f[1]);
-      dyx0 = dyx1 = funi<R>(a.f[2]);
-      dyy0 = dyy1 = funi<R>(a.f[3]);
-    } else {
-      fval_pair<R, 0>(a.f[0], i, j, 0, c, sN, dxx1, dxx0);
-      fval_pair<R, 0>(a.f[1], i, j, 0, c, sN, dxy1, dxy0);
-      fval_pair<R, 1>(a.f[2], i, j, 0, c, 1, dyx1, dyx0);
-      fval_pair<R, 1>(a.f[3], i, j, 0, c, 1, dyy1, dyy0);
-    }
+    fval_pair_l<R, 0, FL>(a.f[0], i, j, 0, c, sN, dxx1, dxx0);
+    fval_pair_l<R, 0, FL>(a.f[1], i, j, 0, c, sN, dxy1, dxy0);
+    fval_pair_l<R, 1, FL>(a.f[2], i, j, 0, c, 1, dyx1, dyx0);
+    fval_pair_l<R, 1, FL>(a.f[3], i, j, 0, c, 1, dyy1, dyy0);
     return flux_aniso<R>(q, dxx0, dxx1, dxy0, dxy1, dyx0, dyx1, dyy0, dyy1, a.s);
   }
 }
@@ -718,20 +727,15 @@ __device__ __forceinline__ R diffuse(const KArgs<RA, R>& a, int64_t i, int64_t j
                  (double)u[c + sN + 1] * W[8]);
     } else if constexpr (!EXACT) {
       const Hood2<R> q = load_hood2<ST>(a, c, uc);
-      if constexpr (FL == kFieldsUniform) return flux2d<ST, true>(a, i, j, c, uc, q);
-      return a.field_layout == kFieldsUniform ? flux2d<ST, true>(a, i, j, c, uc, q)
-                                              : flux2d<ST, false>(a, i, j, c, uc, q);
+      if constexpr (FL != kFieldsGeneral) return flux2d<ST, FL>(a, i, j, c, uc, q);
+      return a.field_layout == kFieldsUniform ? flux2d<ST, kFieldsUniform>(a, i, j, c, uc, q)
+                                              : flux2d<ST, kFieldsGeneral>(a, i, j, c, uc, q);
     } else if constexpr (ST == 0) {
       const int mN = a.code[c - sN] & 1, mS = a.code[c + sN] & 1;
       const int mW = a.code[c - 1] & 1, mE = a.code[c + 1] & 1;
       R dN, dS, dW, dE;
-      if constexpr (FL == kFieldsUniform) {
-        dN = dS = funi<R>(a.f[0]);
-        dW = dE = funi<R>(a.f[1]);
-      } else {
-        fval_pair<R, 0>(a.f[0], i, j, 0, c, sN, dS, dN);
-        fval_pair<R, 1>(a.f[1], i, j, 0, c, 1, dE, dW);
-      }
+      fval_pair_l<R, 0, FL>(a.f[0], i, j, 0, c, sN, dS, dN);
+      fval_pair_l<R, 1, FL>(a.f[1], i, j, 0, c, 1, dE, dW);
       double W[5];
       if (FL == kFieldsUniform && (mN & mS & mW & mE)) {
         // every neighbour conducts: the host's weights for such a node
@@ -758,17 +762,10 @@ __device__ __forceinline__ R diffuse(const KArgs<RA, R>& a, int64_t i, int64_t j
           M.m[(di + 1) * 9 + (dj + 1) * 3 + 1] = a.code[c + di * sN + dj] & 1;
         }
       R dxx0, dxx1, dxy0, dxy1, dyx0, dyx1, dyy0, dyy1;
-      if constexpr (FL == kFieldsUniform) {
-        dxx0 = dxx1 = funi<R>(a.f[0]);
-        dxy0 = dxy1 = funi<R>(a.f[1]);
-        dyx0 = dyx1 = funi<R>(a.f[2]);
-        dyy0 = dyy1 = funi<R>(a.f[3]);
-      } else {
-        fval_pair<R, 0>(a.f[0], i, j, 0, c, sN, dxx1, dxx0);
-        fval_pair<R, 0>(a.f[1], i, j, 0, c, sN, dxy1, dxy0);
-        fval_pair<R, 1>(a.f[2], i, j, 0, c, 1, dyx1, dyx0);
-        fval_pair<R, 1>(a.f[3], i, j, 0, c, 1, dyy1, dyy0);
-      }
+      fval_pair_l<R, 0, FL>(a.f[0], i, j, 0, c, sN, dxx1, dxx0);
+      fval_pair_l<R, 0, FL>(a.f[1], i, j, 0, c, sN, dxy1, dxy0);
+      fval_pair_l<R, 1, FL>(a.f[2], i, j, 0, c, 1, dyx1, dyx0);
+      fval_pair_l<R, 1, FL>(a.f[3], i, j, 0, c, 1, dyy1, dyy0);
       double W[9];
       int all = 1;
 #pragma unroll
@@ -899,12 +896,14 @@ __device__ __forceinline__ R diffuse(const KArgs<RA, R>& a, int64_t i, int64_t j
 // Waves per SIMD the compiler must leave room for.  The 2D TP06 steps hold 5:
 // FP64 then takes 96 registers and spills 7 (uniform-field instance; 1026^2,
 // 132.3 -> 127.4 us per step against 4 waves without spills; the compiler
-// alone would choose 3); FP32 takes 91-94 without spills.  The 3D
-// anisotropic FP64 step would spill 74 registers under a 128-register
-// budget.  Other steps keep the compiler's choice.
+// alone would choose 3); FP32 takes 91-94 without spills.  The 3D FP64 LR91
+// steps hold 4, spilling 5 registers at most (131 x 115 x 147, per-node fibres,
+// 164 -> 148 us per step against the compiler's 3); with 4 the Bueno-Orovio
+// ones would spill 36 and more (90 -> 253 us).  Other steps keep the compiler's
+// choice.
 template <int NDIM, int MODEL, int PREC>
 constexpr int step_min_waves() {
-  return (NDIM == 2 && MODEL == 6) ? 5 : 1;
+  return (NDIM == 2 && MODEL == 6) ? 5 : (NDIM == 3 && PREC == 0 && MODEL == 5) ? 4 : 1;
 }
 
 // 4 values of consecutive nodes, element-aligned: one vector load or store
@@ -1009,7 +1008,7 @@ __device__ __forceinline__ void step_node(const KArgs<R, UType<MODEL, R>>& a, in
         // update, as in the batched step
         const Hood2<U> q = load_hood2<ST>(a, c, uc);
         v = node_update<MODEL, R>(uc, a.st, c, a.dt, a.P, [&] {
-          return flux2d<ST, FL == kFieldsUniform>(a, i, j, c, uc, q);
+          return flux2d<ST, FL>(a, i, j, c, uc, q);
         });
       } else {
         v = node_update<MODEL, R>(uc, a.st, c, a.dt, a.P, [&] {

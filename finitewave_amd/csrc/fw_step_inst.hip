@@ -52,6 +52,11 @@ static void launch(const fw_plan* plan, const KArgs<Real, UReal>& a, hipStream_t
                          dim3(plan->grid), dim3(kBlock), 0, s, a);
       return;
     }
+    if (a.field_layout == kFieldsFull) {
+      hipLaunchKernelGGL((k_step<NDIM, ST, FW_MODEL, Real, FW_PREC, kFieldsFull>),
+                         dim3(plan->grid), dim3(kBlock), 0, s, a);
+      return;
+    }
     if constexpr (NDIM == 3) {
       if (a.field_layout == kFieldsK) {
         hipLaunchKernelGGL((k_step<NDIM, ST, FW_MODEL, Real, FW_PREC, kFieldsK>),
@@ -101,6 +106,14 @@ static void fill_args(const fw_plan* plan, const void* u, void* u_new, const Sta
       a.f[q].axis = 2;
       a.f[q].data = plan->ktab[q];
       a.f[q].fdata = plan->fktab[q];
+    }
+  }
+  if (plan->field_layout == kFieldsFull) {
+    for (int q = 0; q < d.n_fields; ++q) {
+      a.f[q].axis = a.f[q].mode == FW_FIELD_FULL ? -1 : 0;
+      if (a.f[q].mode == FW_FIELD_FULL) continue;
+      a.f[q].data = uniform_values(plan->step_words) + q;
+      a.f[q].fdata = uniform_fvalues(plan->step_words) + q;
     }
   }
   if (d.stencil == FW_STENCIL_WEIGHTS) a.f[0].mode = plan->K;
