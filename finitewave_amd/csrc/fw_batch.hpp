@@ -55,7 +55,7 @@ struct BatchTissue {
 
 // A unit of the multi-step launch shape (fw_batch_tb.hpp): tissue, first
 // column of its 64-lane window, own columns [c0, c1) and own rows [r0, r1)
-// (16 bits each).
+// (16 bits each).  cols 0: the outer columns' nodes of the own rows.
 struct alignas(16) TbUnit {
   int32_t tissue;
   int32_t w0;
@@ -64,6 +64,7 @@ struct alignas(16) TbUnit {
 };
 
 constexpr int kTbWaves = kBlock / 64;  // units per block
+constexpr int kTbEdgeRows = 256;       // rows of an outer columns' unit: 8 nodes per lane
 
 struct TbLaunch {
   const TbUnit* __restrict__ units;  // this launch's units (of one stencil)

@@ -168,7 +168,14 @@ __device__ __forceinline__ void tb_march(const BatchArgs<R, R>& a, const BatchTi
 
   Row nxt = load(x_lo);
   int32_t x = x_lo;
-  (void)act_start;
+  // the two time constants an FP32 Mitchell-Schaeffer level selects from stay in
+  // vector registers: a select of two scalars first moves both into them, 2 of
+  // the level's 28 operations (512 tissues of 64 to 512 columns: 100 -> 98.6 us
+  // per step)
+  Params prm = a.P;
+  if constexpr (MODEL == 2 && sizeof(R) == 4) {
+    asm("" : "+v"(prm.f[5]), "+v"(prm.f[6]));
+  }
   auto body = [&](auto ph) -> bool {
     constexpr int PH = decltype(ph)::value;  // slot of row x
     if (x > x_end) return false;
@@ -211,7 +218,7 @@ __device__ __forceinline__ void tb_march(const BatchArgs<R, R>& a, const BatchTi
       R val;
       if constexpr (COEF) {
         const float uW = from_west(uc), uE = from_east(uc);
-        val = node_update<MODEL, R>(uc, s1, 0, a.dt, a.P, [&] {
+        val = node_update<MODEL, R>(uc, s1, 0, a.dt, prm, [&] {
           return tb_flux_iso(cf[sy], U[l][sN], uW, uE, U[l][sS], uc, a.s);
         });
       } else {
@@ -241,7 +248,7 @@ __device__ __forceinline__ void tb_march(const BatchArgs<R, R>& a, const BatchTi
         q.m[6] = (pS >> 8) & 1;
         q.m[7] = pS & 1;
         q.m[8] = (pS >> 16) & 1;
-        val = node_update<MODEL, R>(uc, s1, 0, a.dt, a.P, [&] {
+        val = node_update<MODEL, R>(uc, s1, 0, a.dt, prm, [&] {
           return diffuse9<R, EXACT>(stencil, dd, df, q, a.D, a.dtd, a.rdr2, a.s);
         });
       }
@@ -277,6 +284,32 @@ __device__ __forceinline__ void tb_march(const BatchArgs<R, R>& a, const BatchTi
   }
 }
 
+// K steps of the outer columns' nodes of rows [r0, r1): activation times and the
+// probe.  Both buffers and state sets hold the nodes' values since admission.
+template <typename R, int K>
+__device__ __forceinline__ void tb_edge(const BatchTissue& d, const int32_t ls0,
+                                        const int32_t phase, const int32_t r0, const int32_t r1) {
+  global_t<int32_t>* const act = (global_t<int32_t>*)d.act;
+  global_t<R>* const probe = (global_t<R>*)d.probe;
+  R thr;
+  if constexpr (sizeof(R) == 8) thr = d.act_thr;
+  else thr = d.act_thr_f;
+  // the launch's first step whose potentials are recorded
+  const int32_t first = ls0 > d.act_start ? ls0 : d.act_start;
+  const bool record = act && d.act_start >= 0 && first < ls0 + K;
+  const bool probing = probe && ls0 < d.probe_len;
+  if (!record && !probing) return;
+  const int32_t in_b = (ls0 & 1) ^ ((K % 2 == 0) ? phase : 0);
+  const global_t<R>* const u = (const global_t<R>*)(in_b ? d.un : d.u);
+  for (int32_t q = (int32_t)(threadIdx.x & 63); q < 2 * (r1 - r0); q += 64) {
+    const int32_t c = (r0 + (q >> 1)) * d.nj + (q & 1) * (d.nj - 1);
+    const R v = u[c];
+    if (record && v > thr && act[c] < 0) act[c] = first;
+    if (probing && c == d.probe_idx)
+      for (int32_t t = ls0; t < ls0 + K && t < d.probe_len; ++t) probe[t] = v;
+  }
+}
+
 template <int MODEL, typename R, int K, bool AN, bool NT>
 __global__ __launch_bounds__(kBlock) void k_batch_tb(const BatchArgs<R, R> a, const TbLaunch L) {
   const uint32_t b = blockIdx.x;
@@ -295,6 +328,10 @@ __global__ __launch_bounds__(kBlock) void k_batch_tb(const BatchArgs<R, R> a, co
   if (ls0 < 0) return;  // not admitted yet: the host launches no such unit
   const int32_t c0 = cols & 0xffff, c1 = (int32_t)((uint32_t)cols >> 16);
   const int32_t r0 = rows & 0xffff, r1 = (int32_t)((uint32_t)rows >> 16);
+  if (cols == 0) {
+    tb_edge<R, K>(d, ls0, L.phase, r0, r1);
+    return;
+  }
   if (d.act && d.act_start >= 0 && ls0 + K - 1 >= d.act_start)
     tb_march<MODEL, R, K, AN, NT, true>(a, d, ls0, L.phase, w0, c0, c1, r0, r1);
   else
