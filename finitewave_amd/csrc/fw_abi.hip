@@ -1432,7 +1432,8 @@ static void drop_tb_graphs(fw_batch* b) {
 // Builds the unit table of the active tissues for the multi-step variant
 // (the 5-point stencil's units first, then the 9-point stencil's).
 static int build_units(fw_batch* b, const int32_t* slots, int32_t n_slots, hipStream_t s) {
-  const int K = batch_tb_k(b->variant), rows = batch_tb_rows(b->variant);
+  const int K = batch_tb_k(b->variant);
+  const int rows = batch_tb_rows(b->variant);
   const int nst = model_n_state(b->model);
   int64_t n = 0;
   for (int32_t q = 0; q < n_slots; ++q) {
@@ -1448,8 +1449,25 @@ static int build_units(fw_batch* b, const int32_t* slots, int32_t n_slots, hipSt
                   "multi-step shapes need one", slots[q]);
         return FW_E_INVALID;
       }
-    tb_tissue_units(d, slots[q], K, rows, nullptr, &n);
   }
+  // The 5-point units' rows are halved until there are 3 wavefronts per SIMD
+  // (fewer leave the march's latency open), at most to 16 (the halo of 2K rows).
+  // FP32, us per step: 20 Mitchell-Schaeffer tissues of 64 to 512 columns 15.3 ->
+  // 7.4, 512 of 64 10.4 -> 7.1, 20 of Aliev-Panfilov of 128 to 1024 20.3 -> 19.4;
+  // 512 of 128 columns have 3072 units of 65 rows, 19.8, and would take 20.9
+  // halved twice.  The 9-point units, with more work per row, gain less than
+  // their halo costs.
+  int rows_iso = rows;
+  for (;; rows_iso /= 2) {
+    n = 0;
+    for (int32_t q = 0; q < n_slots; ++q)
+      if (b->host[slots[q]].stencil == FW_STENCIL_ISO)
+        tb_tissue_units(b->host[slots[q]], slots[q], K, rows_iso, nullptr, &n);
+    if (n == 0 || n >= kTbMinUnits || rows_iso <= kTbMinRows) break;
+  }
+  for (int32_t q = 0; q < n_slots; ++q)
+    if (b->host[slots[q]].stencil != FW_STENCIL_ISO)
+      tb_tissue_units(b->host[slots[q]], slots[q], K, rows, nullptr, &n);
   if (n > INT32_MAX / 8) {
     set_error("fw_batch_set_active: too many units");
     return FW_E_INVALID;
@@ -1464,7 +1482,7 @@ static int build_units(fw_batch* b, const int32_t* slots, int32_t n_slots, hipSt
     for (int32_t q = 0; q < n_slots; ++q) {
       const fw_tissue_desc& d = b->host[slots[q]];
       if ((d.stencil != FW_STENCIL_ISO) != (pass == 1)) continue;
-      tb_tissue_units(d, slots[q], K, rows, hu, &m);
+      tb_tissue_units(d, slots[q], K, pass == 0 ? rows_iso : rows, hu, &m);
       if (pass == 0) n_iso = m;
     }
   if (n > b->cap_units) {

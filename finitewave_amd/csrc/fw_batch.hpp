@@ -64,6 +64,7 @@ struct alignas(16) TbUnit {
 };
 
 constexpr int kTbWaves = kBlock / 64;  // units per block
+constexpr int kTbMinUnits = 3072, kTbMinRows = 16;
 constexpr int kTbEdgeRows = 256;       // rows of an outer columns' unit: 8 nodes per lane
 
 struct TbLaunch {
