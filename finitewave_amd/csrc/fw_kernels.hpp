@@ -893,17 +893,17 @@ __device__ __forceinline__ R diffuse(const KArgs<RA, R>& a, int64_t i, int64_t j
   }
 }
 
-// Waves per SIMD the compiler must leave room for.  The 2D TP06 steps hold 5:
-// FP64 then takes 96 registers and spills 7 (uniform-field instance; 1026^2,
-// 132.3 -> 127.4 us per step against 4 waves without spills; the compiler
-// alone would choose 3); FP32 takes 91-94 without spills.  The 3D FP64 LR91
-// steps hold 4, spilling 5 registers at most (131 x 115 x 147, per-node fibres,
-// 164 -> 148 us per step against the compiler's 3); with 4 the Bueno-Orovio
-// ones would spill 36 and more (90 -> 253 us).  Other steps keep the compiler's
-// choice.
+// Waves per SIMD the compiler must leave room for.  The 2D TP06 steps hold 4 in
+// FP64 (128 registers, 8 spilled; with the 5 that its former single update did
+// best with, 50 are and 1026^2 takes 113 us per step against 92) and 5 in FP32
+// (88 without spills).  The 3D FP64 LR91 steps hold 4 (131 x 115 x 147, per-node
+// fibres, 164 -> 148 us per step against the compiler's 3 when it was set); with
+// 4 the Bueno-Orovio ones would spill 36 and more (90 -> 253 us).  Other steps
+// keep the compiler's choice.
 template <int NDIM, int MODEL, int PREC>
 constexpr int step_min_waves() {
-  return (NDIM == 2 && MODEL == 6) ? 5 : (NDIM == 3 && PREC == 0 && MODEL == 5) ? 4 : 1;
+  if (NDIM == 2 && MODEL == 6) return PREC == 0 ? 4 : 5;
+  return NDIM == 3 && MODEL == 5 && PREC == 0 ? 4 : 1;
 }
 
 // 4 values of consecutive nodes, element-aligned: one vector load or store
@@ -1007,11 +1007,11 @@ __device__ __forceinline__ void step_node(const KArgs<R, UType<MODEL, R>>& a, in
         // FP32 flux form: the neighbourhood is loaded before the ionic
         // update, as in the batched step
         const Hood2<U> q = load_hood2<ST>(a, c, uc);
-        v = node_update<MODEL, R>(uc, a.st, c, a.dt, a.P, [&] {
+        v = node_update<MODEL, R, NDIM == 2>(uc, a.st, c, a.dt, a.P, [&] {
           return flux2d<ST, FL>(a, i, j, c, uc, q);
         });
       } else {
-        v = node_update<MODEL, R>(uc, a.st, c, a.dt, a.P, [&] {
+        v = node_update<MODEL, R, NDIM == 2>(uc, a.st, c, a.dt, a.P, [&] {
           return diffuse<NDIM, ST, R, U, PREC == 0, FL>(a, i, j, k, c, uc);
         });
       }
@@ -1244,7 +1244,7 @@ __global__ __launch_bounds__(kBlock) void k_ionic(UType<MODEL, R>* __restrict__ 
   const int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (q >= n) return;
   const int64_t c = idx[q];
-  u_new[c] = ionic_update<MODEL, R>(u[c], u_new[c], st, c, dt, P);
+  u_new[c] = ionic_update<MODEL, R, false>(u[c], u_new[c], st, c, dt, P);
 }
 
 template <typename R>

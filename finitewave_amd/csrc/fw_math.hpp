@@ -84,10 +84,12 @@ FW_HD inline double t128_exp_special(double x, double tmp, uint64_t sbits, uint6
   return 0x1p-1022 * y;
 }
 
-// tab: kExpTab, or a kernel's copy of it
-template <typename Tab>
-FW_HD inline double t128_exp_tab(double x, const Tab* tab) {
-  double kd = fma(mt::kInvLn2N, x, mt::kShift);
+// tab: kExpTab, or a kernel's copy of it; shift, c2, c4: kShift, kC2, kC4 (a
+// kernel keeps them in vector registers); CHECKED: x may be anything, else
+// |x| < 512
+template <bool CHECKED, typename Tab>
+FW_HD inline double t128_exp_with(double x, const Tab* tab, double shift, double c2, double c4) {
+  double kd = fma(mt::kInvLn2N, x, shift);
   const uint64_t ki = f64_bits(kd);
   kd -= mt::kShift;
   const double r = fma(kd, mt::kNegLn2loN, fma(kd, mt::kNegLn2hiN, x));
@@ -96,11 +98,16 @@ FW_HD inline double t128_exp_tab(double x, const Tab* tab) {
   const uint64_t sbits = tab[2 * j + 1] + (ki << 45);
   const double r2 = r * r;
   const double tmp =
-      fma(r2 * r2, fma(r, mt::kC5, mt::kC4), fma(r2, fma(r, mt::kC3, mt::kC2), tail + r));
-  if (__builtin_expect(!(__builtin_fabs(x) < 512.0), 0))  // |x| >= 512, inf, NaN
+      fma(r2 * r2, fma(r, mt::kC5, c4), fma(r2, fma(r, mt::kC3, c2), tail + r));
+  if (CHECKED && __builtin_expect(!(__builtin_fabs(x) < 512.0), 0))  // |x| >= 512, inf, NaN
     return t128_exp_special(x, tmp, sbits, ki);
   const double scale = f64_from(sbits);
   return fma(scale, tmp, scale);
+}
+
+template <typename Tab>
+FW_HD inline double t128_exp_tab(double x, const Tab* tab) {
+  return t128_exp_with<true>(x, tab, mt::kShift, mt::kC2, mt::kC4);
 }
 
 FW_HD inline double t128_exp(double x) { return t128_exp_tab(x, mt::kExpTab); }

@@ -69,6 +69,22 @@ __device__ __forceinline__ void exp_table_to_lds() {
 
 __device__ __forceinline__ double fexp(double x) { return t128_exp_tab(x, exp_lds()); }
 __device__ __forceinline__ float fexp(float x) { return __expf(x); }
+
+// The exp of a model's update: fexp with its three addends in vector registers
+// for the whole update (a fused multiply-add with two scalar constants moves one
+// into a vector register first, 6 of an exp's 46 operations).  !CHECKED: every
+// argument is below 512 in magnitude, and an exp is straight-line code.
+template <typename R, bool CHECKED = true, bool REGS = true>
+struct Exp {
+  double shift = mt::kShift, c2 = mt::kC2, c4 = mt::kC4;
+  __device__ __forceinline__ Exp() {
+    if constexpr (sizeof(R) == 8 && REGS) asm("" : "+v"(shift), "+v"(c2), "+v"(c4));
+  }
+  __device__ __forceinline__ R operator()(R x) const {
+    if constexpr (sizeof(R) == 8) return t128_exp_with<CHECKED>(x, exp_lds(), shift, c2, c4);
+    else return __expf(x);
+  }
+};
 __device__ __forceinline__ double flog(double x) { return dd_log(x); }
 __device__ __forceinline__ float flog(float x) { return __logf(x); }
 __device__ __forceinline__ double fsqrt(double x) { return sqrt(x); }
@@ -261,8 +277,8 @@ __host__ __device__ constexpr double state_offset(int model, int prec, int k) {
 // the conduction velocity with it.  Stored as d the stall band is half an ulp
 // of d over dt / tau (6.5e-6 for |d| < 0.031), and 1 - e taken from expm1
 // keeps the digits a float e would lose for slow gates.
-template <typename R>
-__device__ __forceinline__ R rl_gate(R d, R inf, R tau, R dt, R g0) {
+template <typename R, typename E>
+__device__ __forceinline__ R rl_gate(const E& fexp, R d, R inf, R tau, R dt, R g0) {
   if constexpr (sizeof(R) == 4) {
     const R em = -expm1f(-dt / tau);
     return d + ((inf - g0) - d) * em;
@@ -407,7 +423,8 @@ __device__ __forceinline__ R ionic_bo(R u, R un, SP& S, int64_t c,
 // FP64: bound by VALU issue and, on sheets of a wave or two per SIMD, by the
 // chain of dependent operations.  Divisions through dv and divc and the five
 // parameter-only logarithms and roots from the host: 291 x 259 iso 11.0 ->
-// 9.3 us per step, the same bits.
+// 9.3 us per step, the same bits; exps without their check, in straight-line code
+// (lr91_update<R, false>), 8.7 -> 7.4, 1026^2 40.5 -> 36.8.
 template <typename R>
 __device__ __forceinline__ R lr91_gate(R var, R dt, R alpha, R beta) {
   const R tau = dv(R(1), alpha + beta);
@@ -416,9 +433,9 @@ __device__ __forceinline__ R lr91_gate(R var, R dt, R alpha, R beta) {
   return var;
 }
 
-template <typename R, typename SP, typename U = R>
-__device__ __forceinline__ U ionic_lr91(U u_in, U un, SP& S, int64_t c, R dt,
-                                        const Params& P) {
+template <typename R, bool CHECKED, typename SP, typename U>
+__device__ __forceinline__ U lr91_update(U u_in, U un, SP& S, int64_t c, R dt, const Params& P) {
+  const Exp<R, CHECKED> fexp;
   const R u = (R)u_in;  // the potential in the arithmetic type
   const R gna = par<R>(P, 0), gsi = par<R>(P, 1), gk = par<R>(P, 2), gk1 = par<R>(P, 3),
           gkp = par<R>(P, 4), gb = par<R>(P, 5), ko = par<R>(P, 6), ki = par<R>(P, 7),
@@ -542,12 +559,26 @@ __device__ __forceinline__ U ionic_lr91(U u_in, U un, SP& S, int64_t c, R dt,
   return un - dt * (ina + isi + ik1t + ik);
 }
 
+template <typename R, typename SP, typename U = R>
+__device__ __forceinline__ U ionic_lr91(U u_in, U un, SP& S, int64_t c, R dt,
+                                        const Params& P) {
+  if constexpr (sizeof(R) == 8) {
+    // every exp argument is a function of u or of u - E_K1, at most 75 in
+    // magnitude for |u| <= 160 and 209 for |u - E_K1| <= 400: a wavefront of
+    // such nodes needs no exp's check
+    const bool safe = fabs(u_in) <= 160.0 && fabs(u_in - P.v[kLrEK1]) <= 400.0;
+    if (__builtin_expect(__all(safe), 1)) return lr91_update<R, false>(u_in, un, S, c, dt, P);
+  }
+  return lr91_update<R, true>(u_in, un, S, c, dt, P);
+}
+
 // ---- TP06  tp06_2d.py:242-1103 -----------------------------------------------
 // state order (tp06_2d.py:1073 call): cai casr cass nai Ki m h j xr1 xr2 xs r
 // s d f f2 fcass rr oo ; the first five are double in both precisions.
-template <typename R, typename SP, typename U = R>
-__device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
-                                        const Params& P) {
+template <typename R, bool SPLIT, bool CHECKED, typename SP, typename U>
+__device__ __forceinline__ U tp06_update(U u_in, U un, SP& S, int64_t c, R dt, const Params& P) {
+  const Exp<R, true, false> fexp;
+  const Exp<R, CHECKED, false> uexp;
   const R u = (R)u_in;  // the potential in the arithmetic type
   typedef double D;
   const R ko = par<R>(P, 0), cao = par<R>(P, 1), nao = par<R>(P, 2);
@@ -602,41 +633,41 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
     auto&& mr = ref<R>(S, 5, c);
     auto&& hr = ref<R>(S, 6, c);
     auto&& jr = ref<R>(S, 7, c);
-    const R alpha_m = dv(R(1.0), R(1.0) + fexp(divc(R(-60.0) - u, R(5.0))));
-    const R beta_m = dv(R(0.1), R(1.0) + fexp(divc(u + R(35.0), R(5.0)))) +
-                     dv(R(0.1), R(1.0) + fexp(divc(u - R(50.0), R(200.0))));
+    const R alpha_m = dv(R(1.0), R(1.0) + uexp(divc(R(-60.0) - u, R(5.0))));
+    const R beta_m = dv(R(0.1), R(1.0) + uexp(divc(u + R(35.0), R(5.0)))) +
+                     dv(R(0.1), R(1.0) + uexp(divc(u - R(50.0), R(200.0))));
     const R tau_m = alpha_m * beta_m;
-    const R m_inf = dv(R(1.0), (R(1.0) + fexp(divc(R(-56.86) - u, R(9.03)))) *
-                              (R(1.0) + fexp(divc(R(-56.86) - u, R(9.03)))));
+    const R m_inf = dv(R(1.0), (R(1.0) + uexp(divc(R(-56.86) - u, R(9.03)))) *
+                              (R(1.0) + uexp(divc(R(-56.86) - u, R(9.03)))));
     R alpha_h, beta_h;
     if (u >= R(-40.0)) {
       alpha_h = R(0.0);
-      beta_h = dv(R(0.77), R(0.13) * (R(1.0) + fexp(divc(-(u + R(10.66)), R(11.1)))));
+      beta_h = dv(R(0.77), R(0.13) * (R(1.0) + uexp(divc(-(u + R(10.66)), R(11.1)))));
     } else {
-      alpha_h = R(0.057) * fexp(divc(-(u + R(80.0)), R(6.8)));
-      beta_h = R(2.7) * fexp(R(0.079) * u) + R(310000.0) * fexp(R(0.3485) * u);
+      alpha_h = R(0.057) * uexp(divc(-(u + R(80.0)), R(6.8)));
+      beta_h = R(2.7) * uexp(R(0.079) * u) + R(310000.0) * uexp(R(0.3485) * u);
     }
     const R tau_h = dv(R(1.0), alpha_h + beta_h);
-    const R h_inf = dv(R(1.0), (R(1.0) + fexp(divc(u + R(71.55), R(7.43)))) *
-                              (R(1.0) + fexp(divc(u + R(71.55), R(7.43)))));
+    const R h_inf = dv(R(1.0), (R(1.0) + uexp(divc(u + R(71.55), R(7.43)))) *
+                              (R(1.0) + uexp(divc(u + R(71.55), R(7.43)))));
     R alpha_j, beta_j;
     if (u >= R(-40.0)) {
       alpha_j = R(0.0);
-      beta_j = dv(R(0.6) * fexp(R(0.057) * u),
-                R(1.0) + fexp(R(-0.1) * (u + R(32.0))));
+      beta_j = dv(R(0.6) * uexp(R(0.057) * u),
+                R(1.0) + uexp(R(-0.1) * (u + R(32.0))));
     } else {
-      alpha_j = dv((R(-25428.0) * fexp(R(0.2444) * u) -
-                    R(6.948e-06) * fexp(R(-0.04391) * u)) *
+      alpha_j = dv((R(-25428.0) * uexp(R(0.2444) * u) -
+                    R(6.948e-06) * uexp(R(-0.04391) * u)) *
                        (u + R(37.78)),
-                   R(1.0) + fexp(R(0.311) * (u + R(79.23))));
-      beta_j = dv(R(0.02424) * fexp(R(-0.01052) * u),
-                R(1.0) + fexp(R(-0.1378) * (u + R(40.14))));
+                   R(1.0) + uexp(R(0.311) * (u + R(79.23))));
+      beta_j = dv(R(0.02424) * uexp(R(-0.01052) * u),
+                R(1.0) + uexp(R(-0.1378) * (u + R(40.14))));
     }
     const R tau_j = dv(R(1.0), alpha_j + beta_j);
     const R j_inf = h_inf;
     const R m = m_inf - (m_inf - mr) * fexp(dv(-dt, tau_m));
-    const R hd = rl_gate<R>(hr, h_inf, tau_h, dt, kH0);
-    const R jd = rl_gate<R>(jr, j_inf, tau_j, dt, kJ0);
+    const R hd = rl_gate<R>(fexp, hr, h_inf, tau_h, dt, kH0);
+    const R jd = rl_gate<R>(fexp, jr, j_inf, tau_j, dt, kJ0);
     mr = m;
     hr = hd;
     jr = jd;
@@ -650,20 +681,20 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
     auto&& fr = ref<R>(S, 14, c);
     auto&& f2r = ref<R>(S, 15, c);
     auto&& fcr = ref<R>(S, 16, c);
-    const R d_inf = dv(R(1.0), R(1.0) + fexp(divc(R(-8) - u, R(7.5))));
-    const R Ad = dv(R(1.4), R(1.0) + fexp(divc(R(-35) - u, R(13)))) + R(0.25);
-    const R Bd = dv(R(1.4), R(1.0) + fexp(divc(u + R(5), R(5))));
-    const R Cd = dv(R(1.0), R(1.0) + fexp(divc(R(50) - u, R(20))));
+    const R d_inf = dv(R(1.0), R(1.0) + uexp(divc(R(-8) - u, R(7.5))));
+    const R Ad = dv(R(1.4), R(1.0) + uexp(divc(R(-35) - u, R(13)))) + R(0.25);
+    const R Bd = dv(R(1.4), R(1.0) + uexp(divc(u + R(5), R(5))));
+    const R Cd = dv(R(1.0), R(1.0) + uexp(divc(R(50) - u, R(20))));
     const R tau_d = Ad * Bd + Cd;
-    const R f_inf = dv(R(1.0), R(1.0) + fexp(divc(u + R(20), R(7))));
-    const R Af = R(1102.5) * fexp(divc(-(u + R(27)) * (u + R(27)), R(225)));
-    const R Bf = dv(R(200.0), R(1) + fexp(divc(R(13) - u, R(10.0))));
-    const R Cf = dv(R(180.0), R(1) + fexp(divc(u + R(30), R(10)))) + R(20);
+    const R f_inf = dv(R(1.0), R(1.0) + uexp(divc(u + R(20), R(7))));
+    const R Af = R(1102.5) * uexp(divc(-(u + R(27)) * (u + R(27)), R(225)));
+    const R Bf = dv(R(200.0), R(1) + uexp(divc(R(13) - u, R(10.0))));
+    const R Cf = dv(R(180.0), R(1) + uexp(divc(u + R(30), R(10)))) + R(20);
     const R tau_f = Af + Bf + Cf;
-    const R f2_inf = dv(R(0.67), R(1.0) + fexp(divc(u + R(35), R(7)))) + R(0.33);
-    const R Af2 = R(600) * fexp(divc(-(u + R(25)) * (u + R(25)), R(170)));
-    const R Bf2 = dv(R(31), R(1.0) + fexp(divc(R(25) - u, R(10))));
-    const R Cf2 = dv(R(16), R(1.0) + fexp(divc(u + R(30), R(10))));
+    const R f2_inf = dv(R(0.67), R(1.0) + uexp(divc(u + R(35), R(7)))) + R(0.33);
+    const R Af2 = R(600) * uexp(divc(-(u + R(25)) * (u + R(25)), R(170)));
+    const R Bf2 = dv(R(31), R(1.0) + uexp(divc(R(25) - u, R(10))));
+    const R Cf2 = dv(R(16), R(1.0) + uexp(divc(u + R(30), R(10))));
     const R tau_f2 = Af2 + Bf2 + Cf2;
     const R fcass_inf = dv(R(0.6), R(1) + divc(cass, R(0.05)) * divc(cass, R(0.05))) + R(0.4);
     const R tau_fcass = dv(R(80.0), R(1) + divc(cass, R(0.05)) * divc(cass, R(0.05))) + R(2.0);
@@ -692,11 +723,11 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
   {
     auto&& rr_ = ref<R>(S, 11, c);
     auto&& sr = ref<R>(S, 12, c);
-    const R r_inf = dv(R(1.0), R(1.0) + fexp(divc(R(20) - u, R(6.0))));
-    const R s_inf = dv(R(1.0), R(1.0) + fexp(divc(u + R(20), R(5.0))));
-    const R tau_r = R(9.5) * fexp(divc(-(u + R(40.0)) * (u + R(40.0)), R(1800.0))) + R(0.8);
-    const R tau_s = R(85.0) * fexp(divc(-(u + R(45.0)) * (u + R(45.0)), R(320.0))) +
-                    dv(R(5.0), R(1.0) + fexp(divc(u - R(20.0), R(5.0)))) + R(3.0);
+    const R r_inf = dv(R(1.0), R(1.0) + uexp(divc(R(20) - u, R(6.0))));
+    const R s_inf = dv(R(1.0), R(1.0) + uexp(divc(u + R(20), R(5.0))));
+    const R tau_r = R(9.5) * uexp(divc(-(u + R(40.0)) * (u + R(40.0)), R(1800.0))) + R(0.8);
+    const R tau_s = R(85.0) * uexp(divc(-(u + R(45.0)) * (u + R(45.0)), R(320.0))) +
+                    dv(R(5.0), R(1.0) + uexp(divc(u - R(20.0), R(5.0)))) + R(3.0);
     const R s = s_inf - (s_inf - sr) * fexp(dv(-dt, tau_s));
     const R r = r_inf - (r_inf - rr_) * fexp(dv(-dt, tau_r));
     sr = s;
@@ -708,13 +739,13 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
   {
     auto&& x1r = ref<R>(S, 8, c);
     auto&& x2r = ref<R>(S, 9, c);
-    const R xr1_inf = dv(R(1.0), R(1.0) + fexp(divc(R(-26.0) - u, R(7.0))));
-    const R axr1 = dv(R(450.0), R(1.0) + fexp(divc(R(-45.0) - u, R(10.0))));
-    const R bxr1 = dv(R(6.0), R(1.0) + fexp(divc(u - R(-30.0), R(11.5))));
+    const R xr1_inf = dv(R(1.0), R(1.0) + uexp(divc(R(-26.0) - u, R(7.0))));
+    const R axr1 = dv(R(450.0), R(1.0) + uexp(divc(R(-45.0) - u, R(10.0))));
+    const R bxr1 = dv(R(6.0), R(1.0) + uexp(divc(u - R(-30.0), R(11.5))));
     const R tau_xr1 = axr1 * bxr1;
-    const R xr2_inf = dv(R(1.0), R(1.0) + fexp(divc(u - R(-88.0), R(24.0))));
-    const R axr2 = dv(R(3.0), R(1.0) + fexp(divc(R(-60.0) - u, R(20.0))));
-    const R bxr2 = dv(R(1.12), R(1.0) + fexp(divc(u - R(60.0), R(20.0))));
+    const R xr2_inf = dv(R(1.0), R(1.0) + uexp(divc(u - R(-88.0), R(24.0))));
+    const R axr2 = dv(R(3.0), R(1.0) + uexp(divc(R(-60.0) - u, R(20.0))));
+    const R bxr2 = dv(R(1.12), R(1.0) + uexp(divc(u - R(60.0), R(20.0))));
     const R tau_xr2 = axr2 * bxr2;
     const R xr1 = xr1_inf - (xr1_inf - x1r) * fexp(dv(-dt, tau_xr1));
     const R xr2 = xr2_inf - (xr2_inf - x2r) * fexp(dv(-dt, tau_xr2));
@@ -726,10 +757,10 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
   R iks;
   {
     auto&& xsr = ref<R>(S, 10, c);
-    const R Axs = dv(R(1400.0), fsqrt(R(1.0) + fexp(divc(R(5.0) - u, R(6)))));
-    const R Bxs = dv(R(1.0), R(1.0) + fexp(divc(u - R(35.0), R(15.0))));
+    const R Axs = dv(R(1400.0), fsqrt(R(1.0) + uexp(divc(R(5.0) - u, R(6)))));
+    const R Bxs = dv(R(1.0), R(1.0) + uexp(divc(u - R(35.0), R(15.0))));
     const R tau_xs = Axs * Bxs + R(80);
-    const R xs_inf = dv(R(1.0), R(1.0) + fexp(divc(R(-5.0) - u, R(14.0))));
+    const R xs_inf = dv(R(1.0), R(1.0) + uexp(divc(R(-5.0) - u, R(14.0))));
     const R xs = xs_inf - (xs_inf - xsr) * fexp(dv(-dt, tau_xs));
     xsr = xs;
     iks = gks * xs * xs * (u - Eks);
@@ -753,7 +784,7 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
   const R inak =
       knak * par<R>(P, kTp06Derived + kKoOverKoKmK) * dv(nai, nai + KmNa) * rec_iNaK;
   const R ipca = dv(gpca * cai, KpCa + cai);
-  const R rec_ipK = dv(R(1.0), R(1.0) + fexp(divc(R(25) - u, R(5.98))));
+  const R rec_ipK = dv(R(1.0), R(1.0) + uexp(divc(R(25) - u, R(5.98))));
   const R ipk = gpk * rec_ipK * (u - Ek);
   const R ibna = gbna * (u - Ena);
   const R ibca = gbca * (u - Eca);
@@ -810,6 +841,22 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
                     inaca + ipca + ipk);
 }
 
+// SPLIT: the exps of a function of u only, at most 202 in magnitude for |u| <= 160,
+// without their check where a wavefront's nodes lie there: straight-line code
+// that overlaps their table reads, in a second copy of the update (126 against 96
+// registers: the 2D single-tissue step; 1026^2 95.6 -> 95.1 us per step, 300^2
+// 18.9 -> 17.2, 200^2 15.3 -> 12.9; a 3D block of 131 x 115 x 147 would lose 3 %
+// and a batch of four 24 %).
+template <typename R, bool SPLIT, typename SP, typename U = R>
+__device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
+                                        const Params& P) {
+  if constexpr (SPLIT && sizeof(R) == 8) {
+    if (__builtin_expect(__all(fabs(u_in) <= 160.0), 1))
+      return tp06_update<R, SPLIT, false>(u_in, un, S, c, dt, P);
+  }
+  return tp06_update<R, SPLIT, true>(u_in, un, S, c, dt, P);
+}
+
 // ---- Courtemanche  courtemanche_2d.py:180-641 -------------------------------
 // state order = the kernel's parameter order (courtemanche_2d.py:568-569):
 // nai ki cai caup carel m h j_ d f oa oi ua ui xs xr fca irel vrel urel wrel;
@@ -817,14 +864,15 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
 // FP64: bound by VALU issue.  Divisions through dv and div_recip, the
 // parameter-only quantities from the host and pow15 for the device pow:
 // 514 x 387, 10 % fibrosis, per-node fibres, 49.8 -> 37.6 us per step.
-template <typename R>
-__device__ __forceinline__ R crn_gate(R x, R x_inf, R tau_x, R dt) {
+template <typename R, typename E>
+__device__ __forceinline__ R crn_gate(const E& fexp, R x, R x_inf, R tau_x, R dt) {
   return x_inf - (x_inf - x) * fexp(dv(-dt, tau_x));
 }
 
-template <typename R, typename SP, typename U = R>
-__device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
-                                        const Params& P) {
+template <typename R, bool SPLIT, bool CHECKED, typename SP, typename U>
+__device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, const Params& P) {
+  const Exp<R, true, SPLIT> fexp;
+  const Exp<R, CHECKED, SPLIT> uexp;
   const R u = (R)u_in;  // the potential in the arithmetic type
   const R gna = par<R>(P, 0), gnab = par<R>(P, 1), gk1 = par<R>(P, 2), gks = par<R>(P, 4),
           gto = par<R>(P, 5), gcal = par<R>(P, 6), gcab = par<R>(P, 7),
@@ -868,13 +916,13 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
       if (u == R(-47.13)) {
         am = R(3.2);
       } else {
-        am = dv(R(0.32) * (u + R(47.13)), R(1) - fexp(R(-0.1) * (u + R(47.13))));
+        am = dv(R(0.32) * (u + R(47.13)), R(1) - uexp(R(-0.1) * (u + R(47.13))));
       }
     }
-    const R bm = R(0.08) * fexp(divc(-u, R(11)));
+    const R bm = R(0.08) * uexp(divc(-u, R(11)));
     const R m_inf = dv(am, am + bm);
     const R tau_m = dv(R(1), am + bm);
-    m = crn_gate<R>(mr, m_inf, tau_m, dt);
+    m = crn_gate<R>(fexp, mr, m_inf, tau_m, dt);
     mr = m;
   }
   {
@@ -882,14 +930,14 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
     R ah, bh;
     if (u >= R(-40)) {
       ah = R(0);
-      bh = dv(R(1), R(0.13) * (R(1) + fexp(divc(-(u + R(10.66)), R(11.1)))));
+      bh = dv(R(1), R(0.13) * (R(1) + uexp(divc(-(u + R(10.66)), R(11.1)))));
     } else {
-      ah = R(0.135) * fexp(divc(-(R(80) + u), R(6.8)));
-      bh = R(3.56) * fexp(R(0.079) * u) + R(310000) * fexp(R(0.35) * u);
+      ah = R(0.135) * uexp(divc(-(R(80) + u), R(6.8)));
+      bh = R(3.56) * uexp(R(0.079) * u) + R(310000) * uexp(R(0.35) * u);
     }
     const R h_inf = dv(ah, ah + bh);
     const R tau_h = dv(R(1), ah + bh);
-    h = crn_gate<R>(hr, h_inf, tau_h, dt);
+    h = crn_gate<R>(fexp, hr, h_inf, tau_h, dt);
     hr = h;
   }
   {
@@ -897,12 +945,12 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
     R aj, bj;
     if (u >= R(-40)) {
       aj = R(0);
-      bj = dv(R(0.3) * fexp(R(-2.535e-07) * u), R(1) + fexp(R(-0.1) * (u + R(32))));
+      bj = dv(R(0.3) * uexp(R(-2.535e-07) * u), R(1) + uexp(R(-0.1) * (u + R(32))));
     } else {
-      aj = dv((R(-127140) * fexp(R(0.2444) * u) - R(3.474e-05) * fexp(R(-0.04391) * u)) *
+      aj = dv((R(-127140) * uexp(R(0.2444) * u) - R(3.474e-05) * uexp(R(-0.04391) * u)) *
                   (u + R(37.78)),
-              R(1) + fexp(R(0.311) * (u + R(79.23))));
-      bj = dv(R(0.1212) * fexp(R(-0.01052) * u), R(1) + fexp(R(-0.1378) * (u + R(40.14))));
+              R(1) + uexp(R(0.311) * (u + R(79.23))));
+      bj = dv(R(0.1212) * uexp(R(-0.01052) * u), R(1) + uexp(R(-0.1378) * (u + R(40.14))));
     }
     const R j_inf = dv(aj, aj + bj);
     const R tau_j = dv(R(1), aj + bj);
@@ -910,22 +958,22 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
     jr = j;
   }
   const R ina = gna * (m * (m * m)) * h * j * (u - ena);
-  const R ik1 = dv(gk1 * (u - ek), R(1) + fexp(R(0.07) * (u + R(80))));
+  const R ik1 = dv(gk1 * (u - ek), R(1) + uexp(R(0.07) * (u + R(80))));
   // calc_ito
   R ito;
   {
     auto&& oar = ref<R>(S, 10, c);
     auto&& oir = ref<R>(S, 11, c);
-    const R ao = dv(R(0.65), fexp(divc(-(u + R(10)), R(8.5))) + fexp(divc(-(u - R(30)), R(59.0))));
-    const R bo = dv(R(0.65), R(2.5) + fexp(divc(u + R(82), R(17.0))));
+    const R ao = dv(R(0.65), uexp(divc(-(u + R(10)), R(8.5))) + uexp(divc(-(u - R(30)), R(59.0))));
+    const R bo = dv(R(0.65), R(2.5) + uexp(divc(u + R(82), R(17.0))));
     const R tau_o = dv(R(1), kq10 * (ao + bo));
-    const R o_inf = dv(R(1), R(1) + fexp(divc(-(u + R(20.47)), R(17.54))));
-    const R aoi = dv(R(1), R(18.53) + fexp(divc(u + R(113.7), R(10.95))));
-    const R boi = dv(R(1), R(35.56) + fexp(divc(-(u + R(1.26)), R(7.44))));
+    const R o_inf = dv(R(1), R(1) + uexp(divc(-(u + R(20.47)), R(17.54))));
+    const R aoi = dv(R(1), R(18.53) + uexp(divc(u + R(113.7), R(10.95))));
+    const R boi = dv(R(1), R(35.56) + uexp(divc(-(u + R(1.26)), R(7.44))));
     const R tau_oi = dv(R(1), kq10 * (aoi + boi));
-    const R oi_inf = dv(R(1), R(1) + fexp(divc(u + R(43.1), R(5.3))));
-    const R oa = crn_gate<R>(oar, o_inf, tau_o, dt);
-    const R oi = crn_gate<R>(oir, oi_inf, tau_oi, dt);
+    const R oi_inf = dv(R(1), R(1) + uexp(divc(u + R(43.1), R(5.3))));
+    const R oa = crn_gate<R>(fexp, oar, o_inf, tau_o, dt);
+    const R oi = crn_gate<R>(fexp, oir, oi_inf, tau_oi, dt);
     oar = oa;
     oir = oi;
     ito = gto * (oa * (oa * oa)) * oi * (u - ek);
@@ -935,17 +983,17 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
   {
     auto&& uar = ref<R>(S, 12, c);
     auto&& uir = ref<R>(S, 13, c);
-    const R gkur = R(0.005) + dv(R(0.05), R(1) + fexp(divc(-(u - R(15)), R(13.0))));
-    const R aua = dv(R(0.65), fexp(divc(-(u + R(10)), R(8.5))) + fexp(divc(-(u - R(30)), R(59.0))));
-    const R bua = dv(R(0.65), R(2.5) + fexp(divc(u + R(82), R(17.0))));
+    const R gkur = R(0.005) + dv(R(0.05), R(1) + uexp(divc(-(u - R(15)), R(13.0))));
+    const R aua = dv(R(0.65), uexp(divc(-(u + R(10)), R(8.5))) + uexp(divc(-(u - R(30)), R(59.0))));
+    const R bua = dv(R(0.65), R(2.5) + uexp(divc(u + R(82), R(17.0))));
     const R tau_ua = dv(R(1), kq10 * (aua + bua));
-    const R ua_inf = dv(R(1), R(1) + fexp(divc(-(u + R(30.3)), R(9.6))));
-    const R aui = dv(R(1), R(21) + fexp(divc(-(u - R(185)), R(28.0))));
-    const R bui = fexp(divc(u - R(158), R(16.0)));
+    const R ua_inf = dv(R(1), R(1) + uexp(divc(-(u + R(30.3)), R(9.6))));
+    const R aui = dv(R(1), R(21) + uexp(divc(-(u - R(185)), R(28.0))));
+    const R bui = uexp(divc(u - R(158), R(16.0)));
     const R tau_ui = dv(R(1), kq10 * (aui + bui));
-    const R ui_inf = dv(R(1), R(1) + fexp(divc(u - R(99.45), R(27.48))));
-    const R ua = crn_gate<R>(uar, ua_inf, tau_ua, dt);
-    const R ui = crn_gate<R>(uir, ui_inf, tau_ui, dt);
+    const R ui_inf = dv(R(1), R(1) + uexp(divc(u - R(99.45), R(27.48))));
+    const R ua = crn_gate<R>(fexp, uar, ua_inf, tau_ua, dt);
+    const R ui = crn_gate<R>(fexp, uir, ui_inf, tau_ui, dt);
     uar = ua;
     uir = ui;
     ikur = gkur_coeff * gkur * (ua * (ua * ua)) * ui * (u - ek);
@@ -960,14 +1008,14 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
       axr = R(0.0003 * 5) / exprel(-(u + R(14.1)) / R(5));
       bxr = R(7.3898e-05 * 5.1237) / exprel((u - R(3.3328)) / R(5.1237));
     } else {
-      axr = dv(R(0.0003) * (u + R(14.1)), R(1) - fexp(divc(-(u + R(14.1)), R(5))));
-      bxr = dv(R(7.3898e-05) * (u - R(3.3328)), fexp(divc(u - R(3.3328), R(5.1237))) - R(1));
+      axr = dv(R(0.0003) * (u + R(14.1)), R(1) - uexp(divc(-(u + R(14.1)), R(5))));
+      bxr = dv(R(7.3898e-05) * (u - R(3.3328)), uexp(divc(u - R(3.3328), R(5.1237))) - R(1));
     }
     const R tau_xr = dv(R(1), axr + bxr);
-    const R xr_inf = dv(R(1), R(1) + fexp(divc(-(u + R(14.1)), R(6.5))));
-    const R xr = crn_gate<R>(xrr, xr_inf, tau_xr, dt);
+    const R xr_inf = dv(R(1), R(1) + uexp(divc(-(u + R(14.1)), R(6.5))));
+    const R xr = crn_gate<R>(fexp, xrr, xr_inf, tau_xr, dt);
     xrr = xr;
-    ikr = dv(gkr * xr * (u - ek), R(1) + fexp(divc(u + R(15), R(22.4))));
+    ikr = dv(gkr * xr * (u - ek), R(1) + uexp(divc(u + R(15), R(22.4))));
   }
   // calc_iks on the kernel's xs slot (index 14)
   R iks;
@@ -978,12 +1026,12 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
       axs = R(4e-05 * 17) / exprel(-(u - R(19.9)) / R(17));
       bxs = R(3.5e-05 * 9) / exprel((u - R(19.9)) / R(9));
     } else {
-      axs = dv(R(4e-05) * (u - R(19.9)), R(1) - fexp(divc(-(u - R(19.9)), R(17))));
-      bxs = dv(R(3.5e-05) * (u - R(19.9)), fexp(divc(u - R(19.9), R(9))) - R(1));
+      axs = dv(R(4e-05) * (u - R(19.9)), R(1) - uexp(divc(-(u - R(19.9)), R(17))));
+      bxs = dv(R(3.5e-05) * (u - R(19.9)), uexp(divc(u - R(19.9), R(9))) - R(1));
     }
     const R tau_xs = dv(R(1), R(2) * (axs + bxs));
-    const R xs_inf = dv(R(1), fsqrt(R(1) + fexp(divc(-(u - R(19.9)), R(12.7)))));
-    const R xs = crn_gate<R>(xsr, xs_inf, tau_xs, dt);
+    const R xs_inf = dv(R(1), fsqrt(R(1) + uexp(divc(-(u - R(19.9)), R(12.7)))));
+    const R xs = crn_gate<R>(fexp, xsr, xs_inf, tau_xs, dt);
     xsr = xs;
     iks = gks * (xs * xs) * (u - ek);
   }
@@ -998,18 +1046,18 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
       const R y = -(u + R(10)) / R(6.24);
       tau_d = exprel(y) / (R(6.24 * 0.035) * (R(1) + fexp(y)));
     } else {
-      const R e = fexp(divc(-(u + R(10)), R(6.24)));
+      const R e = uexp(divc(-(u + R(10)), R(6.24)));
       tau_d = dv(R(1) - e, R(0.035) * (u + R(10)) * (R(1) + e));
     }
-    const R d_inf = dv(R(1), R(1) + fexp(divc(-(u + R(10)), R(8.0))));
-    const R tau_f = dv(R(9), R(0.0197) * fexp(-R(0.0337 * 0.0337) * ((u + R(10)) * (u + R(10)))) +
+    const R d_inf = dv(R(1), R(1) + uexp(divc(-(u + R(10)), R(8.0))));
+    const R tau_f = dv(R(9), R(0.0197) * uexp(-R(0.0337 * 0.0337) * ((u + R(10)) * (u + R(10)))) +
                                  R(0.02));
-    const R f_inf = dv(R(1), R(1) + fexp(divc(u + R(28), R(6.9))));
+    const R f_inf = dv(R(1), R(1) + uexp(divc(u + R(28), R(6.9))));
     const R tau_fca = R(2);
     const R fca_inf = dv(R(1), R(1) + divc(cai, R(0.00035)));
-    const R d = crn_gate<R>(dr, d_inf, tau_d, dt);
-    const R f = crn_gate<R>(fr, f_inf, tau_f, dt);
-    const R fca = crn_gate<R>(fcar, fca_inf, tau_fca, dt);
+    const R d = crn_gate<R>(fexp, dr, d_inf, tau_d, dt);
+    const R f = crn_gate<R>(fexp, fr, f_inf, tau_f, dt);
+    const R fca = crn_gate<R>(fexp, fcar, fca_inf, tau_fca, dt);
     dr = d;
     fr = f;
     fcar = fca;
@@ -1057,13 +1105,13 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
       const R y = -(u - R(7.9)) / R(5.0);
       tau_w = R(6.0 / 5.0) * exprel(y) / (R(1) + R(0.3) * fexp(y));
     } else {
-      const R e = fexp(divc(-(u - R(7.9)), R(5.0)));
+      const R e = uexp(divc(-(u - R(7.9)), R(5.0)));
       tau_w = dv(R(6) * (R(1) - e), (R(1) + R(0.3) * e) * (u - R(7.9)));
     }
-    const R w_inf = R(1) - dv(R(1), R(1) + fexp(divc(-(u - R(40)), R(17.0))));
-    const R urel = crn_gate<R>(urr, u_inf, tau_u, dt);
-    const R vrel = crn_gate<R>(vrr, v_inf, tau_v, dt);
-    const R wrel = crn_gate<R>(wrr, w_inf, tau_w, dt);
+    const R w_inf = R(1) - dv(R(1), R(1) + uexp(divc(-(u - R(40)), R(17.0))));
+    const R urel = crn_gate<R>(fexp, urr, u_inf, tau_u, dt);
+    const R vrel = crn_gate<R>(fexp, vrr, v_inf, tau_v, dt);
+    const R wrel = crn_gate<R>(fexp, wrr, w_inf, tau_w, dt);
     urr = urel;
     vrr = vrel;
     wrr = wrel;
@@ -1092,6 +1140,20 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
                     inaca + ibna + ibca);
 }
 
+// SPLIT: as TP06's; here the arguments stay below 75, and the 2D single-tissue
+// step takes 148 registers and 3 waves against 116 and 4 (1026^2 with 10 % of
+// fibrosis 98.0 -> 92.7 us per step, 500^2 30.1 -> 28.9, 200^2 14.6 -> 11.9; the 3D
+// block would lose 3 %).
+template <typename R, bool SPLIT, typename SP, typename U = R>
+__device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
+                                        const Params& P) {
+  if constexpr (SPLIT && sizeof(R) == 8) {
+    if (__builtin_expect(__all(fabs(u_in) <= 160.0), 1))
+      return crn_update<R, SPLIT, false>(u_in, un, S, c, dt, P);
+  }
+  return crn_update<R, SPLIT, true>(u_in, un, S, c, dt, P);
+}
+
 // u and u_new are stored as UType<MODEL, R>: the arithmetic type, except on
 // the FP32 path of the millivolt-scale models (LR91, TP06, Courtemanche),
 // whose potential is kept double.  There the step's increment dt * sum(I) at
@@ -1109,7 +1171,7 @@ __host__ __device__ constexpr bool u_is_f64(int model, int precision) {
 template <int MODEL, typename R>
 using UType = std::conditional_t<(sizeof(R) == 8 || MODEL >= 5), double, R>;
 
-template <int MODEL, typename R, typename SP, typename U>
+template <int MODEL, typename R, bool SPLIT, typename SP, typename U>
 __device__ __forceinline__ U ionic_update(U u, U un, SP& S, int64_t c, R dt,
                                           const Params& P) {
   if constexpr (MODEL == 0) return ionic_ap<R>(u, un, S, c, dt, P);
@@ -1118,8 +1180,8 @@ __device__ __forceinline__ U ionic_update(U u, U un, SP& S, int64_t c, R dt,
   else if constexpr (MODEL == 3) return ionic_fk<R>(u, un, S, c, dt, P);
   else if constexpr (MODEL == 4) return ionic_bo<R>(u, un, S, c, dt, P);
   else if constexpr (MODEL == 5) return ionic_lr91<R, SP, U>(u, un, S, c, dt, P);
-  else if constexpr (MODEL == 6) return ionic_tp06<R, SP, U>(u, un, S, c, dt, P);
-  else return ionic_crn<R, SP, U>(u, un, S, c, dt, P);
+  else if constexpr (MODEL == 6) return ionic_tp06<R, SPLIT, SP, U>(u, un, S, c, dt, P);
+  else return ionic_crn<R, SPLIT, SP, U>(u, un, S, c, dt, P);
 }
 
 // number of state arrays per model (state_vars minus u)
@@ -1137,14 +1199,15 @@ __host__ __device__ constexpr int model_n_state(int model) {
 // reference's value exactly.  FP32 builds fuse multiply-adds within one
 // expression only, so the single-tissue and batched kernels, which both use
 // this function, stay bit-identical.
-template <int MODEL, typename R, typename U, typename SP, typename Diffusion>
+template <int MODEL, typename R, bool SPLIT = false, typename U, typename SP,
+          typename Diffusion>
 __device__ __forceinline__ U node_update(U uc, SP& S, int64_t c, R dt, const Params& P,
                                          Diffusion&& diffusion) {
   if constexpr (MODEL >= 5) {
-    const U r = ionic_update<MODEL, R>(uc, U(0), S, c, dt, P);
+    const U r = ionic_update<MODEL, R, SPLIT>(uc, U(0), S, c, dt, P);
     return diffusion() + r;
   } else {
-    return ionic_update<MODEL, R>(uc, diffusion(), S, c, dt, P);
+    return ionic_update<MODEL, R, SPLIT>(uc, diffusion(), S, c, dt, P);
   }
 }
 
