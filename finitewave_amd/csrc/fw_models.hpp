@@ -843,9 +843,9 @@ __device__ __forceinline__ U tp06_update(U u_in, U un, SP& S, int64_t c, R dt, c
 
 // SPLIT: the exps of a function of u only, at most 202 in magnitude for |u| <= 160,
 // without their check where a wavefront's nodes lie there: straight-line code
-// that overlaps their table reads, in a second copy of the update (126 against 96
-// registers: the 2D single-tissue step; 1026^2 95.6 -> 95.1 us per step, 300^2
-// 18.9 -> 17.2, 200^2 15.3 -> 12.9; a 3D block of 131 x 115 x 147 would lose 3 %
+// that overlaps their table reads, in a second copy of the update (128 against 96
+// registers: the 2D single-tissue step; 1026^2 93.9 -> 91.8 us per step, 300^2
+// 18.9 -> 17.2, 200^2 15.2 -> 12.9; a 3D block of 131 x 115 x 147 would lose 3 %
 // and a batch of four 24 %).
 template <typename R, bool SPLIT, typename SP, typename U = R>
 __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
@@ -1142,7 +1142,7 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
 
 // SPLIT: as TP06's; here the arguments stay below 75, and the 2D single-tissue
 // step takes 148 registers and 3 waves against 116 and 4 (1026^2 with 10 % of
-// fibrosis 98.0 -> 92.7 us per step, 500^2 30.1 -> 28.9, 200^2 14.6 -> 11.9; the 3D
+// fibrosis 97.7 -> 93.0 us per step, 500^2 30.0 -> 28.9, 200^2 14.5 -> 11.8; the 3D
 // block would lose 3 %).
 template <typename R, bool SPLIT, typename SP, typename U = R>
 __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
