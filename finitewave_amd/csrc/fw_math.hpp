@@ -160,13 +160,16 @@ FW_HD inline double dd_log(double x) {
 }
 
 // 1/b as an unevaluated sum: hi = RN(1/b) and lo = RN(1/b - hi), from the exact
-// remainder 1 - b hi.
+// remainder 1 - b hi.  An infinite or zero b (a current or relaxation switched
+// off) has no remainder: with hi, 0 or infinite, for both halves div_recip gives
+// a/b.
 struct Recip {
   double hi, lo;
 };
 
 FW_HD inline Recip recip(double b) {
   const double hi = 1.0 / b;
+  if (hi == 0.0 || __builtin_fabs(hi) == HUGE_VAL) return Recip{hi, hi};
   return Recip{hi, __builtin_fma(-b, hi, 1.0) / b};
 }
 
