@@ -123,16 +123,20 @@ __device__ __forceinline__ R divc(R a, R b) {
 // quotients), wherever the full sequence would not rescale: a, b, 1/b and a/b
 // normal and their exponents less than 768 apart (the models' rates, gates,
 // concentrations and time constants stay far inside that while the state is
-// finite).  It differs for b infinite (NaN instead of 0) and for a = -0
-// (+0).  The TP06 update divides 76 times: with this and div_recip 1026^2 went
-// from 101.8 to 94.6 us per step.  FP32: the plain division.
-template <typename R>
+// finite).  It differs for b infinite (NaN instead of 0) or zero (NaN instead of
+// infinity) and for a = -0 (+0); FIX: the hardware's fix-up gives those as the
+// full division does, in a seventh operation.  The TP06 update divides 76 times:
+// with this and div_recip 1026^2 went from 101.8 to 94.6 us per step.  FP32: the
+// plain division.
+template <typename R, bool FIX = false>
 __device__ __forceinline__ R dv(R a, R b) {
   if constexpr (sizeof(R) == 8) {
     double r = __builtin_amdgcn_rcp(b);
     r = fma(fma(-b, r, 1.0), r, r);
-    const double q = a * r;
-    return fma(fma(-b, q, a), r, q);
+    double q = a * r;
+    q = fma(fma(-b, q, a), r, q);
+    if constexpr (FIX) q = __builtin_amdgcn_div_fixup(q, b, a);
+    return q;
   } else {
     return a / b;
   }
@@ -296,7 +300,7 @@ __device__ __forceinline__ R ionic_ap(R u, R un, SP& S, int64_t c,
   auto&& vref = ref<R>(S, 0, c);
   R v = vref;
   // calc_v: v += (-dt*(eap + (mu_1*v)/(mu_2 + u)) * (v + k*u*(u - a - 1.)))
-  v += (-dt * (eap + dv(mu_1 * v, mu_2 + u)) * (v + k * u * (u - a - R(1))));
+  v += (-dt * (eap + dv<R, true>(mu_1 * v, mu_2 + u)) * (v + k * u * (u - a - R(1))));
   vref = v;
   // u_new += dt*(-k*u*(u - a)*(u - 1.) - u*v)
   return un + dt * (-k * u * (u - a) * (u - R(1)) - u * v);
@@ -425,17 +429,19 @@ __device__ __forceinline__ R ionic_bo(R u, R un, SP& S, int64_t c,
 // parameter-only logarithms and roots from the host: 291 x 259 iso 11.0 ->
 // 9.3 us per step, the same bits; exps without their check, in straight-line code
 // (lr91_update<R, false>), 8.7 -> 7.4, 1026^2 40.5 -> 36.8.
-template <typename R>
+template <typename R, bool FIX>
 __device__ __forceinline__ R lr91_gate(R var, R dt, R alpha, R beta) {
-  const R tau = dv(R(1), alpha + beta);
-  const R inf = dv(alpha, alpha + beta);
-  var += dv(dt * (inf - var), tau);
+  const R tau = dv<R, FIX>(R(1), alpha + beta);
+  const R inf = dv<R, FIX>(alpha, alpha + beta);
+  var += dv<R, FIX>(dt * (inf - var), tau);
   return var;
 }
 
 template <typename R, bool CHECKED, typename SP, typename U>
 __device__ __forceinline__ U lr91_update(U u_in, U un, SP& S, int64_t c, R dt, const Params& P) {
   const Exp<R, CHECKED> fexp;
+  // a divisor is infinite or zero only where an exp overflows
+  auto udv = [](R a, R b) { return dv<R, CHECKED>(a, b); };
   const R u = (R)u_in;  // the potential in the arithmetic type
   const R gna = par<R>(P, 0), gsi = par<R>(P, 1), gk = par<R>(P, 2), gk1 = par<R>(P, 3),
           gkp = par<R>(P, 4), gb = par<R>(P, 5), ko = par<R>(P, 6), ki = par<R>(P, 7),
@@ -459,15 +465,15 @@ __device__ __forceinline__ U lr91_update(U u_in, U un, SP& S, int64_t c, R dt, c
   {
     R alpha_h = 0, beta_h = 0, beta_J = 0, alpha_J = 0;
     if (u >= R(-40.0)) {
-      beta_h = dv(R(1.0), R(0.13) * (R(1) + fexp(divc(u + R(10.66), R(-11.1)))));
-      beta_J = dv(R(0.3) * fexp(R(-2.535 * 1e-07) * u), R(1) + fexp(R(-0.1) * (u + R(32))));
+      beta_h = udv(R(1.0), R(0.13) * (R(1) + fexp(divc(u + R(10.66), R(-11.1)))));
+      beta_J = udv(R(0.3) * fexp(R(-2.535 * 1e-07) * u), R(1) + fexp(R(-0.1) * (u + R(32))));
     } else {
       alpha_h = R(0.135) * fexp(divc(R(80) + u, R(-6.8)));
       beta_h = R(3.56) * fexp(R(0.079) * u) +
                R(3.1 * 100000.0) * fexp(R(0.35) * u);
-      beta_J = dv(R(0.1212) * fexp(R(-0.01052) * u),
+      beta_J = udv(R(0.1212) * fexp(R(-0.01052) * u),
                   R(1) + fexp(R(-0.1378) * (u + R(40.14))));
-      alpha_J = dv((R(-1.2714 * 100000.0) * fexp(R(0.2444) * u) -
+      alpha_J = udv((R(-1.2714 * 100000.0) * fexp(R(0.2444) * u) -
                     R(3.474 * 1e-05) * fexp(R(-0.04391) * u)) *
                        (u + R(37.78)),
                    R(1) + fexp(R(0.311) * (u + R(79.23))));
@@ -476,11 +482,11 @@ __device__ __forceinline__ U lr91_update(U u_in, U un, SP& S, int64_t c, R dt, c
     if constexpr (sizeof(R) == 4)
       alpha_m = R(3.2) / exprel(R(-0.1) * (u + R(47.13)));
     else
-      alpha_m = dv(R(0.32) * (u + R(47.13)), R(1) - fexp(R(-0.1) * (u + R(47.13))));
+      alpha_m = udv(R(0.32) * (u + R(47.13)), R(1) - fexp(R(-0.1) * (u + R(47.13))));
     const R beta_m = R(0.08) * fexp(divc(-u, R(11)));
-    const R m = lr91_gate<R>(mr, dt, alpha_m, beta_m);
-    const R h = lr91_gate<R>(hr, dt, alpha_h, beta_h);
-    const R j = lr91_gate<R>(jr, dt, alpha_J, beta_J);
+    const R m = lr91_gate<R, CHECKED>(mr, dt, alpha_m, beta_m);
+    const R h = lr91_gate<R, CHECKED>(hr, dt, alpha_h, beta_h);
+    const R j = lr91_gate<R, CHECKED>(jr, dt, alpha_J, beta_J);
     mr = m;
     hr = h;
     jr = j;
@@ -492,16 +498,16 @@ __device__ __forceinline__ U lr91_update(U u_in, U un, SP& S, int64_t c, R dt, c
     R d = dr, f = fr, cai = cair;
     const R E_Si = R(7.7) - R(13.0287) * flog(cai);
     isi = gsi * d * f * (u - E_Si);
-    const R alpha_d = dv(R(0.095) * fexp(R(-0.01) * (u - R(5))),
+    const R alpha_d = udv(R(0.095) * fexp(R(-0.01) * (u - R(5))),
                          R(1) + fexp(R(-0.072) * (u - R(5))));
-    const R beta_d = dv(R(0.07) * fexp(R(-0.017) * (u + R(44))),
+    const R beta_d = udv(R(0.07) * fexp(R(-0.017) * (u + R(44))),
                         R(1) + fexp(R(0.05) * (u + R(44))));
-    const R alpha_f = dv(R(0.012) * fexp(R(-0.008) * (u + R(28))),
+    const R alpha_f = udv(R(0.012) * fexp(R(-0.008) * (u + R(28))),
                          R(1) + fexp(R(0.15) * (u + R(28))));
-    const R beta_f = dv(R(0.0065) * fexp(R(-0.02) * (u + R(30))),
+    const R beta_f = udv(R(0.0065) * fexp(R(-0.02) * (u + R(30))),
                         R(1) + fexp(R(-0.2) * (u + R(30))));
-    d = lr91_gate<R>(d, dt, alpha_d, beta_d);
-    f = lr91_gate<R>(f, dt, alpha_f, beta_f);
+    d = lr91_gate<R, CHECKED>(d, dt, alpha_d, beta_d);
+    f = lr91_gate<R, CHECKED>(f, dt, alpha_f, beta_f);
     cai += dt * (R(-0.0001) * isi + R(0.07) * (R(0.0001) - cai));
     dr = d;
     fr = f;
@@ -523,18 +529,18 @@ __device__ __forceinline__ U lr91_update(U u_in, U un, SP& S, int64_t c, R dt, c
       if constexpr (sizeof(R) == 4)
         Xi = R(2.837 * 0.04) * exprel(R(0.04) * (u + R(77))) / fexp(R(0.04) * (u + R(35)));
       else
-        Xi = dv(R(2.837) * (fexp(R(0.04) * (u + R(77))) - R(1)),
+        Xi = udv(R(2.837) * (fexp(R(0.04) * (u + R(77))) - R(1)),
                 (u + R(77)) * fexp(R(0.04) * (u + R(35))));
     } else {
       Xi = R(1);
     }
     const R x = xr;
     ik = G_K * x * Xi * (u - E_K);
-    const R alpha_x = dv(R(0.0005) * fexp(R(0.083) * (u + R(50))),
+    const R alpha_x = udv(R(0.0005) * fexp(R(0.083) * (u + R(50))),
                          R(1) + fexp(R(0.057) * (u + R(50))));
-    const R beta_x = dv(R(0.0013) * fexp(R(-0.06) * (u + R(20))),
+    const R beta_x = udv(R(0.0013) * fexp(R(-0.06) * (u + R(20))),
                         R(1) + fexp(R(-0.04) * (u + R(20))));
-    xr = lr91_gate<R>(x, dt, alpha_x, beta_x);
+    xr = lr91_gate<R, CHECKED>(x, dt, alpha_x, beta_x);
   }
   R E_K1, G_K1;
   if constexpr (F64) {
@@ -545,14 +551,14 @@ __device__ __forceinline__ U lr91_update(U u_in, U un, SP& S, int64_t c, R dt, c
     G_K1 = gk1 * fsqrt(ko / R(5.4));
   }
   // calc_ik1
-  const R alpha_K1 = dv(R(1.02), R(1) + fexp(R(0.2385) * (u - E_K1 - R(59.215))));
-  const R beta_K1 = dv(R(0.49124) * fexp(R(0.08032) * (u - E_K1 + R(5.476))) +
+  const R alpha_K1 = udv(R(1.02), R(1) + fexp(R(0.2385) * (u - E_K1 - R(59.215))));
+  const R beta_K1 = udv(R(0.49124) * fexp(R(0.08032) * (u - E_K1 + R(5.476))) +
                            fexp(R(0.06175) * (u - E_K1 - R(594.31))),
                        R(1) + fexp(R(-0.5143) * (u - E_K1 + R(4.753))));
-  const R K_1x = dv(alpha_K1, alpha_K1 + beta_K1);
+  const R K_1x = udv(alpha_K1, alpha_K1 + beta_K1);
   const R ik1 = G_K1 * K_1x * (u - E_K1);
   // calc_ikp, calc_ib
-  const R K_p = dv(R(1.0), R(1) + fexp(divc(R(7.488) - u, R(5.98))));
+  const R K_p = udv(R(1.0), R(1) + fexp(divc(R(7.488) - u, R(5.98))));
   const R ikp = gkp * K_p * (u - E_K1);
   const R ib = gb * (u + R(59.87));
   const R ik1t = ik1 + ikp + ib;
@@ -864,15 +870,20 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
 // FP64: bound by VALU issue.  Divisions through dv and div_recip, the
 // parameter-only quantities from the host and pow15 for the device pow:
 // 514 x 387, 10 % fibrosis, per-node fibres, 49.8 -> 37.6 us per step.
-template <typename R, typename E>
+template <typename R, bool FIX, typename E>
 __device__ __forceinline__ R crn_gate(const E& fexp, R x, R x_inf, R tau_x, R dt) {
-  return x_inf - (x_inf - x) * fexp(dv(-dt, tau_x));
+  return x_inf - (x_inf - x) * fexp(dv<R, FIX>(-dt, tau_x));
 }
 
 template <typename R, bool SPLIT, bool CHECKED, typename SP, typename U>
 __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, const Params& P) {
   const Exp<R, true, SPLIT> fexp;
   const Exp<R, CHECKED, SPLIT> uexp;
+  // udv: by a divisor of u alone, infinite or zero only where an exp overflows;
+  // fdv: by one that holds a parameter or the state, or (xr) that a node one ulp
+  // from its singularity makes zero
+  auto udv = [](R a, R b) { return dv<R, CHECKED>(a, b); };
+  auto fdv = [](R a, R b) { return dv<R, true>(a, b); };
   const R u = (R)u_in;  // the potential in the arithmetic type
   const R gna = par<R>(P, 0), gnab = par<R>(P, 1), gk1 = par<R>(P, 2), gks = par<R>(P, 4),
           gto = par<R>(P, 5), gcal = par<R>(P, 6), gcab = par<R>(P, 7),
@@ -896,9 +907,9 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
   constexpr bool F64 = sizeof(R) == 8;
   const R rtf = F64 ? par<R>(P, kCrnRTF) : R_ * T / F;
   const R rt2f = F64 ? par<R>(P, kCrnRT2F) : R_ * T / (R(2) * F);
-  const R ena = rtf * flog(dv(nao, nai));
-  const R ek = rtf * flog(dv(ko, ki));
-  const R eca = rt2f * flog(dv(cao, cai));
+  const R ena = rtf * flog(fdv(nao, nai));
+  const R ek = rtf * flog(fdv(ko, ki));
+  const R eca = rt2f * flog(fdv(cao, cai));
   // x / b for a uniform b whose reciprocal pair is derived parameter iq
   auto divu = [&](R x, R b, int iq) -> R {
     if constexpr (F64) return div_recip(x, par_recip(P, iq));
@@ -916,13 +927,13 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
       if (u == R(-47.13)) {
         am = R(3.2);
       } else {
-        am = dv(R(0.32) * (u + R(47.13)), R(1) - uexp(R(-0.1) * (u + R(47.13))));
+        am = udv(R(0.32) * (u + R(47.13)), R(1) - uexp(R(-0.1) * (u + R(47.13))));
       }
     }
     const R bm = R(0.08) * uexp(divc(-u, R(11)));
-    const R m_inf = dv(am, am + bm);
-    const R tau_m = dv(R(1), am + bm);
-    m = crn_gate<R>(fexp, mr, m_inf, tau_m, dt);
+    const R m_inf = udv(am, am + bm);
+    const R tau_m = udv(R(1), am + bm);
+    m = crn_gate<R, CHECKED>(fexp, mr, m_inf, tau_m, dt);
     mr = m;
   }
   {
@@ -930,14 +941,14 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
     R ah, bh;
     if (u >= R(-40)) {
       ah = R(0);
-      bh = dv(R(1), R(0.13) * (R(1) + uexp(divc(-(u + R(10.66)), R(11.1)))));
+      bh = udv(R(1), R(0.13) * (R(1) + uexp(divc(-(u + R(10.66)), R(11.1)))));
     } else {
       ah = R(0.135) * uexp(divc(-(R(80) + u), R(6.8)));
       bh = R(3.56) * uexp(R(0.079) * u) + R(310000) * uexp(R(0.35) * u);
     }
-    const R h_inf = dv(ah, ah + bh);
-    const R tau_h = dv(R(1), ah + bh);
-    h = crn_gate<R>(fexp, hr, h_inf, tau_h, dt);
+    const R h_inf = udv(ah, ah + bh);
+    const R tau_h = udv(R(1), ah + bh);
+    h = crn_gate<R, CHECKED>(fexp, hr, h_inf, tau_h, dt);
     hr = h;
   }
   {
@@ -945,35 +956,35 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
     R aj, bj;
     if (u >= R(-40)) {
       aj = R(0);
-      bj = dv(R(0.3) * uexp(R(-2.535e-07) * u), R(1) + uexp(R(-0.1) * (u + R(32))));
+      bj = udv(R(0.3) * uexp(R(-2.535e-07) * u), R(1) + uexp(R(-0.1) * (u + R(32))));
     } else {
-      aj = dv((R(-127140) * uexp(R(0.2444) * u) - R(3.474e-05) * uexp(R(-0.04391) * u)) *
+      aj = udv((R(-127140) * uexp(R(0.2444) * u) - R(3.474e-05) * uexp(R(-0.04391) * u)) *
                   (u + R(37.78)),
               R(1) + uexp(R(0.311) * (u + R(79.23))));
-      bj = dv(R(0.1212) * uexp(R(-0.01052) * u), R(1) + uexp(R(-0.1378) * (u + R(40.14))));
+      bj = udv(R(0.1212) * uexp(R(-0.01052) * u), R(1) + uexp(R(-0.1378) * (u + R(40.14))));
     }
-    const R j_inf = dv(aj, aj + bj);
-    const R tau_j = dv(R(1), aj + bj);
-    j = j_inf - (j_inf - jr) * fexp(dv(-dt, tau_j));
+    const R j_inf = udv(aj, aj + bj);
+    const R tau_j = udv(R(1), aj + bj);
+    j = j_inf - (j_inf - jr) * fexp(udv(-dt, tau_j));
     jr = j;
   }
   const R ina = gna * (m * (m * m)) * h * j * (u - ena);
-  const R ik1 = dv(gk1 * (u - ek), R(1) + uexp(R(0.07) * (u + R(80))));
+  const R ik1 = udv(gk1 * (u - ek), R(1) + uexp(R(0.07) * (u + R(80))));
   // calc_ito
   R ito;
   {
     auto&& oar = ref<R>(S, 10, c);
     auto&& oir = ref<R>(S, 11, c);
-    const R ao = dv(R(0.65), uexp(divc(-(u + R(10)), R(8.5))) + uexp(divc(-(u - R(30)), R(59.0))));
-    const R bo = dv(R(0.65), R(2.5) + uexp(divc(u + R(82), R(17.0))));
-    const R tau_o = dv(R(1), kq10 * (ao + bo));
-    const R o_inf = dv(R(1), R(1) + uexp(divc(-(u + R(20.47)), R(17.54))));
-    const R aoi = dv(R(1), R(18.53) + uexp(divc(u + R(113.7), R(10.95))));
-    const R boi = dv(R(1), R(35.56) + uexp(divc(-(u + R(1.26)), R(7.44))));
-    const R tau_oi = dv(R(1), kq10 * (aoi + boi));
-    const R oi_inf = dv(R(1), R(1) + uexp(divc(u + R(43.1), R(5.3))));
-    const R oa = crn_gate<R>(fexp, oar, o_inf, tau_o, dt);
-    const R oi = crn_gate<R>(fexp, oir, oi_inf, tau_oi, dt);
+    const R ao = udv(R(0.65), uexp(divc(-(u + R(10)), R(8.5))) + uexp(divc(-(u - R(30)), R(59.0))));
+    const R bo = udv(R(0.65), R(2.5) + uexp(divc(u + R(82), R(17.0))));
+    const R tau_o = fdv(R(1), kq10 * (ao + bo));
+    const R o_inf = udv(R(1), R(1) + uexp(divc(-(u + R(20.47)), R(17.54))));
+    const R aoi = udv(R(1), R(18.53) + uexp(divc(u + R(113.7), R(10.95))));
+    const R boi = udv(R(1), R(35.56) + uexp(divc(-(u + R(1.26)), R(7.44))));
+    const R tau_oi = fdv(R(1), kq10 * (aoi + boi));
+    const R oi_inf = udv(R(1), R(1) + uexp(divc(u + R(43.1), R(5.3))));
+    const R oa = crn_gate<R, true>(fexp, oar, o_inf, tau_o, dt);
+    const R oi = crn_gate<R, true>(fexp, oir, oi_inf, tau_oi, dt);
     oar = oa;
     oir = oi;
     ito = gto * (oa * (oa * oa)) * oi * (u - ek);
@@ -983,17 +994,18 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
   {
     auto&& uar = ref<R>(S, 12, c);
     auto&& uir = ref<R>(S, 13, c);
-    const R gkur = R(0.005) + dv(R(0.05), R(1) + uexp(divc(-(u - R(15)), R(13.0))));
-    const R aua = dv(R(0.65), uexp(divc(-(u + R(10)), R(8.5))) + uexp(divc(-(u - R(30)), R(59.0))));
-    const R bua = dv(R(0.65), R(2.5) + uexp(divc(u + R(82), R(17.0))));
-    const R tau_ua = dv(R(1), kq10 * (aua + bua));
-    const R ua_inf = dv(R(1), R(1) + uexp(divc(-(u + R(30.3)), R(9.6))));
-    const R aui = dv(R(1), R(21) + uexp(divc(-(u - R(185)), R(28.0))));
+    const R gkur = R(0.005) + udv(R(0.05), R(1) + uexp(divc(-(u - R(15)), R(13.0))));
+    const R aua =
+        udv(R(0.65), uexp(divc(-(u + R(10)), R(8.5))) + uexp(divc(-(u - R(30)), R(59.0))));
+    const R bua = udv(R(0.65), R(2.5) + uexp(divc(u + R(82), R(17.0))));
+    const R tau_ua = fdv(R(1), kq10 * (aua + bua));
+    const R ua_inf = udv(R(1), R(1) + uexp(divc(-(u + R(30.3)), R(9.6))));
+    const R aui = udv(R(1), R(21) + uexp(divc(-(u - R(185)), R(28.0))));
     const R bui = uexp(divc(u - R(158), R(16.0)));
-    const R tau_ui = dv(R(1), kq10 * (aui + bui));
-    const R ui_inf = dv(R(1), R(1) + uexp(divc(u - R(99.45), R(27.48))));
-    const R ua = crn_gate<R>(fexp, uar, ua_inf, tau_ua, dt);
-    const R ui = crn_gate<R>(fexp, uir, ui_inf, tau_ui, dt);
+    const R tau_ui = fdv(R(1), kq10 * (aui + bui));
+    const R ui_inf = udv(R(1), R(1) + uexp(divc(u - R(99.45), R(27.48))));
+    const R ua = crn_gate<R, true>(fexp, uar, ua_inf, tau_ua, dt);
+    const R ui = crn_gate<R, true>(fexp, uir, ui_inf, tau_ui, dt);
     uar = ua;
     uir = ui;
     ikur = gkur_coeff * gkur * (ua * (ua * ua)) * ui * (u - ek);
@@ -1008,14 +1020,14 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
       axr = R(0.0003 * 5) / exprel(-(u + R(14.1)) / R(5));
       bxr = R(7.3898e-05 * 5.1237) / exprel((u - R(3.3328)) / R(5.1237));
     } else {
-      axr = dv(R(0.0003) * (u + R(14.1)), R(1) - uexp(divc(-(u + R(14.1)), R(5))));
-      bxr = dv(R(7.3898e-05) * (u - R(3.3328)), uexp(divc(u - R(3.3328), R(5.1237))) - R(1));
+      axr = udv(R(0.0003) * (u + R(14.1)), R(1) - uexp(divc(-(u + R(14.1)), R(5))));
+      bxr = fdv(R(7.3898e-05) * (u - R(3.3328)), uexp(divc(u - R(3.3328), R(5.1237))) - R(1));
     }
-    const R tau_xr = dv(R(1), axr + bxr);
-    const R xr_inf = dv(R(1), R(1) + uexp(divc(-(u + R(14.1)), R(6.5))));
-    const R xr = crn_gate<R>(fexp, xrr, xr_inf, tau_xr, dt);
+    const R tau_xr = fdv(R(1), axr + bxr);
+    const R xr_inf = udv(R(1), R(1) + uexp(divc(-(u + R(14.1)), R(6.5))));
+    const R xr = crn_gate<R, true>(fexp, xrr, xr_inf, tau_xr, dt);
     xrr = xr;
-    ikr = dv(gkr * xr * (u - ek), R(1) + uexp(divc(u + R(15), R(22.4))));
+    ikr = udv(gkr * xr * (u - ek), R(1) + uexp(divc(u + R(15), R(22.4))));
   }
   // calc_iks on the kernel's xs slot (index 14)
   R iks;
@@ -1026,12 +1038,12 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
       axs = R(4e-05 * 17) / exprel(-(u - R(19.9)) / R(17));
       bxs = R(3.5e-05 * 9) / exprel((u - R(19.9)) / R(9));
     } else {
-      axs = dv(R(4e-05) * (u - R(19.9)), R(1) - uexp(divc(-(u - R(19.9)), R(17))));
-      bxs = dv(R(3.5e-05) * (u - R(19.9)), uexp(divc(u - R(19.9), R(9))) - R(1));
+      axs = udv(R(4e-05) * (u - R(19.9)), R(1) - uexp(divc(-(u - R(19.9)), R(17))));
+      bxs = udv(R(3.5e-05) * (u - R(19.9)), uexp(divc(u - R(19.9), R(9))) - R(1));
     }
-    const R tau_xs = dv(R(1), R(2) * (axs + bxs));
-    const R xs_inf = dv(R(1), fsqrt(R(1) + uexp(divc(-(u - R(19.9)), R(12.7)))));
-    const R xs = crn_gate<R>(fexp, xsr, xs_inf, tau_xs, dt);
+    const R tau_xs = udv(R(1), R(2) * (axs + bxs));
+    const R xs_inf = udv(R(1), fsqrt(R(1) + uexp(divc(-(u - R(19.9)), R(12.7)))));
+    const R xs = crn_gate<R, CHECKED>(fexp, xsr, xs_inf, tau_xs, dt);
     xsr = xs;
     iks = gks * (xs * xs) * (u - ek);
   }
@@ -1047,17 +1059,17 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
       tau_d = exprel(y) / (R(6.24 * 0.035) * (R(1) + fexp(y)));
     } else {
       const R e = uexp(divc(-(u + R(10)), R(6.24)));
-      tau_d = dv(R(1) - e, R(0.035) * (u + R(10)) * (R(1) + e));
+      tau_d = udv(R(1) - e, R(0.035) * (u + R(10)) * (R(1) + e));
     }
-    const R d_inf = dv(R(1), R(1) + uexp(divc(-(u + R(10)), R(8.0))));
-    const R tau_f = dv(R(9), R(0.0197) * uexp(-R(0.0337 * 0.0337) * ((u + R(10)) * (u + R(10)))) +
+    const R d_inf = udv(R(1), R(1) + uexp(divc(-(u + R(10)), R(8.0))));
+    const R tau_f = udv(R(9), R(0.0197) * uexp(-R(0.0337 * 0.0337) * ((u + R(10)) * (u + R(10)))) +
                                  R(0.02));
-    const R f_inf = dv(R(1), R(1) + uexp(divc(u + R(28), R(6.9))));
+    const R f_inf = udv(R(1), R(1) + uexp(divc(u + R(28), R(6.9))));
     const R tau_fca = R(2);
-    const R fca_inf = dv(R(1), R(1) + divc(cai, R(0.00035)));
-    const R d = crn_gate<R>(fexp, dr, d_inf, tau_d, dt);
-    const R f = crn_gate<R>(fexp, fr, f_inf, tau_f, dt);
-    const R fca = crn_gate<R>(fexp, fcar, fca_inf, tau_fca, dt);
+    const R fca_inf = fdv(R(1), R(1) + divc(cai, R(0.00035)));
+    const R d = crn_gate<R, CHECKED>(fexp, dr, d_inf, tau_d, dt);
+    const R f = crn_gate<R, CHECKED>(fexp, fr, f_inf, tau_f, dt);
+    const R fca = crn_gate<R, CHECKED>(fexp, fcar, fca_inf, tau_fca, dt);
     dr = d;
     fr = f;
     fcar = fca;
@@ -1066,9 +1078,9 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
   // calc_inak
   const R sig = F64 ? par<R>(P, kCrnSig) : R(1 / 7.0) * (fexp(nao / R(67.3)) - R(1));
   const R ko_km = F64 ? par<R>(P, kCrnKo) : ko / (ko + kmko);
-  const R fnak = dv(R(1), R(1) + R(0.1245) * fexp(overRT(R(-0.1) * (F * u))) +
+  const R fnak = fdv(R(1), R(1) + R(0.1245) * fexp(overRT(R(-0.1) * (F * u))) +
                               R(0.0365) * sig * fexp(overRT(-(F * u))));
-  const R inak = inakmax * fnak * dv(R(1), R(1) + fpow15(dv(kmnai, nai))) * ko_km;
+  const R inak = inakmax * fnak * fdv(R(1), R(1) + fpow15(fdv(kmnai, nai))) * ko_km;
   // calc_inaca
   const R gamma = R(0.35);
   const R exp_term = fexp(overRT(gamma * (F * u)));
@@ -1080,10 +1092,10 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
   const R term2 = kmcancx + cao;
   const R term12 = F64 ? par<R>(P, kCrnT12) : term1 * term2;
   const R term3 = R(1) + ksatncx * exp_rev_term;
-  const R inaca = dv(numerator, term12 * term3);
+  const R inaca = fdv(numerator, term12 * term3);
   const R ibca = gcab * (u - eca);
   const R ibna = gnab * (u - ena);
-  const R ipca = dv(ipcamax * cai, cai + R(0.0005));
+  const R ipca = fdv(ipcamax * cai, cai + R(0.0005));
   // calc_irel (uses the irel stored by the previous step)
   R irel;
   {
@@ -1106,12 +1118,12 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
       tau_w = R(6.0 / 5.0) * exprel(y) / (R(1) + R(0.3) * fexp(y));
     } else {
       const R e = uexp(divc(-(u - R(7.9)), R(5.0)));
-      tau_w = dv(R(6) * (R(1) - e), (R(1) + R(0.3) * e) * (u - R(7.9)));
+      tau_w = udv(R(6) * (R(1) - e), (R(1) + R(0.3) * e) * (u - R(7.9)));
     }
-    const R w_inf = R(1) - dv(R(1), R(1) + uexp(divc(-(u - R(40)), R(17.0))));
-    const R urel = crn_gate<R>(fexp, urr, u_inf, tau_u, dt);
-    const R vrel = crn_gate<R>(fexp, vrr, v_inf, tau_v, dt);
-    const R wrel = crn_gate<R>(fexp, wrr, w_inf, tau_w, dt);
+    const R w_inf = R(1) - udv(R(1), R(1) + uexp(divc(-(u - R(40)), R(17.0))));
+    const R urel = crn_gate<R, CHECKED>(fexp, urr, u_inf, tau_u, dt);
+    const R vrel = crn_gate<R, CHECKED>(fexp, vrr, v_inf, tau_v, dt);
+    const R wrel = crn_gate<R, CHECKED>(fexp, wrr, w_inf, tau_w, dt);
     urr = urel;
     vrr = vrel;
     wrr = wrel;
@@ -1121,7 +1133,7 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
   auto overFVj = [&](R x) -> R { return divu(x, F * Vj, kCrnInvFVj); };
   const R vrel_vup = F64 ? par<R>(P, kCrnVrelVup) : Vrel / Vup;
   const R itr = divc(caup - carel, R(180));
-  const R iup = dv(iupmax, R(1) + dv(kup, cai));
+  const R iup = fdv(iupmax, R(1) + fdv(kup, cai));
   const R iupleak = divu(caup, caupmax, kCrnInvCaup) * iupmax;
   caupr = caup + dt * (iup - iupleak - itr * vrel_vup);
   nair = nai + dt * overFVj(R(-3) * inak - R(3) * inaca - ibna - ina);
@@ -1130,11 +1142,11 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
     const R B1 = divu(R(2) * inaca - ipca - ical - ibca,
                       R(2) * F * Vj, kCrnInv2FVj) +
                  divu(Vup * (iupleak - iup) + irel * Vrel, Vj, kCrnInvVj);
-    const R B2 = R(1) + dv(trpnmax * kmtrpn, (cai + kmtrpn) * (cai + kmtrpn)) +
-                 dv(cmdnmax * kmcmdn, (cai + kmcmdn) * (cai + kmcmdn));
-    cair = cai + dt * dv(B1, B2);
+    const R B2 = R(1) + fdv(trpnmax * kmtrpn, (cai + kmtrpn) * (cai + kmtrpn)) +
+                 fdv(cmdnmax * kmcmdn, (cai + kmcmdn) * (cai + kmcmdn));
+    cair = cai + dt * fdv(B1, B2);
   }
-  carelr = carel + dt * dv(itr - irel, R(1) + dv(csqnmax * kmcsqn,
+  carelr = carel + dt * fdv(itr - irel, R(1) + fdv(csqnmax * kmcsqn,
                                                  (carel + kmcsqn) * (carel + kmcsqn)));
   return un - dt * (ina + ik1 + ito + ikur + ikr + iks + ical + ipca + inak +
                     inaca + ibna + ibca);
