@@ -503,11 +503,20 @@ int fw_plan_create(const fw_plan_desc* desc, fw_plan** out) {
   const int64_t N = p->N;
   const size_t alt = multi_alt_bytes(p);
   hipError_t e = hipMalloc(&p->step_words, kStepWordBytes + alt);
-  if (e == hipSuccess && alt) p->alt = reinterpret_cast<char*>(p->step_words) + kStepWordBytes;
   if (e != hipSuccess) {
     set_error("fw_plan_create: hipMalloc failed: %s", hipGetErrorString(e));
     delete p;
     return FW_E_NOMEM;
+  }
+  if (alt) {
+    p->alt = reinterpret_cast<char*>(p->step_words) + kStepWordBytes;
+    e = hipEventCreateWithFlags(&p->alt_event, hipEventDisableTiming);
+    if (e != hipSuccess) {
+      set_error("fw_plan_create: event creation failed: %s", hipGetErrorString(e));
+      p->alt_event = nullptr;
+      fw_plan_destroy(p);
+      return FW_E_HIP;
+    }
   }
   // a kernel computing the diffusion in float reads float copies of the
   // tables: 4-byte loads and no conversion per node
@@ -608,6 +617,7 @@ static void drop_graphs(fw_plan* plan) {
 int fw_plan_destroy(fw_plan* plan) {
   if (!plan) return FW_OK;
   drop_graphs(plan);
+  if (plan->alt_event) (void)hipEventDestroy(plan->alt_event);
   if (plan->step_words) (void)hipFree(plan->step_words);
   for (int q = 0; q < FW_MAX_FIELDS; ++q) {
     if (plan->ftab[q]) (void)hipFree(plan->ftab[q]);
@@ -677,23 +687,52 @@ static int run_plain(const fw_plan* plan, void* u, void* u_new, void* const* sta
   return FW_OK;
 }
 
-// Whether the multi-step launches may use the plan's second state set on
-// `stream`.  One set cannot serve two runs in flight: it goes to the first
-// stream that asks, whose calls are ordered, and runs of the plan on any other
-// stream keep to single steps, as does a stream being captured (its graph may
-// be replayed on any stream) and the per-thread stream (one handle, a stream
-// per thread).
-static bool multi_stream_ok(fw_plan* plan, hipStream_t s) {
+// Whether a run on `s` may use the plan's second state set; the caller holds
+// alt_mutex.  A pair of launches writes the set and reads it again, so two runs
+// may share it only one after the other: in the order of one stream, or once the
+// last run's event has completed, which is polled and never waited for on the
+// host.  The default stream's event is recorded when another stream asks (its handle
+// is always good), any other's after each run, as the handle may be gone by then: a
+// record costs 3 us per run.  A handle equal to the last run's may be a new
+// stream's after the old one was destroyed, hence the wait on the device (none at
+// all for the runtime when it is the event's own stream).  A stream being captured
+// keeps to single steps (its graph may be replayed on any stream), as does the
+// per-thread stream (one handle, a stream per thread).
+static bool alt_open(fw_plan* plan, hipStream_t s) {
   if (s == hipStreamPerThread) return false;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
     return false;
   }
-  uintptr_t none = 0;
-  const uintptr_t me = reinterpret_cast<uintptr_t>(s) + 1;
-  return plan->alt_stream.compare_exchange_strong(none, me) || none == me;
+  if (!plan->alt_used || (s == nullptr && plan->alt_stream == nullptr)) return true;
+  if (!plan->alt_marked && (plan->alt_stream != nullptr ||
+                            hipEventRecord(plan->alt_event, plan->alt_stream) != hipSuccess)) {
+    (void)hipGetLastError();
+    return false;
+  }
+  plan->alt_marked = true;
+  const hipError_t e = hipEventQuery(plan->alt_event);
+  if (e == hipSuccess) return true;
+  (void)hipGetLastError();
+  return e == hipErrorNotReady && s == plan->alt_stream &&
+         hipStreamWaitEvent(s, plan->alt_event, 0) == hipSuccess;
 }
+
+// A run's use of the second state set: marked at its end, also when a launch of
+// it failed.
+struct AltUse {
+  fw_plan* plan;
+  AltUse(fw_plan* p, hipStream_t s) : plan(p) {
+    p->alt_used = true;
+    p->alt_stream = s;
+    p->alt_marked = false;
+  }
+  ~AltUse() {
+    if (plan->alt_stream != nullptr)
+      plan->alt_marked = hipEventRecord(plan->alt_event, plan->alt_stream) == hipSuccess;
+  }
+};
 
 // Steps per launch (K) and region rows of a sheet's multi-step launches; K = 0
 // where single steps are the faster.  A launch costs about 5 us before its
@@ -795,7 +834,11 @@ static int run_multi(fw_plan* plan, void* u, void* u_new, void* const* state, in
       if (r0 >= 0 ? track->probe_rows[q] != r0 + q : track->probe_rows[q] >= 0) return FW_OK;
     probes = r0 >= 0;
   }
-  if (!multi_stream_ok(plan, s)) return FW_OK;
+  // runs of the plan enqueued by two threads at once would interleave their
+  // pairs: the second takes single steps
+  const std::unique_lock<std::mutex> hold(plan->alt_mutex, std::try_to_lock);
+  if (!hold.owns_lock() || !alt_open(plan, s)) return FW_OK;
+  const AltUse use(plan, s);
   *done = true;
   const int64_t stim_end = track ? track->stim_end : 0;
   const MultiLauncher L = multi_launcher(plan->desc.precision, plan->desc.model);

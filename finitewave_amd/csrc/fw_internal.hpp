@@ -4,7 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <atomic>
+#include <mutex>
 
 #include "../../include/finitewave_amd.h"
 #include "fw_models.hpp"
@@ -47,10 +47,14 @@ struct fw_plan {
   double* ktab[FW_MAX_FIELDS];
   float* fktab[FW_MAX_FIELDS];
   // the second state set of the multi-step launches (fw_multi2d.hpp), in the
-  // allocation of step_words; null for plans without them.  It belongs to the
-  // first stream that uses it (fw_abi.hip, multi_stream_ok)
+  // allocation of step_words; null for plans without them.  One run at a time
+  // uses it (fw_abi.hip, alt_open)
   void* alt;
-  std::atomic<uintptr_t> alt_stream;  // that stream's handle + 1; 0 while none
+  std::mutex alt_mutex;    // held while a run that uses it is enqueued; guards:
+  hipStream_t alt_stream;  // the stream of the last such run
+  hipEvent_t alt_event;    // after it, once recorded
+  bool alt_used;           // there was one
+  bool alt_marked;         // its event is recorded
 };
 
 namespace fw {

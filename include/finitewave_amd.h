@@ -230,8 +230,11 @@ int fw_plan_set_weights_k(fw_plan* plan, int32_t K);
  * writes `u_new`, then the two swap; after an odd n_steps the result is in
  * the buffer passed as u_new.  state: host array of device pointers.
  * Plans with a second state set take several steps per launch where that is
- * faster (the same bits); the set serves the first stream that uses it, runs
- * of the plan on other streams keep to one step per launch. */
+ * faster (the same bits).  The set serves one run at a time: a run on another
+ * stream than the last one's, before that has completed on the device, and a run
+ * enqueued while another thread enqueues one keep to one step per launch.  So
+ * fw_run calls on one plan with different buffers may overlap, on any streams
+ * and threads. */
 int fw_run(fw_plan* plan, void* u, void* u_new, void* const* state,
            int64_t step0, int32_t n_steps, const fw_track_desc* track,
            void* stream);
