@@ -876,6 +876,7 @@ static int run_multi(fw_plan* plan, void* u, void* u_new, void* const* state, in
     const int64_t to = stim_until(plan, step + 1, step0 + n_steps, stim_end);
     int32_t n = (int32_t)(to - step);
     if (room > 0 && n < room + 1) n = room + 1;
+    n += n % 2;  // the buffers keep their roles, so graphs of one orientation serve
     if (n > n_steps - pos) n = n_steps - pos;
     fw_track_desc sub{};
     if (track) {
@@ -1105,10 +1106,11 @@ static int check_graph_args(fw_plan* plan, void* u, void* u_new, void* const* st
 
 // The graph set fw_run_graph replays for these buffers, tracker and schedule
 // (the plan's schedule is in every captured kernel's arguments; changing it
-// drops the graphs), with the graphs an n_steps run needs captured.
+// drops the graphs), with the graphs `pairs` pairs of steps need captured; the
+// tracker's gate is checked over n_steps.
 static int ensure_graphs(fw_plan* plan, void* u, void* u_new, void* const* state,
-                         int32_t n_steps, const fw_track_desc* track, int32_t* act_on_out,
-                         fw_plan::GraphSet** set_out) {
+                         int32_t n_steps, int32_t pairs, const fw_track_desc* track,
+                         int32_t* act_on_out, fw_plan::GraphSet** set_out) {
   int32_t act_on = 0;
   int rc = check_graph_args(plan, u, u_new, state, n_steps, track, &act_on);
   if (rc) return rc;
@@ -1143,7 +1145,6 @@ static int ensure_graphs(fw_plan* plan, void* u, void* u_new, void* const* state
     gs->un = u_new;
   }
   gs->last_use = ++plan->graph_clock;
-  const int32_t pairs = n_steps / 2;
   const StatePtrs st = make_state(state, ns);
   for (int bit = 0; bit < kGraphBits; ++bit) {
     const int32_t size = 1 << bit;
@@ -1161,10 +1162,11 @@ int fw_run_graph_prepare(fw_plan* plan, void* u, void* u_new, void* const* state
                          int32_t n_steps, const fw_track_desc* track) {
   int32_t act_on = 0;
   fw_plan::GraphSet* gs = nullptr;
-  // multi-step plans replay graphs only across long stimuli
-  if (plan && plan->alt && plan->n_stims == 0)
-    return check_graph_args(plan, u, u_new, state, n_steps, track, &act_on);
-  return ensure_graphs(plan, u, u_new, state, n_steps, track, &act_on, &gs);
+  // a multi-step plan replays graphs across stimuli of any length, and for the
+  // whole run while another one has its second state set: every size then
+  const bool any = plan && plan->alt && n_steps >= kMultiGraphSteps;
+  return ensure_graphs(plan, u, u_new, state, n_steps,
+                       any ? (1 << kGraphBits) - 1 : n_steps / 2, track, &act_on, &gs);
 }
 
 // n_steps single steps: pairs of steps replayed from graphs, an odd last one
@@ -1173,9 +1175,9 @@ static int run_graphs(fw_plan* plan, void* u, void* u_new, void* const* state, i
                       int32_t n_steps, const fw_track_desc* track, void* stream) {
   int32_t act_on = 0;
   fw_plan::GraphSet* gs = nullptr;
-  int rc = ensure_graphs(plan, u, u_new, state, n_steps, track, &act_on, &gs);
-  if (rc) return rc;
   const int32_t pairs = n_steps / 2;
+  int rc = ensure_graphs(plan, u, u_new, state, n_steps, pairs, track, &act_on, &gs);
+  if (rc) return rc;
   hipStream_t s = as_stream(stream);
   if (pairs > 0) {
     hipLaunchKernelGGL(k_set_run_words, dim3(1), dim3(1), 0, s, plan->step_words,
