@@ -465,13 +465,19 @@ constexpr int64_t kMultiMaxNodes = (int64_t)1 << 22;
 constexpr int64_t kMultiMaxTanh = (int64_t)1 << 18;
 constexpr int32_t kMultiGraphSteps = 64;
 
+static void multi_shape(const fw_plan* plan, int32_t* K, int32_t* rows);
+
 // Bytes of a plan's second state set, 0 for plans without multi-step launches
-// (fw_multi2d.hpp): 2D, light models, uniform half-step fields.
+// (fw_multi2d.hpp): 2D, light models, uniform half-step fields, a size at which
+// they are the faster.
 static size_t multi_alt_bytes(const fw_plan* p) {
   const fw_plan_desc& d = p->desc;
   if (d.ndim != 2 || d.model > 4 || d.stencil == FW_STENCIL_WEIGHTS ||
       p->field_layout != fw::kFieldsUniform || p->N > kMultiMaxNodes)
     return 0;
+  int32_t K, rows;
+  multi_shape(p, &K, &rows);
+  if (K == 0) return 0;
   return (size_t)p->N * model_n_state(d.model) *
          (d.precision == FW_PREC_FP64 ? sizeof(double) : sizeof(float));
 }
