@@ -275,16 +275,16 @@ class CardiacModel:
         dt = self.dt
         # stimuli on the device schedule: their steps need no host event
         sched = self._schedule_stims(eng, stims, iters)
-        look = self._can_look_ahead(trackers)
         done, calm = 0, 0
         while done < iters:
-            if look and calm >= _LOOK_AFTER:
+            # asked anew each time: a command may have changed what it rests on
+            if calm >= _LOOK_AFTER and self._can_look_ahead(dt, trackers):
                 calm = 0
                 if len(chunk_flags) == 0:
                     chunk_start[0] = self.step
                 ask = min(iters - done, _CHUNK - len(chunk_flags),
                           _LOOK_AHEAD if len(chunk_flags) < _LOOK_AHEAD else _CHUNK)
-                ahead = self._look_ahead(ask, stims, commands, fused_act, probe_trackers,
+                ahead = self._look_ahead(ask, dt, stims, commands, fused_act, probe_trackers,
                                          extra_act + host_trackers + dev_trackers)
                 n = len(ahead[0])
                 if n:
@@ -400,23 +400,23 @@ class CardiacModel:
         if bar is not None:
             bar.close()
 
-    def _can_look_ahead(self, trackers) -> bool:
-        """Whether the loop may resolve event-free steps in bulk: the time
+    def _can_look_ahead(self, dt, trackers) -> bool:
+        """Whether the loop may resolve event-free steps of dt in bulk: the time
         fold, gates and termination rule are the package's own."""
-        return (isinstance(self.dt, float) and not self.state_saver and
+        return (isinstance(dt, float) and not self.state_saver and
                 type(self).check_termination is CardiacModel.check_termination and
                 "check_termination" not in self.__dict__ and
                 all(type(tr.step) is int and tr.step > 0 for tr in trackers))
 
-    def _look_ahead(self, n, stims, commands, fused_act, probe_trackers, event_trackers):
-        """The event-free steps among the next n: (activation flags, a gate
+    def _look_ahead(self, n, dt, stims, commands, fused_act, probe_trackers, event_trackers):
+        """The event-free steps of dt among the next n: (activation flags, a gate
         per probe tracker, their times, the time after them).  They end
         before the first step with a due stimulus, an open event tracker or a
         due command, and with the step that terminates the run."""
         if not isinstance(self.t, (int, float)):
             return np.zeros(0), [], [], self.t
         # the left fold t += dt (accumulate adds in order)
-        t = np.add.accumulate(np.concatenate(([self.t], np.full(n, self.dt))))
+        t = np.add.accumulate(np.concatenate(([self.t], np.full(n, dt))))
         steps = np.arange(self.step, self.step + n)
 
         def first(mask):
