@@ -21,11 +21,14 @@ from . import _native
 
 _CHUNK = 4096  # steps per library call between host synchronisations
 # event-free steps in a row before the loop looks ahead for more of them, and
-# the steps it then looks at: a look costs some 60 us, a step taken by itself
-# 2.5 us, so runs with an event every few steps never pay for one (model.run()
-# of 1,000 event-free steps on 102 x 102 nodes: 3.04 -> 1.46 ms)
+# the most steps it then looks at: a look costs 27 us and 0.07 us per step, a
+# step taken by itself 2.5 us, so runs with an event every few steps never pay for
+# one (model.run() of 1,000 event-free steps on 102 x 102 nodes: 3.04 -> 1.46 ms).
+# A look ends at the next event as far as that is known and is left out below
+# _LOOK_LEAST steps.
 _LOOK_AFTER = 32
 _LOOK_AHEAD = 1024
+_LOOK_LEAST = 12
 
 
 def _gate_open(tracker, t, step) -> bool:
@@ -282,11 +285,16 @@ class CardiacModel:
                 calm = 0
                 if len(chunk_flags) == 0:
                     chunk_start[0] = self.step
+                events = extra_act + host_trackers + dev_trackers
                 ask = min(iters - done, _CHUNK - len(chunk_flags),
                           _LOOK_AHEAD if len(chunk_flags) < _LOOK_AHEAD else _CHUNK)
-                ahead = self._look_ahead(ask, dt, stims, commands, fused_act, probe_trackers,
-                                         extra_act + host_trackers + dev_trackers)
-                n = len(ahead[0])
+                near = self._steps_to_event(ask, dt, stims, commands, events)
+                n = 0
+                if near >= _LOOK_LEAST:
+                    ask = near
+                    ahead = self._look_ahead(ask, dt, stims, commands, fused_act, probe_trackers,
+                                             events)
+                    n = len(ahead[0])
                 if n:
                     flags, gates, times, t_next = ahead
                     base = len(chunk_flags)
@@ -403,18 +411,30 @@ class CardiacModel:
     def _can_look_ahead(self, dt, trackers) -> bool:
         """Whether the loop may resolve event-free steps of dt in bulk: the time
         fold, gates and termination rule are the package's own."""
-        return (isinstance(dt, float) and not self.state_saver and
+        return (isinstance(dt, float) and isinstance(self.t, (int, float)) and
+                not self.state_saver and
                 type(self).check_termination is CardiacModel.check_termination and
                 "check_termination" not in self.__dict__ and
                 all(type(tr.step) is int and tr.step > 0 for tr in trackers))
+
+    def _steps_to_event(self, n, dt, stims, commands, event_trackers):
+        """About how many of the next n steps come before an event (0: it is due),
+        without the time fold; _look_ahead finds the exact one."""
+        t = self.t
+        for ev in [*stims, *commands]:
+            if not ev.passed and (ev.t - t) / dt < n:
+                n = max(0, int((ev.t - t) / dt) + 1)
+        for tr in event_trackers:
+            wait = -self.step % tr.step  # to its next step, if its window is open then
+            if wait < n and tr.start_time <= t + (wait + 1) * dt and tr.end_time >= t:
+                n = wait
+        return n
 
     def _look_ahead(self, n, dt, stims, commands, fused_act, probe_trackers, event_trackers):
         """The event-free steps of dt among the next n: (activation flags, a gate
         per probe tracker, their times, the time after them).  They end
         before the first step with a due stimulus, an open event tracker or a
         due command, and with the step that terminates the run."""
-        if not isinstance(self.t, (int, float)):
-            return np.zeros(0), [], [], self.t
         # the left fold t += dt (accumulate adds in order)
         t = np.add.accumulate(np.concatenate(([self.t], np.full(n, dt))))
         steps = np.arange(self.step, self.step + n)

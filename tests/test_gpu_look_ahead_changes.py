@@ -71,3 +71,33 @@ def test_look_ahead_after_a_change(change, monkeypatch):
     for after in (3, 32):
         for a, b in zip(_run(after, change, monkeypatch), want):
             assert a.shape == b.shape and a.tobytes() == b.tobytes()
+
+
+@pytest.mark.parametrize("ecg, stim", [(100, 0.0), (50, 0.0), (33, 0.0), (0, 4.5)], ids=str)
+def test_looks_end_at_the_next_event(ecg, stim, monkeypatch):
+    # every step looked at is one taken, or all but: an ECG every few steps, a
+    # stimulus that lasts
+    import finitewave_amd as fw
+    m = fw.AlievPanfilov2D()
+    m.dt, m.dr, m.t_max, m.prog_bar = 0.01, 0.25, 6.0, False
+    m.cardiac_tissue = fw.CardiacTissue2D([24, 20])
+    m.stim_sequence = fw.StimSequence()
+    m.stim_sequence.add_stim(fw.StimVoltageCoord2D(0, 1.0, 0, 24, 0, 5))
+    if stim:
+        m.stim_sequence.add_stim(fw.StimCurrentCoord2D(1.0, 0.01, stim, 0, 24, 10, 15))
+    m.tracker_sequence = fw.TrackerSequence()
+    if ecg:
+        e = fw.ECG2DTracker()
+        e.measure_coords, e.step = np.array([[12, 10, 5.0]]), ecg
+        m.tracker_sequence.add_tracker(e)
+    looks = []
+    whole = type(m)._look_ahead
+
+    def look(self, n, *args):
+        out = whole(self, n, *args)
+        looks.append((n, len(out[0])))
+        return out
+    monkeypatch.setattr(type(m), "_look_ahead", look)
+    m.run()
+    assert bool(looks) == (ecg != 33)
+    assert sum(n for n, _ in looks) <= sum(k for _, k in looks) + 2 * len(looks)
