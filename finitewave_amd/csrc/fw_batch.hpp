@@ -206,14 +206,13 @@ __host__ __device__ constexpr int batch_unroll(int variant) {
 // kernel.  The FP64 TP06 step (exact weights formed per node) would take 132
 // registers (3 waves); held to 4 waves it takes 122 without spills and steps a
 // batch of six fibrotic 400^2 tissues in 185 us against 200 (5 waves would
-// spill 45).  The FP32 one is held to 5, and then takes 80 registers where the
-// compiler's choice is 98 and 4 waves: ten fibrotic tissues of 128 to 1024 columns
-// 160 -> 147 us per step.  The FP64 shapes of 4 nodes per work-item take 142
-// registers; held to 4 waves they would spill 21 (84 -> 89 us).  Other instances
-// keep the compiler's choice.
+// spill 45).  The FP64 shapes of 4 nodes per work-item take 142 registers; held
+// to 4 waves they would spill 21 (84 -> 89 us).  Other instances keep the
+// compiler's choice (FP32 TP06: 89 registers, 5 waves; held to 5 it takes 80 and
+// ten fibrotic tissues of 128 to 1024 columns 146.2 us against 144.9).
 template <int MODEL, typename R>
 constexpr int batch_min_waves() {
-  return MODEL == 6 ? (sizeof(R) == 8 ? 4 : 5) : 1;
+  return MODEL == 6 && sizeof(R) == 8 ? 4 : 1;
 }
 
 template <int MODEL, typename R, int V>

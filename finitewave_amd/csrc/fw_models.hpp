@@ -127,12 +127,13 @@ __device__ __forceinline__ R divc(R a, R b) {
 // infinity) and for a = -0 (+0); FIX: the hardware's fix-up gives those as the
 // full division does, in a seventh operation.  The TP06 update divides 76 times:
 // with this and div_recip 1026^2 went from 101.8 to 94.6 us per step.  FP32: the
-// plain division.
-template <typename R, bool FIX = false>
+// plain division.  NEWTON: Newton steps on the estimate.
+template <typename R, bool FIX = false, int NEWTON = 1>
 __device__ __forceinline__ R dv(R a, R b) {
   if constexpr (sizeof(R) == 8) {
     double r = __builtin_amdgcn_rcp(b);
-    r = fma(fma(-b, r, 1.0), r, r);
+#pragma unroll
+    for (int k = 0; k < NEWTON; ++k) r = fma(fma(-b, r, 1.0), r, r);
     double q = a * r;
     q = fma(fma(-b, q, a), r, q);
     if constexpr (FIX) q = __builtin_amdgcn_div_fixup(q, b, a);
@@ -587,6 +588,12 @@ __device__ __forceinline__ U tp06_update(U u_in, U un, SP& S, int64_t c, R dt, c
   const Exp<R, CHECKED, false> uexp;
   const R u = (R)u_in;  // the potential in the arithmetic type
   typedef double D;
+  // The calcium terms divide in double on both paths.  On the FP32 path a second
+  // Newton step is the faster: without it the compiler schedules the batch kernel
+  // into 98 registers and 4 waves per SIMD, with it into 89 and 5 (ten fibrotic
+  // tissues of 128 to 1024 columns 159.3 -> 144.9 us per step; 146.2 without it
+  // and held to 5 waves).
+  auto ddv = [](D a, D b) { return dv<D, false, sizeof(R) == 8 ? 1 : 2>(a, b); };
   const R ko = par<R>(P, 0), cao = par<R>(P, 1), nao = par<R>(P, 2);
   const D Vc = P.v[3], Vsr = P.v[4], Vss = P.v[5];
   const D Bufsr = P.v[8], Kbufsr = P.v[9], Bufss = P.v[10], Kbufss = P.v[11],
@@ -800,25 +807,25 @@ __device__ __forceinline__ U tp06_update(U u_in, U un, SP& S, int64_t c, R dt, c
     auto&& rrr = ref<R>(S, 17, c);
     auto&& oor = ref<R>(S, 18, c);
     const D casrD = casrr, cassD = cassr;
-    const D kCaSR = maxsr - dv(maxsr - minsr, 1 + dv(EC, casrD) * dv(EC, casrD));
-    const D k1 = dv(k1_, kCaSR);
+    const D kCaSR = maxsr - ddv(maxsr - minsr, 1 + ddv(EC, casrD) * ddv(EC, casrD));
+    const D k1 = ddv(k1_, kCaSR);
     const D k2 = k2_ * kCaSR;
     D rr = (D)rrr;
     const D drr = k4 * (1 - rr) - k2 * cassD * rr;
     rr += (D)dt * drr;
-    const D oo = dv(k1 * cassD * cassD * rr, k3 + k1 * cassD * cassD);
+    const D oo = ddv(k1 * cassD * cassD * rr, k3 + k1 * cassD * cassD);
     rrr = (R)rr;
     oor = (R)oo;
     irel = Vrel * oo * (casrD - cassD);
   }
   const D caiD = cair, casrD = casrr, cassD = cassr;
   const D ileak = Vleak * (casrD - caiD);
-  const D iup = dv(Vmaxup, 1.0 + dv(Kup * Kup, caiD * caiD));
+  const D iup = ddv(Vmaxup, 1.0 + ddv(Kup * Kup, caiD * caiD));
   const D ixfer = Vxfer * (cassD - caiD);
   const D dtD = (D)dt;
   // calc_casr: closed-form buffer quadratic
   {
-    const D CaCSQN = dv(Bufsr * casrD, casrD + Kbufsr);
+    const D CaCSQN = ddv(Bufsr * casrD, casrD + Kbufsr);
     const D dCaSR = dtD * (iup - irel - ileak);
     const D bjsr = Bufsr - CaCSQN - dCaSR - casrD + Kbufsr;
     const D cjsr = Kbufsr * (CaCSQN + dCaSR + casrD);
@@ -826,7 +833,7 @@ __device__ __forceinline__ U tp06_update(U u_in, U un, SP& S, int64_t c, R dt, c
   }
   // calc_cass
   {
-    const D CaSSBuf = dv(Bufss * cassD, cassD + Kbufss);
+    const D CaSSBuf = ddv(Bufss * cassD, cassD + Kbufss);
     const D dCaSS = dtD * (-ixfer * Dv[kVcOverVss] + irel * Dv[kVsrOverVss] +
                            -(D)ical * inversevssF2 * CAPACITANCE);
     const D bcss = Bufss - CaSSBuf - dCaSS - cassD + Kbufss;
