@@ -178,9 +178,20 @@ FW_HD inline Recip recip(double b) {
 // its one rounding (Brisebarre and Muller, IEEE Trans. Computers 53(8), 2004).
 // The result is RN(a/b) unless a/b lies that close to a rounding boundary,
 // which no quotient by a divisor of up to 50 significant bits does: a boundary
-// is then at least 2^-104 away.  Holds while a lo does not underflow; a zero
-// quotient may come out with the other sign.
+// is then at least 2^-104 away.  Of the divisors with more bits one in a hundred
+// has a numerator (a significand, at any exponent) whose quotient comes out one
+// ulp off; none of the models' literals (literal_recip) or default parameters
+// has.  Holds while a lo does not underflow; a zero quotient may come out with
+// the other sign.
 FW_HD inline double div_recip(double a, Recip y) { return fma(a, y.hi, a * y.lo); }
+
+// The pair of a literal divisor.  27.48's would miss for the one significand
+// 1.4044140624999992; with lo one ulp up none is left.
+FW_HD inline Recip literal_recip(double b) {
+  Recip y = recip(b);
+  if (b == 27.48) y.lo = 0x1.6ed425dcbe99bp-59;
+  return y;
+}
 
 // x^1.5 as x sqrt(x), with the root's remainder r = x - s s (sqrt(x) = s +
 // r / 2s, so x sqrt(x) = x s + s r / 2 to second order) and the product's

@@ -109,7 +109,7 @@ __device__ __forceinline__ float exprel(float y) {
 // division.
 template <typename R>
 __device__ __forceinline__ R divc(R a, R b) {
-  if constexpr (sizeof(R) == 8) return div_recip(a, recip(b));
+  if constexpr (sizeof(R) == 8) return div_recip(a, literal_recip(b));
   else return a / b;
 }
 
