@@ -1502,7 +1502,7 @@ static int build_units(fw_batch* b, const int32_t* slots, int32_t n_slots, hipSt
       }
   }
   // The 5-point units' rows are halved until there are 3 wavefronts per SIMD
-  // (fewer leave the march's latency open), at most to 16 (the halo of 2K rows).
+  // (fewer leave the march's latency open), at most to 16 (twice the halo of 2K).
   // FP32, us per step: 20 Mitchell-Schaeffer tissues of 64 to 512 columns 15.3 ->
   // 7.4, 512 of 64 10.4 -> 7.1, 20 of Aliev-Panfilov of 128 to 1024 20.3 -> 19.4;
   // 512 of 128 columns have 3072 units of 65 rows, 19.8, and would take 20.9

@@ -64,7 +64,8 @@ struct alignas(16) TbUnit {
 };
 
 constexpr int kTbWaves = kBlock / 64;  // units per block
-constexpr int kTbMinUnits = 3072, kTbMinRows = 16;
+constexpr int kTbMinUnits = 3072;      // 256 CUs, 4 SIMDs, 3 wavefronts: fewer shorten the runs
+constexpr int kTbMinRows = 16;         // down to twice the halo (2 K = 8 rows at K = 4)
 constexpr int kTbEdgeRows = 256;       // rows of an outer columns' unit: 8 nodes per lane
 
 struct TbLaunch {

@@ -156,12 +156,6 @@ __global__ __launch_bounds__(kBlock) void k_step3_march(const KArgs<float, float
 #pragma unroll
     for (int r = 0; r < RL; ++r) cd[r] = cp[off[r]];
   };
-  auto pack = [&](const uint32_t (&cd)[RL]) {
-    uint32_t m = 0;
-#pragma unroll
-    for (int r = 0; r < RL; ++r) m |= (cd[r] & 1u) << (4 * r);
-    return m;
-  };
   constexpr int NS = model_n_state(MODEL);
   // planes i, i + 1 and i + 2 live in slots c, n and f of three, a phase of
   // the loop each: nothing moves between registers, so no wait for a load in

@@ -582,7 +582,7 @@ __device__ __forceinline__ U ionic_lr91(U u_in, U un, SP& S, int64_t c, R dt,
 // ---- TP06  tp06_2d.py:242-1103 -----------------------------------------------
 // state order (tp06_2d.py:1073 call): cai casr cass nai Ki m h j xr1 xr2 xs r
 // s d f f2 fcass rr oo ; the first five are double in both precisions.
-template <typename R, bool SPLIT, bool CHECKED, typename SP, typename U>
+template <typename R, bool CHECKED, typename SP, typename U>
 __device__ __forceinline__ U tp06_update(U u_in, U un, SP& S, int64_t c, R dt, const Params& P) {
   const Exp<R, true, false> fexp;
   const Exp<R, CHECKED, false> uexp;
@@ -865,9 +865,9 @@ __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
                                         const Params& P) {
   if constexpr (SPLIT && sizeof(R) == 8) {
     if (__builtin_expect(__all(fabs(u_in) <= 160.0), 1))
-      return tp06_update<R, SPLIT, false>(u_in, un, S, c, dt, P);
+      return tp06_update<R, false>(u_in, un, S, c, dt, P);
   }
-  return tp06_update<R, SPLIT, true>(u_in, un, S, c, dt, P);
+  return tp06_update<R, true>(u_in, un, S, c, dt, P);
 }
 
 // ---- Courtemanche  courtemanche_2d.py:180-641 -------------------------------
