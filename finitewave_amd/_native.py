@@ -31,7 +31,7 @@ EXPORTS = (
     "fw_abi_version", "fw_last_error", "fw_model_info", "fw_state_is_f64", "fw_state_offset",
     "fw_u_is_f64",
     "fw_compute_weights", "fw_diffusion", "fw_ionic", "fw_plan_create",
-    "fw_plan_destroy", "fw_plan_set_weights_k", "fw_run", "fw_run_graph",
+    "fw_plan_destroy", "fw_plan_set_weights_k", "fw_plan_launch_shape", "fw_run", "fw_run_graph",
     "fw_run_graph_prepare", "fw_run_noalloc",
     "fw_stim_apply", "fw_plan_set_stims", "fw_stim_apply_step", "fw_act_time_update",
     "fw_lat_update", "fw_spiral_tips", "fw_ecg",
@@ -110,6 +110,7 @@ def lib():
     L.fw_plan_create.argtypes = [POINTER(fw_plan_desc), POINTER(vp)]
     L.fw_plan_destroy.argtypes = [vp]
     L.fw_plan_set_weights_k.argtypes = [vp, i32]
+    L.fw_plan_launch_shape.argtypes = [vp, i32, POINTER(i32), POINTER(i32)]
     L.fw_run.argtypes = [vp, vp, vp, POINTER(vp), i64, i32, POINTER(fw_track_desc), vp]
     L.fw_run_graph.argtypes = [vp, vp, vp, POINTER(vp), i64, i32, POINTER(fw_track_desc), vp]
     L.fw_run_graph_prepare.argtypes = [vp, vp, vp, POINTER(vp), i32, POINTER(fw_track_desc)]

@@ -804,6 +804,13 @@ static int64_t stim_until(const fw_plan* plan, int64_t step, int64_t last, int64
   return step;
 }
 
+// K of a stretch of `room` steps: pairs of the shape's, or of 4 or 2 steps (a
+// region of 2 K + 4 rows or more owns some); 0 where none fits.
+static int32_t multi_fit(int32_t k, int64_t room) {
+  while (k > 2 && 2 * k > room) k /= 2;
+  return 2 * k <= room ? k : 0;
+}
+
 // n_steps with multi-step launches wherever they apply, single steps
 // elsewhere (among them the last: u_new then holds the step before).
 // `singles` runs the single steps.  *done = false: nothing launched, the run
@@ -816,14 +823,7 @@ static int run_multi(fw_plan* plan, void* u, void* u_new, void* const* state, in
   if (!plan->alt) return FW_OK;
   int32_t shape_k, rows;
   multi_shape(plan, &shape_k, &rows);
-  // K of a stretch of `room` steps: pairs of the shape's, or of 4 or 2 steps
-  // (a region of 2 K + 4 rows or more owns some)
-  auto fit = [&](int64_t room) {
-    int32_t k = shape_k;
-    while (k > 2 && 2 * k > room) k /= 2;
-    return 2 * k <= room ? k : 0;
-  };
-  int32_t K = fit(n_steps - 1);
+  int32_t K = multi_fit(shape_k, n_steps - 1);
   if (K == 0 || step0 < 0 || step0 + n_steps > INT32_MAX) return FW_OK;
   int32_t act_on = 0;
   bool probes = false;
@@ -855,7 +855,7 @@ static int run_multi(fw_plan* plan, void* u, void* u_new, void* const* state, in
   while (pos < n_steps) {
     const int64_t step = step0 + pos;
     const int32_t room = (int32_t)stim_free(plan, step, n_steps - 1 - pos, stim_end);
-    K = fit(room);
+    K = multi_fit(shape_k, room);
     if (K > 0) {
       TrackArgs tr{};
       tr.step = (int32_t)step;
@@ -899,6 +899,21 @@ static int run_multi(fw_plan* plan, void* u, void* u_new, void* const* state, in
       b = t;
     }
   }
+  return FW_OK;
+}
+
+int fw_plan_launch_shape(const fw_plan* plan, int32_t n_steps, int32_t* steps, int32_t* rows) {
+  if (!plan || !steps || !rows || n_steps < 0) {
+    set_error("fw_plan_launch_shape: bad arguments");
+    return FW_E_INVALID;
+  }
+  int32_t k = 0, r = 0;
+  if (plan->alt) {
+    multi_shape(plan, &k, &r);
+    k = multi_fit(k, n_steps - 1);
+  }
+  *steps = k > 0 ? k : 1;
+  *rows = k > 0 ? r : 0;
   return FW_OK;
 }
 
