@@ -284,8 +284,11 @@ __device__ __forceinline__ void tb_march(const BatchArgs<R, R>& a, const BatchTi
   }
 }
 
-// K steps of the outer columns' nodes of rows [r0, r1): activation times and the
-// probe.  Both buffers and state sets hold the nodes' values since admission.
+// K steps of the outer columns' nodes of rows [r0, r1): activation times, the
+// probe and, once per pair, their potentials to the other buffer, which the caller
+// need not have filled: strips write nodes that are not updated too, and read the
+// outer columns as neighbours.  Their states stay where they are, in `state`.
+// (512 tissues of 64 to 512 columns: 87.8 -> 88.0 us per step for the copy.)
 template <typename R, int K>
 __device__ __forceinline__ void tb_edge(const BatchTissue& d, const int32_t ls0,
                                         const int32_t phase, const int32_t r0, const int32_t r1) {
@@ -298,12 +301,16 @@ __device__ __forceinline__ void tb_edge(const BatchTissue& d, const int32_t ls0,
   const int32_t first = ls0 > d.act_start ? ls0 : d.act_start;
   const bool record = act && d.act_start >= 0 && first < ls0 + K;
   const bool probing = probe && ls0 < d.probe_len;
-  if (!record && !probing) return;
-  const int32_t in_b = (ls0 & 1) ^ ((K % 2 == 0) ? phase : 0);
+  const bool copy = phase == 0;
+  if (!copy && !record && !probing) return;
+  static_assert(K % 2 == 0, "the pair's second launch reads what its first one wrote");
+  const int32_t in_b = (ls0 & 1) ^ phase;
   const global_t<R>* const u = (const global_t<R>*)(in_b ? d.un : d.u);
+  global_t<R>* const out = (global_t<R>*)(in_b ? d.u : d.un);
   for (int32_t q = (int32_t)(threadIdx.x & 63); q < 2 * (r1 - r0); q += 64) {
     const int32_t c = (r0 + (q >> 1)) * d.nj + (q & 1) * (d.nj - 1);
     const R v = u[c];
+    if (copy) out[c] = v;
     if (record && v > thr && act[c] < 0) act[c] = first;
     if (probing && c == d.probe_idx)
       for (int32_t t = ls0; t < ls0 + K && t < d.probe_len; ++t) probe[t] = v;
