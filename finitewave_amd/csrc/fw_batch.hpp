@@ -209,8 +209,7 @@ __host__ __device__ constexpr int batch_unroll(int variant) {
 // batch of six fibrotic 400^2 tissues in 185 us against 200 (5 waves would
 // spill 45).  The FP64 shapes of 4 nodes per work-item take 142 registers; held
 // to 4 waves they would spill 21 (84 -> 89 us).  Other instances keep the
-// compiler's choice (FP32 TP06: 89 registers, 5 waves; held to 5 it takes 80 and
-// ten fibrotic tissues of 128 to 1024 columns 146.2 us against 144.9).
+// compiler's choice (FP32 TP06: 94 registers, 5 waves; tp06_update says how).
 template <int MODEL, typename R>
 constexpr int batch_min_waves() {
   return MODEL == 6 && sizeof(R) == 8 ? 4 : 1;
@@ -296,7 +295,7 @@ __global__ __launch_bounds__(kBlock, (batch_min_waves<MODEL, R>())) void k_batch
         q.v[k] = need ? u[c + di * nj + dj] : U(0);
         q.m[k] = need ? (code[c + di * nj + dj] & 1) : 0;
       }
-    const U val = node_update<MODEL, R>(uc, S, (int64_t)c, a.dt, a.P, [&] {
+    const U val = node_update<MODEL, R, kBatchForm>(uc, S, (int64_t)c, a.dt, a.P, [&] {
       return diffuse9<U, EXACT>(stencil, dd, df, q, a.D, a.dtd, a.rdr2, a.s);
     });
     st_state<NT>(un + c, val);

@@ -988,6 +988,7 @@ __device__ __forceinline__ U stim_node(const A& a, int32_t s, int64_t i, int64_t
 template <int NDIM, int ST, int MODEL, typename R, int PREC, int FL>
 __device__ __forceinline__ void step_node(const KArgs<R, UType<MODEL, R>>& a, int64_t c,
                                           int32_t step) {
+  constexpr UpdateForm FORM = NDIM == 2 ? kSplitForm : kWholeForm;
   using U = UType<MODEL, R>;
   const uint8_t code = a.code[c];
   const U uc = a.u[c];
@@ -1007,11 +1008,11 @@ __device__ __forceinline__ void step_node(const KArgs<R, UType<MODEL, R>>& a, in
         // FP32 flux form: the neighbourhood is loaded before the ionic
         // update, as in the batched step
         const Hood2<U> q = load_hood2<ST>(a, c, uc);
-        v = node_update<MODEL, R, NDIM == 2>(uc, a.st, c, a.dt, a.P, [&] {
+        v = node_update<MODEL, R, FORM>(uc, a.st, c, a.dt, a.P, [&] {
           return flux2d<ST, FL>(a, i, j, c, uc, q);
         });
       } else {
-        v = node_update<MODEL, R, NDIM == 2>(uc, a.st, c, a.dt, a.P, [&] {
+        v = node_update<MODEL, R, FORM>(uc, a.st, c, a.dt, a.P, [&] {
           return diffuse<NDIM, ST, R, U, PREC == 0, FL>(a, i, j, k, c, uc);
         });
       }
@@ -1244,7 +1245,7 @@ __global__ __launch_bounds__(kBlock) void k_ionic(UType<MODEL, R>* __restrict__ 
   const int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (q >= n) return;
   const int64_t c = idx[q];
-  u_new[c] = ionic_update<MODEL, R, false>(u[c], u_new[c], st, c, dt, P);
+  u_new[c] = ionic_update<MODEL, R, kWholeForm>(u[c], u_new[c], st, c, dt, P);
 }
 
 template <typename R>

@@ -70,6 +70,11 @@ __device__ __forceinline__ void exp_table_to_lds() {
 __device__ __forceinline__ double fexp(double x) { return t128_exp_tab(x, exp_lds()); }
 __device__ __forceinline__ float fexp(float x) { return __expf(x); }
 
+// How a kernel wants the large models' updates compiled: as they stand, with a
+// second copy for ordinary potentials (the 2D sheet's step) or in the batch step's
+// scheduling regions.  The same operations in each.
+enum UpdateForm { kWholeForm, kSplitForm, kBatchForm };
+
 // The exp of a model's update: fexp with its three addends in vector registers
 // for the whole update (a fused multiply-add with two scalar constants moves one
 // into a vector register first, 6 of an exp's 46 operations).  !CHECKED: every
@@ -127,13 +132,12 @@ __device__ __forceinline__ R divc(R a, R b) {
 // infinity) and for a = -0 (+0); FIX: the hardware's fix-up gives those as the
 // full division does, in a seventh operation.  The TP06 update divides 76 times:
 // with this and div_recip 1026^2 went from 101.8 to 94.6 us per step.  FP32: the
-// plain division.  NEWTON: Newton steps on the estimate.
-template <typename R, bool FIX = false, int NEWTON = 1>
+// plain division.
+template <typename R, bool FIX = false>
 __device__ __forceinline__ R dv(R a, R b) {
   if constexpr (sizeof(R) == 8) {
     double r = __builtin_amdgcn_rcp(b);
-#pragma unroll
-    for (int k = 0; k < NEWTON; ++k) r = fma(fma(-b, r, 1.0), r, r);
+    r = fma(fma(-b, r, 1.0), r, r);
     double q = a * r;
     q = fma(fma(-b, q, a), r, q);
     if constexpr (FIX) q = __builtin_amdgcn_div_fixup(q, b, a);
@@ -582,18 +586,12 @@ __device__ __forceinline__ U ionic_lr91(U u_in, U un, SP& S, int64_t c, R dt,
 // ---- TP06  tp06_2d.py:242-1103 -----------------------------------------------
 // state order (tp06_2d.py:1073 call): cai casr cass nai Ki m h j xr1 xr2 xs r
 // s d f f2 fcass rr oo ; the first five are double in both precisions.
-template <typename R, bool CHECKED, typename SP, typename U>
+template <typename R, UpdateForm FORM, bool CHECKED, typename SP, typename U>
 __device__ __forceinline__ U tp06_update(U u_in, U un, SP& S, int64_t c, R dt, const Params& P) {
   const Exp<R, true, false> fexp;
   const Exp<R, CHECKED, false> uexp;
   const R u = (R)u_in;  // the potential in the arithmetic type
   typedef double D;
-  // The calcium terms divide in double on both paths.  On the FP32 path a second
-  // Newton step is the faster: without it the compiler schedules the batch kernel
-  // into 98 registers and 4 waves per SIMD, with it into 89 and 5 (ten fibrotic
-  // tissues of 128 to 1024 columns 159.3 -> 144.9 us per step; 146.2 without it
-  // and held to 5 waves).
-  auto ddv = [](D a, D b) { return dv<D, false, sizeof(R) == 8 ? 1 : 2>(a, b); };
   const R ko = par<R>(P, 0), cao = par<R>(P, 1), nao = par<R>(P, 2);
   const D Vc = P.v[3], Vsr = P.v[4], Vss = P.v[5];
   const D Bufsr = P.v[8], Kbufsr = P.v[9], Bufss = P.v[10], Kbufss = P.v[11],
@@ -807,33 +805,39 @@ __device__ __forceinline__ U tp06_update(U u_in, U un, SP& S, int64_t c, R dt, c
     auto&& rrr = ref<R>(S, 17, c);
     auto&& oor = ref<R>(S, 18, c);
     const D casrD = casrr, cassD = cassr;
-    const D kCaSR = maxsr - ddv(maxsr - minsr, 1 + ddv(EC, casrD) * ddv(EC, casrD));
-    const D k1 = ddv(k1_, kCaSR);
+    const D kCaSR = maxsr - dv(maxsr - minsr, 1 + dv(EC, casrD) * dv(EC, casrD));
+    const D k1 = dv(k1_, kCaSR);
     const D k2 = k2_ * kCaSR;
     D rr = (D)rrr;
     const D drr = k4 * (1 - rr) - k2 * cassD * rr;
     rr += (D)dt * drr;
-    const D oo = ddv(k1 * cassD * cassD * rr, k3 + k1 * cassD * cassD);
+    const D oo = dv(k1 * cassD * cassD * rr, k3 + k1 * cassD * cassD);
     rrr = (R)rr;
     oor = (R)oo;
     irel = Vrel * oo * (casrD - cassD);
   }
   const D caiD = cair, casrD = casrr, cassD = cassr;
   const D ileak = Vleak * (casrD - caiD);
-  const D iup = ddv(Vmaxup, 1.0 + ddv(Kup * Kup, caiD * caiD));
+  const D iup = dv(Vmaxup, 1.0 + dv(Kup * Kup, caiD * caiD));
   const D ixfer = Vxfer * (cassD - caiD);
   const D dtD = (D)dt;
   // calc_casr: closed-form buffer quadratic
   {
-    const D CaCSQN = ddv(Bufsr * casrD, casrD + Kbufsr);
+    const D CaCSQN = dv(Bufsr * casrD, casrD + Kbufsr);
     const D dCaSR = dtD * (iup - irel - ileak);
+    // FP32 batch steps: what follows is scheduled by itself.  In one region with the
+    // rest the kernel takes 98 registers and 4 waves per SIMD, so 94 and 5 (ten
+    // fibrotic tissues of 128 to 1024 columns 159.3 -> 145.1 us per step; held to 5
+    // waves it takes 80 registers and 146.1).  The sheet's and the block's steps lose
+    // by it (300^2 7.60 -> 7.92 us, 131 x 115 x 147 144.6 -> 146.1).
+    if constexpr (!F64 && FORM == kBatchForm) __builtin_amdgcn_sched_barrier(0);
     const D bjsr = Bufsr - CaCSQN - dCaSR - casrD + Kbufsr;
     const D cjsr = Kbufsr * (CaCSQN + dCaSR + casrD);
     casrr = (sqrt(bjsr * bjsr + 4 * cjsr) - bjsr) / 2;
   }
   // calc_cass
   {
-    const D CaSSBuf = ddv(Bufss * cassD, cassD + Kbufss);
+    const D CaSSBuf = dv(Bufss * cassD, cassD + Kbufss);
     const D dCaSS = dtD * (-ixfer * Dv[kVcOverVss] + irel * Dv[kVsrOverVss] +
                            -(D)ical * inversevssF2 * CAPACITANCE);
     const D bcss = Bufss - CaSSBuf - dCaSS - cassD + Kbufss;
@@ -854,20 +858,20 @@ __device__ __forceinline__ U tp06_update(U u_in, U un, SP& S, int64_t c, R dt, c
                     inaca + ipca + ipk);
 }
 
-// SPLIT: the exps of a function of u only, at most 202 in magnitude for |u| <= 160,
+// kSplitForm: the exps of a function of u only, at most 202 in magnitude for |u| <= 160,
 // without their check where a wavefront's nodes lie there: straight-line code
 // that overlaps their table reads, in a second copy of the update (128 against 96
 // registers: the 2D single-tissue step; 1026^2 93.9 -> 91.8 us per step, 300^2
 // 18.9 -> 17.2, 200^2 15.2 -> 12.9; a 3D block of 131 x 115 x 147 would lose 3 %
 // and a batch of four 24 %).
-template <typename R, bool SPLIT, typename SP, typename U = R>
+template <typename R, UpdateForm FORM, typename SP, typename U = R>
 __device__ __forceinline__ U ionic_tp06(U u_in, U un, SP& S, int64_t c, R dt,
                                         const Params& P) {
-  if constexpr (SPLIT && sizeof(R) == 8) {
+  if constexpr (FORM == kSplitForm && sizeof(R) == 8) {
     if (__builtin_expect(__all(fabs(u_in) <= 160.0), 1))
-      return tp06_update<R, false>(u_in, un, S, c, dt, P);
+      return tp06_update<R, FORM, false>(u_in, un, S, c, dt, P);
   }
-  return tp06_update<R, true>(u_in, un, S, c, dt, P);
+  return tp06_update<R, FORM, true>(u_in, un, S, c, dt, P);
 }
 
 // ---- Courtemanche  courtemanche_2d.py:180-641 -------------------------------
@@ -1159,13 +1163,14 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
                     inaca + ibna + ibca);
 }
 
-// SPLIT: as TP06's; here the arguments stay below 75, and the 2D single-tissue
+// kSplitForm: as TP06's; here the arguments stay below 75, and the 2D single-tissue
 // step takes 148 registers and 3 waves against 116 and 4 (1026^2 with 10 % of
 // fibrosis 97.7 -> 93.0 us per step, 500^2 30.0 -> 28.9, 200^2 14.5 -> 11.8; the 3D
 // block would lose 3 %).
-template <typename R, bool SPLIT, typename SP, typename U = R>
+template <typename R, UpdateForm FORM, typename SP, typename U = R>
 __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
                                         const Params& P) {
+  constexpr bool SPLIT = FORM == kSplitForm;
   if constexpr (SPLIT && sizeof(R) == 8) {
     if (__builtin_expect(__all(fabs(u_in) <= 160.0), 1))
       return crn_update<R, SPLIT, false>(u_in, un, S, c, dt, P);
@@ -1190,7 +1195,7 @@ __host__ __device__ constexpr bool u_is_f64(int model, int precision) {
 template <int MODEL, typename R>
 using UType = std::conditional_t<(sizeof(R) == 8 || MODEL >= 5), double, R>;
 
-template <int MODEL, typename R, bool SPLIT, typename SP, typename U>
+template <int MODEL, typename R, UpdateForm FORM, typename SP, typename U>
 __device__ __forceinline__ U ionic_update(U u, U un, SP& S, int64_t c, R dt,
                                           const Params& P) {
   if constexpr (MODEL == 0) return ionic_ap<R>(u, un, S, c, dt, P);
@@ -1199,8 +1204,8 @@ __device__ __forceinline__ U ionic_update(U u, U un, SP& S, int64_t c, R dt,
   else if constexpr (MODEL == 3) return ionic_fk<R>(u, un, S, c, dt, P);
   else if constexpr (MODEL == 4) return ionic_bo<R>(u, un, S, c, dt, P);
   else if constexpr (MODEL == 5) return ionic_lr91<R, SP, U>(u, un, S, c, dt, P);
-  else if constexpr (MODEL == 6) return ionic_tp06<R, SPLIT, SP, U>(u, un, S, c, dt, P);
-  else return ionic_crn<R, SPLIT, SP, U>(u, un, S, c, dt, P);
+  else if constexpr (MODEL == 6) return ionic_tp06<R, FORM, SP, U>(u, un, S, c, dt, P);
+  else return ionic_crn<R, FORM, SP, U>(u, un, S, c, dt, P);
 }
 
 // number of state arrays per model (state_vars minus u)
@@ -1218,15 +1223,15 @@ __host__ __device__ constexpr int model_n_state(int model) {
 // reference's value exactly.  FP32 builds fuse multiply-adds within one
 // expression only, so the single-tissue and batched kernels, which both use
 // this function, stay bit-identical.
-template <int MODEL, typename R, bool SPLIT = false, typename U, typename SP,
+template <int MODEL, typename R, UpdateForm FORM = kWholeForm, typename U, typename SP,
           typename Diffusion>
 __device__ __forceinline__ U node_update(U uc, SP& S, int64_t c, R dt, const Params& P,
                                          Diffusion&& diffusion) {
   if constexpr (MODEL >= 5) {
-    const U r = ionic_update<MODEL, R, SPLIT>(uc, U(0), S, c, dt, P);
+    const U r = ionic_update<MODEL, R, FORM>(uc, U(0), S, c, dt, P);
     return diffusion() + r;
   } else {
-    return ionic_update<MODEL, R, SPLIT>(uc, diffusion(), S, c, dt, P);
+    return ionic_update<MODEL, R, FORM>(uc, diffusion(), S, c, dt, P);
   }
 }
 
