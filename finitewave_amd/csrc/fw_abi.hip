@@ -457,12 +457,11 @@ static int plan_host_init(const fw_plan_desc* desc, fw_plan* p, const char* who)
 constexpr size_t kStepWordBytes = 256;
 static_assert(16 + FW_MAX_FIELDS * (sizeof(double) + sizeof(float)) <= kStepWordBytes);
 
-// The largest sheet stepped by multi-step launches (2000^2 still gains 2 % to
-// 17 %, past it both are bound by HBM), the largest of the models with tanh
-// where multi_shape says so, and the single steps in a row (a long stimulus)
-// that are worth capturing a graph for beside them.
+// The largest sheet stepped by multi-step launches, the single steps in a row (a
+// long stimulus) that are worth capturing a graph for beside them, and the largest
+// sheet that takes two steps per launch in fw_run (multi_least).
 constexpr int64_t kMultiMaxNodes = (int64_t)1 << 22;
-constexpr int64_t kMultiMaxTanh = (int64_t)1 << 18;
+constexpr int64_t kMultiMaxPairs = (int64_t)3 << 17;
 constexpr int32_t kMultiGraphSteps = 64;
 
 static void multi_shape(const fw_plan* plan, int32_t* K, int32_t* rows);
@@ -750,13 +749,30 @@ struct AltUse {
 // 6.1 / 9.2; FP32 0.81 / 1.22 / 2.64, 1.73 / 1.86 / 2.94, 5.7 / 4.6 / 6.0).
 // The FP64 Fenton-Karma and Bueno-Orovio updates cost 4 and 10 times as much,
 // so redundant nodes stop paying once CUs are shared (400^2 iso: 5.2 and 10.9
-// at K = 4 against 5.3 and 7.8); in FP32 with the 9-point stencil they do
-// between 400^2 (3.1 and 4.1 against 3.6 and 4.3) and 900^2 (9.2 and 11.3
-// against 8.3 and 10.4), Bueno-Orovio with the 5-point one at 560^2 (4.8
-// against 4.7).
+// at K = 4 against 5.3 and 7.8).  multi_limit has the size at which the others
+// stop gaining.
 static int32_t multi_blocks(const fw_plan* plan, int32_t K, int32_t rows) {
   const int64_t w = kMultiW - 2 * K, h = rows - 2 * K;
   return (int32_t)(((plan->desc.shape[0] + h - 1) / h) * ((plan->desc.shape[1] + w - 1) / w));
+}
+
+// The largest sheet whose K = 4 launches beat single steps (us per step of runs of
+// 200 steps, K = 4 / single, on either side of each line; in runs of 10 to 20 steps,
+// where launches count, K = 4 gains 5 to 15 % more):
+//   Fenton-Karma and Bueno-Orovio FP32, 9-point: 400^2 3.1 and 4.1 / 3.6 and 4.3,
+//     900^2 9.2 and 11.3 / 8.3 and 10.4; Bueno-Orovio 5-point 560^2 4.8 / 4.7
+//   FP64 9-point: Aliev-Panfilov 560^2 4.7 / 5.0, 700^2 6.4 / 6.4, 850^2 8.5 / 8.2,
+//     2000^2 a third slower; Mitchell-Schaeffer 560^2 5.2 / 5.2, 700^2 7.3 / 6.6
+//   FP32 5-point: Aliev-Panfilov 1000^2 5.0 / 5.2, 1200^2 6.5 / 6.4, 1500^2 9.8 / 8.7
+//   FP64 5-point: Mitchell-Schaeffer 1200^2 10.7 / 11.6, 1800^2 22.2 / 21.5;
+//     Aliev-Panfilov 2000^2 23.0 / 24.7
+//   FP32 9-point: within 3 % of each other from 1500^2 on
+static int64_t multi_limit(const fw_plan_desc& d) {
+  const bool f64 = d.precision == FW_PREC_FP64, aniso = d.stencil == FW_STENCIL_ANISO;
+  if (d.model >= 3 && !f64 && (aniso || d.model == 4)) return (int64_t)1 << 18;
+  if (f64 && aniso) return d.model == 2 ? (int64_t)3 << 17 : (int64_t)1 << 19;
+  if (f64) return d.model == 2 ? (int64_t)5 << 19 : kMultiMaxNodes;
+  return aniso ? kMultiMaxNodes : (int64_t)3 << 19;
 }
 
 static void multi_shape(const fw_plan* plan, int32_t* K, int32_t* rows) {
@@ -772,14 +788,20 @@ static void multi_shape(const fw_plan* plan, int32_t* K, int32_t* rows) {
     if (heavy) break;
   }
   *K = 4;
-  *rows = 16;
-  if (heavy) {
-    if (multi_blocks(plan, 4, 16) > kCus) *K = 0;
-  } else if (tanh_model && (aniso || d.model == 4)) {
-    if (plan->N > kMultiMaxTanh) *K = 0;
-  } else if (!(aniso && f64)) {
-    *rows = 32;
-  }
+  *rows = (f64 && (aniso || tanh_model)) || (tanh_model && (aniso || d.model == 4)) ? 16 : 32;
+  if (heavy ? multi_blocks(plan, 4, 16) > kCus : plan->N > multi_limit(d)) *K = 0;
+}
+
+// The fewest steps per launch worth taking, for short runs and the rest of long
+// ones.  A pair of two-step launches replaces four single steps of 2.5 to 3 us each
+// (us per run of 6 steps, FP32 Aliev-Panfilov iso 560^2 22.3 instead of 25.7, 700^2
+// 30.4 instead of 28.0), not those of FP64 Bueno-Orovio, which cost more (200^2, 5 steps: 39.1 instead of 28.2).
+// fw_run_graph's alternative for a short run is a graph launch (6 steps of FP64
+// Aliev-Panfilov iso 700^2: 39.5 instead of 46.4).
+static int32_t multi_least(const fw_plan* plan, bool graph) {
+  const fw_plan_desc& d = plan->desc;
+  if (d.precision == FW_PREC_FP64 && d.model == 4) return 4;
+  return !graph && plan->N > kMultiMaxPairs ? 4 : 2;
 }
 
 // Steps a run can take in multi-step pairs before a scheduled stimulus
@@ -804,10 +826,10 @@ static int64_t stim_until(const fw_plan* plan, int64_t step, int64_t last, int64
   return step;
 }
 
-// K of a stretch of `room` steps: pairs of the shape's, or of 4 or 2 steps (a
-// region of 2 K + 4 rows or more owns some); 0 where none fits.
-static int32_t multi_fit(int32_t k, int64_t room) {
-  while (k > 2 && 2 * k > room) k /= 2;
+// K of a stretch of `room` steps: pairs of the shape's, or of fewer down to
+// `least` (a region of 2 K + 4 rows or more owns some); 0 where none fits.
+static int32_t multi_fit(int32_t k, int32_t least, int64_t room) {
+  while (k > least && 2 * k > room) k /= 2;
   return 2 * k <= room ? k : 0;
 }
 
@@ -817,13 +839,14 @@ static int32_t multi_fit(int32_t k, int64_t room) {
 // has no multi-step form.
 typedef std::function<int(void*, void*, int64_t, int32_t, const fw_track_desc*)> Singles;
 static int run_multi(fw_plan* plan, void* u, void* u_new, void* const* state, int64_t step0,
-                     int32_t n_steps, const fw_track_desc* track, hipStream_t s,
+                     int32_t n_steps, const fw_track_desc* track, hipStream_t s, bool graph,
                      const Singles& singles, bool* done) {
   *done = false;
   if (!plan->alt) return FW_OK;
   int32_t shape_k, rows;
   multi_shape(plan, &shape_k, &rows);
-  int32_t K = multi_fit(shape_k, n_steps - 1);
+  const int32_t least = multi_least(plan, graph);
+  int32_t K = multi_fit(shape_k, least, n_steps - 1);
   if (K == 0 || step0 < 0 || step0 + n_steps > INT32_MAX) return FW_OK;
   int32_t act_on = 0;
   bool probes = false;
@@ -855,7 +878,7 @@ static int run_multi(fw_plan* plan, void* u, void* u_new, void* const* state, in
   while (pos < n_steps) {
     const int64_t step = step0 + pos;
     const int32_t room = (int32_t)stim_free(plan, step, n_steps - 1 - pos, stim_end);
-    K = multi_fit(shape_k, room);
+    K = multi_fit(shape_k, least, room);
     if (K > 0) {
       TrackArgs tr{};
       tr.step = (int32_t)step;
@@ -910,7 +933,7 @@ int fw_plan_launch_shape(const fw_plan* plan, int32_t n_steps, int32_t* steps, i
   int32_t k = 0, r = 0;
   if (plan->alt) {
     multi_shape(plan, &k, &r);
-    k = multi_fit(k, n_steps - 1);
+    k = multi_fit(k, multi_least(plan, false), n_steps - 1);
   }
   *steps = k > 0 ? k : 1;
   *rows = k > 0 ? r : 0;
@@ -922,7 +945,7 @@ int fw_run(fw_plan* plan, void* u, void* u_new, void* const* state, int64_t step
   int rc = check_run_args(plan, u, u_new, state, n_steps, track);
   if (rc) return rc;
   bool done = false;
-  rc = run_multi(plan, u, u_new, state, step0, n_steps, track, as_stream(stream),
+  rc = run_multi(plan, u, u_new, state, step0, n_steps, track, as_stream(stream), false,
                  [&](void* a, void* b, int64_t step, int32_t n, const fw_track_desc* t) {
                    return run_plain(plan, a, b, state, step, n, t, stream);
                  },
@@ -1237,7 +1260,7 @@ int fw_run_graph(fw_plan* plan, void* u, void* u_new, void* const* state, int64_
   int rc = check_graph_args(plan, u, u_new, state, n_steps, track, &act_on);
   if (rc) return rc;
   bool done = false;
-  rc = run_multi(plan, u, u_new, state, step0, n_steps, track, as_stream(stream),
+  rc = run_multi(plan, u, u_new, state, step0, n_steps, track, as_stream(stream), true,
                  [&](void* a, void* b, int64_t step, int32_t n, const fw_track_desc* t) {
                    return n >= kMultiGraphSteps
                               ? run_graphs(plan, a, b, state, step, n, t, stream)

@@ -239,10 +239,9 @@ int fw_run(fw_plan* plan, void* u, void* u_new, void* const* state,
            int64_t step0, int32_t n_steps, const fw_track_desc* track,
            void* stream);
 
-/* How fw_run and fw_run_graph launch n_steps steps of this plan without stimuli,
- * the tracker's gate and probe rows steady: *steps steps per launch at first (1:
- * single steps) and, where there are several, the rows of a block's region (else
- * 0). */
+/* How fw_run launches n_steps steps of this plan without stimuli, the tracker's
+ * gate and probe rows steady: *steps steps per launch at first (1: single steps)
+ * and, where there are several, the rows of a block's region (else 0). */
 int fw_plan_launch_shape(const fw_plan* plan, int32_t n_steps, int32_t* steps, int32_t* rows);
 
 /* Same step as fw_run with n_steps = 1, recorded into a HIP graph of

@@ -47,8 +47,30 @@ def test_every_launch_shape(gpu, name, precision, shape):
         want = _expected(name, shape, precision, aniso)
         assert _shape(eng, 40) == want
         if want != (1, 0):
-            assert _shape(eng, 5) == (2, want[1]) and _shape(eng, 9) == (4, want[1])
+            # FP64 Bueno-Orovio takes no two-step launches
+            two = (1, 0) if (name, precision) == ("BuenoOrovio2D", "fp64") else (2, want[1])
+            assert _shape(eng, 5) == two and _shape(eng, 9) == (4, want[1])
         assert _shape(eng, 4) == (1, 0)
         eng.close()
         for n in (5, 9, 27):
             _same(_run(m, n, True), _run(m, n, False))
+
+
+# (model, precision, aniso, side) on either side of the sizes up to which several
+# steps per launch, and two steps for a short run, are the faster
+@pytest.mark.parametrize("name, precision, aniso, side, many, few", [
+    ("AlievPanfilov2D", "fp64", True, 724, 4, 1), ("AlievPanfilov2D", "fp64", True, 725, 1, 1),
+    ("MitchellSchaeffer2D", "fp64", True, 627, 4, 2),
+    ("MitchellSchaeffer2D", "fp64", True, 628, 1, 1),
+    ("MitchellSchaeffer2D", "fp64", False, 1619, 4, 1),
+    ("MitchellSchaeffer2D", "fp64", False, 1620, 1, 1),
+    ("Barkley2D", "fp64", False, 2048, 4, 1), ("Barkley2D", "fp64", False, 2049, 1, 1),
+    ("AlievPanfilov2D", "fp32", False, 1254, 4, 1), ("AlievPanfilov2D", "fp32", False, 1255, 1, 1),
+    ("AlievPanfilov2D", "fp32", True, 627, 4, 2), ("AlievPanfilov2D", "fp32", True, 628, 4, 1),
+    ("FentonKarma2D", "fp32", True, 512, 4, 2), ("FentonKarma2D", "fp32", True, 513, 1, 1),
+])
+def test_where_the_lines_lie(gpu, name, precision, aniso, side, many, few):
+    from finitewave_amd.engine import Engine
+    eng = Engine(_model(name, (side, side), precision, aniso, frozen=False))
+    assert _shape(eng, 40)[0] == many and _shape(eng, 5)[0] == few
+    eng.close()
