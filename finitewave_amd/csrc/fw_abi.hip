@@ -127,9 +127,19 @@ static void derive_crn(Params& P) {
   put_recip(P.v + kCrnInvFVj, F * Vj);
   put_recip(P.v + kCrnInv2FVj, 2.0 * F * Vj);
   put_recip(P.v + kCrnInvVj, Vj);
+  // kq10, a factor of four time constants' divisors, and the exchanger's
+  bool ordinary = P.v[38] != 0.0 && P.v[kCrnT12] != 0.0;
+  for (int q = 0; q < kCrnOrdinary; ++q) ordinary = ordinary && fabs(P.v[q]) < HUGE_VAL;
+  P.v[kCrnOrdinary] = ordinary ? 1.0 : 0.0;
 }
 
 void complete_params(int model, Params& P) {
+  if (model == 0 && fabs(P.v[4]) == HUGE_VAL && fabs(P.v[3]) < HUGE_VAL) {
+    // Aliev-Panfilov, mu_1 v / (mu_2 + u) with an infinite mu_2: the zero it is,
+    // by a divisor that the six-operation division takes
+    P.v[3] = 0.0;
+    P.v[4] = 1e300;
+  }
   if (model == 2) {
     // Mitchell-Schaeffer, float path: 1 / tau_open, 1 / tau_close
     P.v[5] = 1.0 / P.v[1];

@@ -173,6 +173,7 @@ enum CrnDerived {
   kCrnInv2FVjLo,
   kCrnInvVj,
   kCrnInvVjLo,
+  kCrnOrdinary,   // 1 when no divisor is infinite or zero by a parameter's value, else 0
   kCrnNDerivedEnd
 };
 static_assert(kCrnNDerivedEnd <= 64, "parameter block size");
@@ -305,7 +306,7 @@ __device__ __forceinline__ R ionic_ap(R u, R un, SP& S, int64_t c,
   auto&& vref = ref<R>(S, 0, c);
   R v = vref;
   // calc_v: v += (-dt*(eap + (mu_1*v)/(mu_2 + u)) * (v + k*u*(u - a - 1.)))
-  v += (-dt * (eap + dv<R, true>(mu_1 * v, mu_2 + u)) * (v + k * u * (u - a - R(1))));
+  v += (-dt * (eap + dv(mu_1 * v, mu_2 + u)) * (v + k * u * (u - a - R(1))));
   vref = v;
   // u_new += dt*(-k*u*(u - a)*(u - 1.) - u*v)
   return un + dt * (-k * u * (u - a) * (u - R(1)) - u * v);
@@ -890,10 +891,10 @@ template <typename R, bool SPLIT, bool CHECKED, typename SP, typename U>
 __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, const Params& P) {
   const Exp<R, true, SPLIT> fexp;
   const Exp<R, CHECKED, SPLIT> uexp;
-  // udv: by a divisor of u alone, infinite or zero only where an exp overflows;
-  // fdv: by one that holds a parameter or the state, or (xr) that a node one ulp
-  // from its singularity makes zero
-  auto udv = [](R a, R b) { return dv<R, CHECKED>(a, b); };
+  // pdv: by a divisor that a parameter or an overflowing exp may make infinite or
+  // zero, which ionic_crn rules out for the unchecked copy; fdv: by one that a node
+  // an ulp from the xr rate's singularity makes zero
+  auto pdv = [](R a, R b) { return dv<R, CHECKED>(a, b); };
   auto fdv = [](R a, R b) { return dv<R, true>(a, b); };
   const R u = (R)u_in;  // the potential in the arithmetic type
   const R gna = par<R>(P, 0), gnab = par<R>(P, 1), gk1 = par<R>(P, 2), gks = par<R>(P, 4),
@@ -918,9 +919,9 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
   constexpr bool F64 = sizeof(R) == 8;
   const R rtf = F64 ? par<R>(P, kCrnRTF) : R_ * T / F;
   const R rt2f = F64 ? par<R>(P, kCrnRT2F) : R_ * T / (R(2) * F);
-  const R ena = rtf * flog(fdv(nao, nai));
-  const R ek = rtf * flog(fdv(ko, ki));
-  const R eca = rt2f * flog(fdv(cao, cai));
+  const R ena = rtf * flog(pdv(nao, nai));
+  const R ek = rtf * flog(pdv(ko, ki));
+  const R eca = rt2f * flog(pdv(cao, cai));
   // x / b for a uniform b whose reciprocal pair is derived parameter iq
   auto divu = [&](R x, R b, int iq) -> R {
     if constexpr (F64) return div_recip(x, par_recip(P, iq));
@@ -938,12 +939,12 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
       if (u == R(-47.13)) {
         am = R(3.2);
       } else {
-        am = udv(R(0.32) * (u + R(47.13)), R(1) - uexp(R(-0.1) * (u + R(47.13))));
+        am = pdv(R(0.32) * (u + R(47.13)), R(1) - uexp(R(-0.1) * (u + R(47.13))));
       }
     }
     const R bm = R(0.08) * uexp(divc(-u, R(11)));
-    const R m_inf = udv(am, am + bm);
-    const R tau_m = udv(R(1), am + bm);
+    const R m_inf = pdv(am, am + bm);
+    const R tau_m = pdv(R(1), am + bm);
     m = crn_gate<R, CHECKED>(fexp, mr, m_inf, tau_m, dt);
     mr = m;
   }
@@ -952,13 +953,13 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
     R ah, bh;
     if (u >= R(-40)) {
       ah = R(0);
-      bh = udv(R(1), R(0.13) * (R(1) + uexp(divc(-(u + R(10.66)), R(11.1)))));
+      bh = pdv(R(1), R(0.13) * (R(1) + uexp(divc(-(u + R(10.66)), R(11.1)))));
     } else {
       ah = R(0.135) * uexp(divc(-(R(80) + u), R(6.8)));
       bh = R(3.56) * uexp(R(0.079) * u) + R(310000) * uexp(R(0.35) * u);
     }
-    const R h_inf = udv(ah, ah + bh);
-    const R tau_h = udv(R(1), ah + bh);
+    const R h_inf = pdv(ah, ah + bh);
+    const R tau_h = pdv(R(1), ah + bh);
     h = crn_gate<R, CHECKED>(fexp, hr, h_inf, tau_h, dt);
     hr = h;
   }
@@ -967,35 +968,35 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
     R aj, bj;
     if (u >= R(-40)) {
       aj = R(0);
-      bj = udv(R(0.3) * uexp(R(-2.535e-07) * u), R(1) + uexp(R(-0.1) * (u + R(32))));
+      bj = pdv(R(0.3) * uexp(R(-2.535e-07) * u), R(1) + uexp(R(-0.1) * (u + R(32))));
     } else {
-      aj = udv((R(-127140) * uexp(R(0.2444) * u) - R(3.474e-05) * uexp(R(-0.04391) * u)) *
+      aj = pdv((R(-127140) * uexp(R(0.2444) * u) - R(3.474e-05) * uexp(R(-0.04391) * u)) *
                   (u + R(37.78)),
               R(1) + uexp(R(0.311) * (u + R(79.23))));
-      bj = udv(R(0.1212) * uexp(R(-0.01052) * u), R(1) + uexp(R(-0.1378) * (u + R(40.14))));
+      bj = pdv(R(0.1212) * uexp(R(-0.01052) * u), R(1) + uexp(R(-0.1378) * (u + R(40.14))));
     }
-    const R j_inf = udv(aj, aj + bj);
-    const R tau_j = udv(R(1), aj + bj);
-    j = j_inf - (j_inf - jr) * fexp(udv(-dt, tau_j));
+    const R j_inf = pdv(aj, aj + bj);
+    const R tau_j = pdv(R(1), aj + bj);
+    j = j_inf - (j_inf - jr) * fexp(pdv(-dt, tau_j));
     jr = j;
   }
   const R ina = gna * (m * (m * m)) * h * j * (u - ena);
-  const R ik1 = udv(gk1 * (u - ek), R(1) + uexp(R(0.07) * (u + R(80))));
+  const R ik1 = pdv(gk1 * (u - ek), R(1) + uexp(R(0.07) * (u + R(80))));
   // calc_ito
   R ito;
   {
     auto&& oar = ref<R>(S, 10, c);
     auto&& oir = ref<R>(S, 11, c);
-    const R ao = udv(R(0.65), uexp(divc(-(u + R(10)), R(8.5))) + uexp(divc(-(u - R(30)), R(59.0))));
-    const R bo = udv(R(0.65), R(2.5) + uexp(divc(u + R(82), R(17.0))));
-    const R tau_o = fdv(R(1), kq10 * (ao + bo));
-    const R o_inf = udv(R(1), R(1) + uexp(divc(-(u + R(20.47)), R(17.54))));
-    const R aoi = udv(R(1), R(18.53) + uexp(divc(u + R(113.7), R(10.95))));
-    const R boi = udv(R(1), R(35.56) + uexp(divc(-(u + R(1.26)), R(7.44))));
-    const R tau_oi = fdv(R(1), kq10 * (aoi + boi));
-    const R oi_inf = udv(R(1), R(1) + uexp(divc(u + R(43.1), R(5.3))));
-    const R oa = crn_gate<R, true>(fexp, oar, o_inf, tau_o, dt);
-    const R oi = crn_gate<R, true>(fexp, oir, oi_inf, tau_oi, dt);
+    const R ao = pdv(R(0.65), uexp(divc(-(u + R(10)), R(8.5))) + uexp(divc(-(u - R(30)), R(59.0))));
+    const R bo = pdv(R(0.65), R(2.5) + uexp(divc(u + R(82), R(17.0))));
+    const R tau_o = pdv(R(1), kq10 * (ao + bo));
+    const R o_inf = pdv(R(1), R(1) + uexp(divc(-(u + R(20.47)), R(17.54))));
+    const R aoi = pdv(R(1), R(18.53) + uexp(divc(u + R(113.7), R(10.95))));
+    const R boi = pdv(R(1), R(35.56) + uexp(divc(-(u + R(1.26)), R(7.44))));
+    const R tau_oi = pdv(R(1), kq10 * (aoi + boi));
+    const R oi_inf = pdv(R(1), R(1) + uexp(divc(u + R(43.1), R(5.3))));
+    const R oa = crn_gate<R, CHECKED>(fexp, oar, o_inf, tau_o, dt);
+    const R oi = crn_gate<R, CHECKED>(fexp, oir, oi_inf, tau_oi, dt);
     oar = oa;
     oir = oi;
     ito = gto * (oa * (oa * oa)) * oi * (u - ek);
@@ -1005,18 +1006,18 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
   {
     auto&& uar = ref<R>(S, 12, c);
     auto&& uir = ref<R>(S, 13, c);
-    const R gkur = R(0.005) + udv(R(0.05), R(1) + uexp(divc(-(u - R(15)), R(13.0))));
+    const R gkur = R(0.005) + pdv(R(0.05), R(1) + uexp(divc(-(u - R(15)), R(13.0))));
     const R aua =
-        udv(R(0.65), uexp(divc(-(u + R(10)), R(8.5))) + uexp(divc(-(u - R(30)), R(59.0))));
-    const R bua = udv(R(0.65), R(2.5) + uexp(divc(u + R(82), R(17.0))));
-    const R tau_ua = fdv(R(1), kq10 * (aua + bua));
-    const R ua_inf = udv(R(1), R(1) + uexp(divc(-(u + R(30.3)), R(9.6))));
-    const R aui = udv(R(1), R(21) + uexp(divc(-(u - R(185)), R(28.0))));
+        pdv(R(0.65), uexp(divc(-(u + R(10)), R(8.5))) + uexp(divc(-(u - R(30)), R(59.0))));
+    const R bua = pdv(R(0.65), R(2.5) + uexp(divc(u + R(82), R(17.0))));
+    const R tau_ua = pdv(R(1), kq10 * (aua + bua));
+    const R ua_inf = pdv(R(1), R(1) + uexp(divc(-(u + R(30.3)), R(9.6))));
+    const R aui = pdv(R(1), R(21) + uexp(divc(-(u - R(185)), R(28.0))));
     const R bui = uexp(divc(u - R(158), R(16.0)));
-    const R tau_ui = fdv(R(1), kq10 * (aui + bui));
-    const R ui_inf = udv(R(1), R(1) + uexp(divc(u - R(99.45), R(27.48))));
-    const R ua = crn_gate<R, true>(fexp, uar, ua_inf, tau_ua, dt);
-    const R ui = crn_gate<R, true>(fexp, uir, ui_inf, tau_ui, dt);
+    const R tau_ui = pdv(R(1), kq10 * (aui + bui));
+    const R ui_inf = pdv(R(1), R(1) + uexp(divc(u - R(99.45), R(27.48))));
+    const R ua = crn_gate<R, CHECKED>(fexp, uar, ua_inf, tau_ua, dt);
+    const R ui = crn_gate<R, CHECKED>(fexp, uir, ui_inf, tau_ui, dt);
     uar = ua;
     uir = ui;
     ikur = gkur_coeff * gkur * (ua * (ua * ua)) * ui * (u - ek);
@@ -1031,14 +1032,14 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
       axr = R(0.0003 * 5) / exprel(-(u + R(14.1)) / R(5));
       bxr = R(7.3898e-05 * 5.1237) / exprel((u - R(3.3328)) / R(5.1237));
     } else {
-      axr = udv(R(0.0003) * (u + R(14.1)), R(1) - uexp(divc(-(u + R(14.1)), R(5))));
+      axr = pdv(R(0.0003) * (u + R(14.1)), R(1) - uexp(divc(-(u + R(14.1)), R(5))));
       bxr = fdv(R(7.3898e-05) * (u - R(3.3328)), uexp(divc(u - R(3.3328), R(5.1237))) - R(1));
     }
     const R tau_xr = fdv(R(1), axr + bxr);
-    const R xr_inf = udv(R(1), R(1) + uexp(divc(-(u + R(14.1)), R(6.5))));
+    const R xr_inf = pdv(R(1), R(1) + uexp(divc(-(u + R(14.1)), R(6.5))));
     const R xr = crn_gate<R, true>(fexp, xrr, xr_inf, tau_xr, dt);
     xrr = xr;
-    ikr = udv(gkr * xr * (u - ek), R(1) + uexp(divc(u + R(15), R(22.4))));
+    ikr = pdv(gkr * xr * (u - ek), R(1) + uexp(divc(u + R(15), R(22.4))));
   }
   // calc_iks on the kernel's xs slot (index 14)
   R iks;
@@ -1049,11 +1050,11 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
       axs = R(4e-05 * 17) / exprel(-(u - R(19.9)) / R(17));
       bxs = R(3.5e-05 * 9) / exprel((u - R(19.9)) / R(9));
     } else {
-      axs = udv(R(4e-05) * (u - R(19.9)), R(1) - uexp(divc(-(u - R(19.9)), R(17))));
-      bxs = udv(R(3.5e-05) * (u - R(19.9)), uexp(divc(u - R(19.9), R(9))) - R(1));
+      axs = pdv(R(4e-05) * (u - R(19.9)), R(1) - uexp(divc(-(u - R(19.9)), R(17))));
+      bxs = pdv(R(3.5e-05) * (u - R(19.9)), uexp(divc(u - R(19.9), R(9))) - R(1));
     }
-    const R tau_xs = udv(R(1), R(2) * (axs + bxs));
-    const R xs_inf = udv(R(1), fsqrt(R(1) + uexp(divc(-(u - R(19.9)), R(12.7)))));
+    const R tau_xs = pdv(R(1), R(2) * (axs + bxs));
+    const R xs_inf = pdv(R(1), fsqrt(R(1) + uexp(divc(-(u - R(19.9)), R(12.7)))));
     const R xs = crn_gate<R, CHECKED>(fexp, xsr, xs_inf, tau_xs, dt);
     xsr = xs;
     iks = gks * (xs * xs) * (u - ek);
@@ -1070,14 +1071,14 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
       tau_d = exprel(y) / (R(6.24 * 0.035) * (R(1) + fexp(y)));
     } else {
       const R e = uexp(divc(-(u + R(10)), R(6.24)));
-      tau_d = udv(R(1) - e, R(0.035) * (u + R(10)) * (R(1) + e));
+      tau_d = pdv(R(1) - e, R(0.035) * (u + R(10)) * (R(1) + e));
     }
-    const R d_inf = udv(R(1), R(1) + uexp(divc(-(u + R(10)), R(8.0))));
-    const R tau_f = udv(R(9), R(0.0197) * uexp(-R(0.0337 * 0.0337) * ((u + R(10)) * (u + R(10)))) +
+    const R d_inf = pdv(R(1), R(1) + uexp(divc(-(u + R(10)), R(8.0))));
+    const R tau_f = pdv(R(9), R(0.0197) * uexp(-R(0.0337 * 0.0337) * ((u + R(10)) * (u + R(10)))) +
                                  R(0.02));
-    const R f_inf = udv(R(1), R(1) + uexp(divc(u + R(28), R(6.9))));
+    const R f_inf = pdv(R(1), R(1) + uexp(divc(u + R(28), R(6.9))));
     const R tau_fca = R(2);
-    const R fca_inf = fdv(R(1), R(1) + divc(cai, R(0.00035)));
+    const R fca_inf = pdv(R(1), R(1) + divc(cai, R(0.00035)));
     const R d = crn_gate<R, CHECKED>(fexp, dr, d_inf, tau_d, dt);
     const R f = crn_gate<R, CHECKED>(fexp, fr, f_inf, tau_f, dt);
     const R fca = crn_gate<R, CHECKED>(fexp, fcar, fca_inf, tau_fca, dt);
@@ -1089,9 +1090,9 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
   // calc_inak
   const R sig = F64 ? par<R>(P, kCrnSig) : R(1 / 7.0) * (fexp(nao / R(67.3)) - R(1));
   const R ko_km = F64 ? par<R>(P, kCrnKo) : ko / (ko + kmko);
-  const R fnak = fdv(R(1), R(1) + R(0.1245) * fexp(overRT(R(-0.1) * (F * u))) +
+  const R fnak = pdv(R(1), R(1) + R(0.1245) * fexp(overRT(R(-0.1) * (F * u))) +
                               R(0.0365) * sig * fexp(overRT(-(F * u))));
-  const R inak = inakmax * fnak * fdv(R(1), R(1) + fpow15(fdv(kmnai, nai))) * ko_km;
+  const R inak = inakmax * fnak * pdv(R(1), R(1) + fpow15(pdv(kmnai, nai))) * ko_km;
   // calc_inaca
   const R gamma = R(0.35);
   const R exp_term = fexp(overRT(gamma * (F * u)));
@@ -1103,10 +1104,10 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
   const R term2 = kmcancx + cao;
   const R term12 = F64 ? par<R>(P, kCrnT12) : term1 * term2;
   const R term3 = R(1) + ksatncx * exp_rev_term;
-  const R inaca = fdv(numerator, term12 * term3);
+  const R inaca = pdv(numerator, term12 * term3);
   const R ibca = gcab * (u - eca);
   const R ibna = gnab * (u - ena);
-  const R ipca = fdv(ipcamax * cai, cai + R(0.0005));
+  const R ipca = pdv(ipcamax * cai, cai + R(0.0005));
   // calc_irel (uses the irel stored by the previous step)
   R irel;
   {
@@ -1129,9 +1130,9 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
       tau_w = R(6.0 / 5.0) * exprel(y) / (R(1) + R(0.3) * fexp(y));
     } else {
       const R e = uexp(divc(-(u - R(7.9)), R(5.0)));
-      tau_w = udv(R(6) * (R(1) - e), (R(1) + R(0.3) * e) * (u - R(7.9)));
+      tau_w = pdv(R(6) * (R(1) - e), (R(1) + R(0.3) * e) * (u - R(7.9)));
     }
-    const R w_inf = R(1) - udv(R(1), R(1) + uexp(divc(-(u - R(40)), R(17.0))));
+    const R w_inf = R(1) - pdv(R(1), R(1) + uexp(divc(-(u - R(40)), R(17.0))));
     const R urel = crn_gate<R, CHECKED>(fexp, urr, u_inf, tau_u, dt);
     const R vrel = crn_gate<R, CHECKED>(fexp, vrr, v_inf, tau_v, dt);
     const R wrel = crn_gate<R, CHECKED>(fexp, wrr, w_inf, tau_w, dt);
@@ -1144,7 +1145,7 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
   auto overFVj = [&](R x) -> R { return divu(x, F * Vj, kCrnInvFVj); };
   const R vrel_vup = F64 ? par<R>(P, kCrnVrelVup) : Vrel / Vup;
   const R itr = divc(caup - carel, R(180));
-  const R iup = fdv(iupmax, R(1) + fdv(kup, cai));
+  const R iup = pdv(iupmax, R(1) + pdv(kup, cai));
   const R iupleak = divu(caup, caupmax, kCrnInvCaup) * iupmax;
   caupr = caup + dt * (iup - iupleak - itr * vrel_vup);
   nair = nai + dt * overFVj(R(-3) * inak - R(3) * inaca - ibna - ina);
@@ -1153,11 +1154,11 @@ __device__ __forceinline__ U crn_update(U u_in, U un, SP& S, int64_t c, R dt, co
     const R B1 = divu(R(2) * inaca - ipca - ical - ibca,
                       R(2) * F * Vj, kCrnInv2FVj) +
                  divu(Vup * (iupleak - iup) + irel * Vrel, Vj, kCrnInvVj);
-    const R B2 = R(1) + fdv(trpnmax * kmtrpn, (cai + kmtrpn) * (cai + kmtrpn)) +
-                 fdv(cmdnmax * kmcmdn, (cai + kmcmdn) * (cai + kmcmdn));
-    cair = cai + dt * fdv(B1, B2);
+    const R B2 = R(1) + pdv(trpnmax * kmtrpn, (cai + kmtrpn) * (cai + kmtrpn)) +
+                 pdv(cmdnmax * kmcmdn, (cai + kmcmdn) * (cai + kmcmdn));
+    cair = cai + dt * pdv(B1, B2);
   }
-  carelr = carel + dt * fdv(itr - irel, R(1) + fdv(csqnmax * kmcsqn,
+  carelr = carel + dt * pdv(itr - irel, R(1) + pdv(csqnmax * kmcsqn,
                                                  (carel + kmcsqn) * (carel + kmcsqn)));
   return un - dt * (ina + ik1 + ito + ikur + ikr + iks + ical + ipca + inak +
                     inaca + ibna + ibca);
@@ -1172,7 +1173,7 @@ __device__ __forceinline__ U ionic_crn(U u_in, U un, SP& S, int64_t c, R dt,
                                         const Params& P) {
   constexpr bool SPLIT = FORM == kSplitForm;
   if constexpr (SPLIT && sizeof(R) == 8) {
-    if (__builtin_expect(__all(fabs(u_in) <= 160.0), 1))
+    if (__builtin_expect(P.v[kCrnOrdinary] != 0.0 && __all(fabs(u_in) <= 160.0), 1))
       return crn_update<R, SPLIT, false>(u_in, un, S, c, dt, P);
   }
   return crn_update<R, SPLIT, true>(u_in, un, S, c, dt, P);
