@@ -168,12 +168,13 @@ class TissueBatch:
     block-to-XCD map; `fw_batch_variants`) that compute the same results bit
     for bit.  With ``autotune`` the batch times each on its own next steps
     (``tune_steps`` each after one untimed step), keeps the fastest and
-    remembers it per (device, model, precision, size class) in memory and in
-    a JSON cache (``FW_AUTOTUNE_CACHE``, default
+    remembers it per (device, model, precision, stencils, size class) in
+    memory and in a JSON cache (``FW_AUTOTUNE_CACHE``, default
     ``~/.cache/finitewave_amd/batch_tune.json``).  The size class is the
     power of two of the batch's node count; admissions and retirements that
-    change it select the shape again (from the cache, or by timing), since
-    the best shape of a few small tissues is not that of many."""
+    change it or the stencils (5-point, 9-point or both) select the shape
+    again (from the cache, or by timing), since the best shape of a few small
+    tissues is not that of many."""
 
     def __init__(self, model_cls, precision: str = "fp32", dt: float = 0.01, dr: float = 0.25,
                  max_tissues: int = 1024, use_graph: bool = True, chunk_cap: int = 4000,
@@ -452,9 +453,15 @@ class TissueBatch:
               "fw_batch_set_variant")
 
     def _tune_key(self) -> str:
-        n = sum(int(self.buffers[s]["desc"].n) for s in self.sims)
+        descs = [self.buffers[s]["desc"] for s in self.sims]
+        n = sum(int(d.n) for d in descs)
+        kinds = {d.stencil for d in descs}
+        # a shape that suits the 5-point stencil can cost the 9-point one a multiple
+        # (40 Mitchell-Schaeffer tissues of 60 to 250 columns: 48.4 us per step in the
+        # shape chosen for 5-point tissues, 12.0 in its own)
+        st = "mixed" if len(kinds) > 1 else ("iso" if _native.STENCIL_ISO in kinds else "aniso")
         dev = self.torch.cuda.get_device_name(self.dev)
-        return f"{dev}|m{self.model_id}|p{self.prec}|n2^{int(math.log2(max(1, n)))}"
+        return f"{dev}|m{self.model_id}|p{self.prec}|{st}|n2^{int(math.log2(max(1, n)))}"
 
     def _tune(self, n_avail: int) -> int:
         """Times every variant on the next steps; returns the steps run."""
