@@ -4,7 +4,6 @@
 #include <stdio.h>
 #include <string.h>
 
-#include <functional>
 #include <mutex>
 #include <vector>
 
@@ -843,14 +842,17 @@ static int32_t multi_fit(int32_t k, int32_t least, int64_t room) {
   return 2 * k <= room ? k : 0;
 }
 
+static int run_graphs(fw_plan* plan, void* u, void* u_new, void* const* state, int64_t step0,
+                      int32_t n_steps, const fw_track_desc* track, void* stream);
+
 // n_steps with multi-step launches wherever they apply, single steps
-// elsewhere (among them the last: u_new then holds the step before).
-// `singles` runs the single steps.  *done = false: nothing launched, the run
-// has no multi-step form.
-typedef std::function<int(void*, void*, int64_t, int32_t, const fw_track_desc*)> Singles;
+// elsewhere (among them the last: u_new then holds the step before), long
+// stretches of those from graphs if `graph`.  *done = false: nothing launched,
+// the run has no multi-step form.
 static int run_multi(fw_plan* plan, void* u, void* u_new, void* const* state, int64_t step0,
-                     int32_t n_steps, const fw_track_desc* track, hipStream_t s, bool graph,
-                     const Singles& singles, bool* done) {
+                     int32_t n_steps, const fw_track_desc* track, void* stream, bool graph,
+                     bool* done) {
+  hipStream_t s = as_stream(stream);
   *done = false;
   if (!plan->alt) return FW_OK;
   int32_t shape_k, rows;
@@ -923,7 +925,10 @@ static int run_multi(fw_plan* plan, void* u, void* u_new, void* const* state, in
       if (track->act_flags) sub.act_flags = track->act_flags + pos;
       if (track->probe_rows) sub.probe_rows = track->probe_rows + pos;
     }
-    const int rc = singles(a, b, step, n, track ? &sub : nullptr);
+    const fw_track_desc* t = track ? &sub : nullptr;
+    const int rc = graph && n >= kMultiGraphSteps
+                       ? run_graphs(plan, a, b, state, step, n, t, stream)
+                       : run_plain(plan, a, b, state, step, n, t, stream);
     if (rc) return rc;
     pos += n;
     if (n % 2) {
@@ -955,11 +960,7 @@ int fw_run(fw_plan* plan, void* u, void* u_new, void* const* state, int64_t step
   int rc = check_run_args(plan, u, u_new, state, n_steps, track);
   if (rc) return rc;
   bool done = false;
-  rc = run_multi(plan, u, u_new, state, step0, n_steps, track, as_stream(stream), false,
-                 [&](void* a, void* b, int64_t step, int32_t n, const fw_track_desc* t) {
-                   return run_plain(plan, a, b, state, step, n, t, stream);
-                 },
-                 &done);
+  rc = run_multi(plan, u, u_new, state, step0, n_steps, track, stream, false, &done);
   if (rc || done) return rc;
   return run_plain(plan, u, u_new, state, step0, n_steps, track, stream);
 }
@@ -1270,13 +1271,7 @@ int fw_run_graph(fw_plan* plan, void* u, void* u_new, void* const* state, int64_
   int rc = check_graph_args(plan, u, u_new, state, n_steps, track, &act_on);
   if (rc) return rc;
   bool done = false;
-  rc = run_multi(plan, u, u_new, state, step0, n_steps, track, as_stream(stream), true,
-                 [&](void* a, void* b, int64_t step, int32_t n, const fw_track_desc* t) {
-                   return n >= kMultiGraphSteps
-                              ? run_graphs(plan, a, b, state, step, n, t, stream)
-                              : run_plain(plan, a, b, state, step, n, t, stream);
-                 },
-                 &done);
+  rc = run_multi(plan, u, u_new, state, step0, n_steps, track, stream, true, &done);
   if (rc || done) return rc;
   return run_graphs(plan, u, u_new, state, step0, n_steps, track, stream);
 }
