@@ -515,8 +515,14 @@ int fw_plan_create(const fw_plan_desc* desc, fw_plan** out) {
   }
   const int need_fields = needed_fields(d);
   const int64_t N = p->N;
-  const size_t alt = multi_alt_bytes(p);
+  size_t alt = multi_alt_bytes(p);
   hipError_t e = hipMalloc(&p->step_words, kStepWordBytes + alt);
+  if (e != hipSuccess && alt) {
+    // single steps need no second state set
+    (void)hipGetLastError();
+    alt = 0;
+    e = hipMalloc(&p->step_words, kStepWordBytes);
+  }
   if (e != hipSuccess) {
     set_error("fw_plan_create: hipMalloc failed: %s", hipGetErrorString(e));
     delete p;
