@@ -8,7 +8,9 @@
  * of its tabulated half-step fields; for a 3D plan whose fields are uniform
  * or tables along the last axis, each field as such a table in double and
  * float -- all read once at creation; for a 2D plan of a light model with
- * uniform fields, a second set of state arrays),
+ * uniform fields, of a size at which launches of several steps are the
+ * faster, a second set of state arrays, which it does without where device
+ * memory is short),
  * fw_batch_create (the tissue descriptor table) and fw_batch_set_active (the
  * block table, when it grows).  `stream` is a
  * hipStream_t passed as void* (NULL = the default stream).  All launches are
